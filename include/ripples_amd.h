@@ -52,7 +52,9 @@ typedef struct {
   uint32_t slots;        /* IC: resident colour groups (persistent workgroups) */
   uint32_t queue_cap;    /* IC lane sampler: vertices one lane's sample may
                             reach before the wave sampler takes it over:
-                            64, 256, 1024, 2048 or 4096 (0 = 1024) */
+                            64, 256, 1024, 2048 or 4096.  0 = automatic: AUTO
+                            runs the wave stage below behind lanes of 64
+                            vertices, LANE takes 1024 */
   uint32_t heavy_degree; /* IC: rows this long wait for the hub phase */
   uint32_t sampler;      /* IC: RIP_SAMPLER_AUTO, _WAVE or _COLOUR */
   uint32_t out_chunk;    /* LT and IC wave sampler: pool elements a wave
@@ -61,18 +63,20 @@ typedef struct {
   uint32_t frontier_cap; /* IC grid sampler (AUTO): frontier entries a BFS
                             level may list (0 = automatic); vertices past it
                             are found again by a scan of the pending masks */
-  uint32_t wave_stage;   /* IC AUTO: nonzero = samples passing queue_cap are
+  uint32_t wave_stage;   /* IC AUTO: nonzero (or queue_cap 0) = samples passing queue_cap are
                             first run one per wave, 64 frontier vertices at a
                             time, up to 4096 vertices, and only the larger
-                            ones go to the grid sampler */
+                            ones go to the grid sampler; calls of up to 16,384
+                            samples start there, with no lanes before */
 } rip_tune;
 
 /* IC sampler kinds (all give the same sets):
  *   AUTO    one reverse BFS per lane (64 samples per wave); samples passing
- *           queue_cap vertices go to the grid sampler: 64-sample colour groups,
- *           many groups per batch, one BFS level of all of them per kernel
- *           (with rip_tune.wave_stage, first to one BFS per wave expanding 64
- *           queued vertices at a time, and to the grid past 4096 vertices)
+ *           queue_cap vertices go to one BFS per wave expanding 64 queued
+ *           vertices at a time (the wave stage; not with a queue_cap given
+ *           and wave_stage 0), and past 4096 vertices to the grid sampler:
+ *           64-sample colour groups, many groups per batch, one BFS level of
+ *           all of them per kernel
  *   WAVE    one reverse BFS per wave for every sample (the plain form), sets
  *           passing 4096 vertices finished by a bitmap-visited BFS per wave
  *   COLOUR  64-sample colour groups for every sample
@@ -239,8 +243,8 @@ int rip_pool_coverage(rip_pool *p, uint64_t num_sets, const uint32_t *seeds,
 int rip_pool_coverage_noalloc(rip_pool *p, uint64_t num_sets, const uint32_t *seeds,
                               uint32_t num_seeds, uint64_t *covered);
 /* Device time of the last rip_pool_sample call's main sampling kernel (IC:
- * the lane kernel, or the wave kernel when the sampler kind has no lane
- * stage; LT: the walk kernel), measured with HIP events on the pool's
+ * the lane kernel, or the wave kernel when the call has no lane stage;
+ * LT: the walk kernel), measured with HIP events on the pool's
  * stream, and the number of kernel launches of the call. */
 int rip_pool_last_kernel_ms(const rip_pool *p, double *ms, uint32_t *launches);
 /* The grid sampler's share of the last rip_pool_sample call (IC, AUTO: the

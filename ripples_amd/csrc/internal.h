@@ -372,6 +372,9 @@ void grid_scratch_free(GridScratch &s);
 // returns how many outgrew a lane's queue, their indices (relative to first)
 // in g->wave.d_over.  Brackets its main kernel with the pool's ev0 / ev1.
 constexpr uint32_t kLaneCapDefault = 1024;
+constexpr uint32_t kLaneCapStaged = 64;   // with the wave stage behind the lanes
+// Whether an AUTO call runs the wave stage: asked for, or no queue_cap given.
+bool ic_wave_stage(const rip_tune *tune);
 uint32_t ic_lane_cap(const rip_tune *tune);
 uint64_t ic_lane_launch(rip_pool *p, uint64_t first, uint64_t count, const rip_tune *tune);
 uint64_t ic_lane_slack(const rip_pool *p, uint64_t count, const rip_tune *tune);

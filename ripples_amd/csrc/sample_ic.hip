@@ -654,10 +654,29 @@ uint32_t ic_launch(rip_pool *p, uint64_t first, uint64_t count,
   return 2;
 }
 
+// Calls of at most this many samples skip the lanes: a lane takes about
+// 0.4 ms to walk a sample of 64 vertices, whatever the launch holds, where a
+// wave of the stage takes under 0.1 ms.  IMM on 1,000 vertices (weighted
+// cascade, k = 5, eps = 0.5): 2.45 ms with the lanes, 1.33 without; OPIM-C on
+// 200,003 vertices (calls of a few thousand sets): 10.3 and 6.9 ms.  Past
+// this the stage's few thousand resident waves become the limit, where the
+// lanes hold hundreds of thousands of samples (thresholds of 4,096 and 65,536
+// measured the same on these and on IMM and serving at 65K-262K vertices).
+constexpr uint64_t kWaveDirectMax = 16384;
+
 uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &cfg,
                    const rip_tune *tune) {
   if (cfg.sampler == RIP_SAMPLER_COLOUR) return ic_launch(p, first, count, cfg);
   uint32_t launches = 0;
+  if (count <= kWaveDirectMax && ic_wave_stage(tune)) {
+    // few samples: one wave each from the start, with no lanes before
+    const uint64_t big = ic_wave_launch(p, first, count, nullptr, cfg.out_chunk, true, true, true);
+    launches += 2;
+    if (big == 0) return launches;
+    return launches + ic_grid_launch(p, first, big, p->g->wave.d_big, true,
+                                     tune ? tune->frontier_cap : 0u,
+                                     tune && tune->colors ? tune->colors : 64u);
+  }
   uint64_t wave_count = count;
   const uint32_t *wave_ids = nullptr;
   const bool lanes = cfg.sampler == RIP_SAMPLER_AUTO || cfg.sampler == RIP_SAMPLER_LANE;
@@ -671,7 +690,7 @@ uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &
     if (cfg.sampler == RIP_SAMPLER_AUTO) {
       const uint32_t frontier_cap = tune ? tune->frontier_cap : 0u;
       const uint32_t colors = tune && tune->colors ? tune->colors : 64u;
-      if (tune && tune->wave_stage) {
+      if (ic_wave_stage(tune)) {
         // one BFS per wave, 64 frontier vertices at a time, for the samples
         // up to the wave list; the grid sampler takes the larger ones
         const uint64_t big = ic_wave_launch(p, first, wave_count, wave_ids, cfg.out_chunk, false,

@@ -206,16 +206,25 @@ __device__ inline bool expand_row(const VertexRec *vrec, const uint32_t *ids,
   return true;
 }
 
+// Candidates a lane collects before their edges are read together.
+constexpr uint32_t kUnitBatch = 4;
+
 // Expands up to 64 queued vertices of the sample whose element 0 is z at
-// once, lane l taking the vertex whose record is rv (when `have`): the lane
-// walks its row's gap blocks one draw per step, as a lane of the lane
-// sampler does; the live edges of a step go through visit() and the first
-// visits are appended to list[tail ...].  Every lane of the wave must call
-// it.  Returns false when the live edges of a step could take the list past
-// cap.  Rows of a few edges (weighted cascade: one candidate per row) keep
-// 64 lanes busy here, where expand_row would give each row a whole wave.
+// once, lane l holding the record rv of one (when `have`).  The rows' gap
+// blocks are the units of work: 64 units at a time, one per lane, found by a
+// wave scan of the block counts when some row has several (a hub's blocks
+// spread over the lanes instead of queueing in one).  A lane draws up to
+// kUnitBatch candidates of its block (arithmetic only), then the wave reads
+// their thresholds and in-neighbours together, so a unit waits for one trip
+// to memory, not one per candidate; the live ones go through visit() and the
+// first visits are appended to list[tail ...].  Against one draw per lane and
+// step, a whole row per lane: the stage's kernels of an IMM run on R-MAT scale
+// 22 weighted cascade took 13.5 ms instead of 15.6 (rows of one block there;
+// hub rows of U[0,0.1] graphs have hundreds).  Every lane of the wave must
+// call it.  Returns false when the live edges of a step could take the list
+// past cap.
 template <typename Visit>
-__device__ inline bool expand_rows_lanes(const uint32_t *ids, const uint32_t *val, bool have,
+__device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *val, bool have,
                                          const VertexRec &rv, uint64_t z,
                                          const Affine *p2, const IcLogTables *tab,
                                          uint32_t *list, uint32_t &tail, uint32_t cap,
@@ -223,86 +232,124 @@ __device__ inline bool expand_rows_lanes(const uint32_t *ids, const uint32_t *va
                                          unsigned long long &st_draws,
                                          unsigned long long &st_bytes,
                                          unsigned long long &st_live, Visit &&visit) {
-  uint32_t T = 0, rbegin = 0, deg = 0, beta = 0, nblk = 0, k = 0, len = 0, pos = 0;
-  bool uniform = true;
-  uint64_t q = 0, rq = 0, ufull = 0, ulast = 0, xb = 0, x = 0;
-  if (have) {
-    T = rv.thr;
-    have = T != 0;                               // no edge of the row can be live
-    if (have) {
-      rbegin = rv.begin;
-      deg = rv.end - rv.begin;
-      uniform = (rv.flags & kRowUniform) != 0;
-      beta = (rv.flags >> kBetaShift) & 31u;
-      q = rv.q;
-      rq = rv.rq;
-      ufull = rv.ufull;
-      ulast = rv.ulast;
-      nblk = ((deg - 1) >> beta) + 1;
-      xb = rv.ja * z + rv.jb;                    // the row's first element
-    }
-  }
-  // block k of the row: its length, and no candidate when one compare says so
-  auto open_block = [&]() {
-    len = min(deg - (k << beta), 1u << beta);
-    x = xb;
-    pos = 0;
-    ++st_draws;
-    if ((xb >> 32) + 1 <= (len == (1u << beta) ? ufull : ulast)) len = 0;
-  };
-  if (have) open_block();
+  const uint32_t lane = lane_id();
+  const bool row = have && rv.thr != 0;            // else no edge of the row can be live
+  const uint32_t rdeg = rv.end - rv.begin;
+  const uint32_t nblk = row ? ((rdeg - 1) >> ((rv.flags >> kBetaShift) & 31u)) + 1 : 0u;
+  const uint64_t x0 = rv.ja * z + rv.jb;           // the row's first element
+  const bool single = __ballot(nblk > 1) == 0;     // a lane's unit is its own row
+  const uint32_t incl = single ? 0u : wave_inclusive_scan(nblk);
+  const uint32_t total = single ? 64u : uniform_u32(__shfl(incl, 63, 64));
   const Affine P = p2[0];
-  for (;;) {
-    bool live = false;
-    uint32_t e = 0;
-    if (have) {
-      if (pos >= len) {
-        if (++k < nblk) {
-          const Affine jb = p2[beta + 1];          // 2B elements: the next block
-          xb = aff_apply(jb, xb);
-          open_block();
-        } else {
-          have = false;
-        }
-      } else {
-        const uint64_t gap = ic_gap_fast(x, q, rq, tab);
-        if (gap >= len - pos) {
-          pos = len;
-        } else {
-          pos += static_cast<uint32_t>(gap);
-          e = rbegin + (k << beta) + pos;
-          const uint64_t a = aff_apply(P, x);      // acceptance element
-          ++st_cand;
-          if (!uniform) {
-            ++st_draws;
-            st_bytes += 4;
-          }
-          live = uniform || ic_accept(a, T, val[e]);
-          if (live) {
-            ++st_live;
-            st_bytes += 4;
-          }
-          ++pos;
-          x = aff_apply(P, a);                     // next gap element
-          if (pos < len) ++st_draws;
-        }
+  for (uint32_t u0 = 0; u0 < total; u0 += 64) {
+    uint32_t e0 = rv.begin, len = 0, T = rv.thr;
+    uint64_t q = rv.q, rq = rv.rq, x = x0;
+    bool uniform = (rv.flags & kRowUniform) != 0;
+    bool skip = true;
+    if (single) {
+      if (row) {
+        len = rdeg;                                // one block, at most its full length
+        const uint32_t beta = (rv.flags >> kBetaShift) & 31u;
+        skip = (x >> 32) + 1 <= (len == (1u << beta) ? rv.ufull : rv.ulast);
+      }
+    } else {
+      // unit u is block k of the row of lane j, the first whose inclusive
+      // prefix passes u
+      const uint32_t u = u0 + lane;
+      uint32_t j = 0;
+#pragma unroll
+      for (uint32_t s = 32; s > 0; s >>= 1) {
+        const uint32_t v = __shfl(incl, static_cast<int>(j + s - 1), 64);
+        if (v <= u) j += s;
+      }
+      const int src = static_cast<int>(min(j, 63u));
+      const uint32_t k = u - (__shfl(incl, src, 64) - __shfl(nblk, src, 64));
+      const uint32_t begin = __shfl(rv.begin, src, 64), deg = __shfl(rdeg, src, 64);
+      const uint32_t flags = __shfl(rv.flags, src, 64);
+      const uint32_t ufull = __shfl(rv.ufull, src, 64), ulast = __shfl(rv.ulast, src, 64);
+      T = __shfl(rv.thr, src, 64);
+      q = __shfl(rv.q, src, 64);
+      rq = __shfl(rv.rq, src, 64);
+      x = __shfl(x0, src, 64);
+      uniform = (flags & kRowUniform) != 0;
+      if (u < total) {
+        const uint32_t beta = (flags >> kBetaShift) & 31u;
+        e0 = begin + (k << beta);
+        len = min(deg - (k << beta), 1u << beta);
+        // block k's first element: 2 B k elements after the row's first
+        for (uint32_t kk = k, bit = beta + 1; kk; kk >>= 1, ++bit)
+          if (kk & 1) x = aff_apply(p2[bit], x);
+        skip = (x >> 32) + 1 <= (len == (1u << beta) ? ufull : ulast);
       }
     }
-    const uint64_t lm = __ballot(live);
-    if (lm) {
-      if (tail + __popcll(lm) > cap) return false;
-      const uint32_t src = live ? ids[e] : 0u;
-      const bool fresh = live && visit(src);
-      const uint64_t fm = __ballot(fresh);
-      if (fresh) list[tail + __popcll(fm & lanes_below())] = src;
-      tail += __popcll(fm);
+    // a block without candidates costs one compare
+    if (len) ++st_draws;
+    bool more = len != 0 && !skip;
+    uint32_t pos = 0;
+    while (__ballot(more)) {
+      uint32_t ce[kUnitBatch], th[kUnitBatch];
+      uint32_t nc = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < kUnitBatch; ++i) {
+        ce[i] = 0;
+        th[i] = 0;
+        if (more) {
+          const uint64_t gap = ic_gap_fast(x, q, rq, tab);
+          if (gap >= len - pos) {
+            more = false;
+          } else {
+            pos += static_cast<uint32_t>(gap);
+            const uint64_t a = aff_apply(P, x);    // acceptance element
+            ce[i] = e0 + pos;
+            // kept iff the edge's threshold t passes this (ic_accept:
+            // hi32(a) T < t 2^32)
+            th[i] = static_cast<uint32_t>(((a >> 32) * T) >> 32);
+            nc = i + 1;
+            if (++pos < len) {
+              x = aff_apply(P, a);                 // next gap element
+              ++st_draws;
+            } else {
+              more = false;
+            }
+          }
+        }
+      }
+      uint32_t t[kUnitBatch], src[kUnitBatch];
+#pragma unroll
+      for (uint32_t i = 0; i < kUnitBatch; ++i) {
+        t[i] = 0xFFFFFFFFu;                        // rows sharing one threshold keep every candidate
+        src[i] = 0;
+        if (i < nc) {
+          src[i] = ids[ce[i]];
+          if (!uniform) t[i] = val[ce[i]];
+        }
+      }
+      st_cand += nc;
+      if (!uniform) {
+        st_draws += nc;
+        st_bytes += 4 * nc;
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < kUnitBatch; ++i) {
+        const bool live = i < nc && t[i] > th[i];
+        const uint64_t lm = __ballot(live);
+        if (lm == 0) continue;
+        if (tail + __popcll(lm) > cap) return false;
+        if (live) {
+          ++st_live;
+          st_bytes += 4;
+        }
+        const bool fresh = live && visit(src[i]);
+        const uint64_t fm = __ballot(fresh);
+        if (fresh) list[tail + __popcll(fm & lanes_below())] = src[i];
+        tail += __popcll(fm);
+      }
     }
-    if (__ballot(have) == 0) break;
   }
   return true;
 }
 
-// VP: expand 64 queued vertices at a time (expand_rows_lanes) instead of
+// VP: expand 64 queued vertices at a time (expand_rows_units) instead of
 // one row per step over its gap blocks (expand_row, the plain form), with
 // the first vertices of each sample marked in LDS.
 template <int BT, bool VP>
@@ -384,7 +431,7 @@ __global__ void __launch_bounds__(BT) ic_wave_kernel(WaveParams P) {
         if (next) recn = P.vrec[vn];
         head = nhead;
         st_exp += take;
-        if (!expand_rows_lanes(P.ids, P.val, have, rec, z, s_p2, &s_tab, list, tail, P.cap,
+        if (!expand_rows_units(P.ids, P.val, have, rec, z, s_p2, &s_tab, list, tail, P.cap,
                                st_cand, st_draws, st_bytes, st_live, visit_vp))
           big = true;
         prec = recn;
