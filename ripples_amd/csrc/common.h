@@ -83,7 +83,7 @@ inline uint32_t ic_threshold(float w) {
 // Device vertex record, one aligned 64-byte line: the jump to the vertex's
 // first stream element (IC: P^(1 + 2 begin), the row's first draw; LT:
 // P^(1 + begin), the threshold) and its CSR row; for IC the row's gap
-// parameters (ic_gap.h): largest threshold T, q and its reciprocal, log2 of
+// parameters (ic_gap.h): largest threshold T, q and its inverse, log2 of
 // the block size and the skip thresholds of a full and of the last block.
 struct alignas(64) VertexRec {
   uint64_t ja, jb;       // jump to the first element, as an affine map
@@ -94,7 +94,7 @@ struct alignas(64) VertexRec {
   uint32_t ufull;        // IC: a full block has no candidate iff hi32(x) + 1 <= ufull
   uint32_t flags;        // kRowUniform, kRowScalar; IC: beta << kBetaShift
   uint32_t ulast;        // IC: the same for the row's last block when it is partial
-  uint64_t rq;           // IC: floor(2^64 / q), the reciprocal of the gap divisor
+  double inv;            // IC: 2^58 / q, what a gap draw multiplies by
   uint32_t pad[2];
 };
 static_assert(sizeof(VertexRec) == 64, "one line per vertex record");

@@ -44,12 +44,12 @@ __global__ void build_vrec_kernel(const unsigned long long *index, const uint32_
   r.thr = thr[v];
   r.ufull = 0;
   r.ulast = 0;
-  r.rq = 0;
+  r.inv = 0.0;
   r.flags = flags[v];
   if (model == RIP_IC && r.thr != 0) {
     const uint32_t beta = ic_block_log2(r.thr);
     r.q = ic_gap_q(r.thr);
-    r.rq = ic_gap_recip(r.q);
+    r.inv = ic_gap_inv(r.q);
     r.ufull = ic_full_skip(r.q, beta);
     // the last block holds d - (nblk - 1) B edges
     const uint32_t d = static_cast<uint32_t>(e - b);

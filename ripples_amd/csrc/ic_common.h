@@ -86,4 +86,9 @@ __device__ inline void fill_step_powers(Affine step, Affine *p2) {
   for (int j = 1; j < 64; ++j) p2[j] = aff_then(p2[j - 1], p2[j - 1]);
 }
 
+// An affine map every lane holds alike, in scalar registers.
+__device__ inline Affine uniform_affine(Affine f) {
+  return Affine{uniform_u64(f.a), uniform_u64(f.b)};
+}
+
 }  // namespace rip

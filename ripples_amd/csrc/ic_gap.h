@@ -85,19 +85,10 @@ __host__ __device__ inline uint64_t ic_neg_log2(uint64_t u) {
   return ic_neg_log2_tab(u, kLog2C, kRecipC);
 }
 
-// The tables of ic_neg_log2, for a copy in LDS.
+// The tables of ic_neg_log2 as one object (the host checks' ic_gap_fast).
 struct IcLogTables {
   uint64_t log2c[256], recipc[256];
 };
-
-// Fills t (LDS) from the constant tables; every thread of the workgroup calls
-// it, the caller synchronises.
-__device__ inline void ic_load_tables(IcLogTables *t) {
-  for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) {
-    t->log2c[i] = kLog2C[i];
-    t->recipc[i] = kRecipC[i];
-  }
-}
 
 // q of a row whose largest threshold is T (1 <= T <= 2^24).
 __host__ __device__ inline uint64_t ic_gap_q(uint32_t T) {
@@ -148,6 +139,8 @@ __host__ __device__ inline uint32_t ic_full_skip(uint64_t q, uint32_t beta) {
   return ic_skip_len(q, 1u << beta);
 }
 
+// The gap in integer arithmetic without a division, which the host checks
+// hold against 128-bit division.
 // floor(2^64 / q) for q >= 2 (0 for q = 0): the reciprocal ic_gap_fast
 // divides by.  Every row has q = 0 or q >= NL(2^32 - 2^8) > 2^34.
 __host__ __device__ inline uint64_t ic_gap_recip(uint64_t q) {
@@ -168,6 +161,78 @@ __host__ __device__ inline uint64_t ic_gap_fast(uint64_t x, uint64_t q, uint64_t
   uint64_t g = mulhi_u64(N, rq);
   if ((g + 1) * q <= N) ++g;
   return g;
+}
+
+// ------------------------------------------------------------ device draws
+// The samplers draw their gaps in double precision and fall back on the
+// integer form only where rounding could decide: the same gap, bit for bit,
+// for about a fifth of the instructions (the integer form is nine 64-bit
+// multiplications, each four quarter-rate instructions, and waves holding a
+// few busy lanes are bound by exactly that).
+//
+// fg approximates NL(U) / q: -log2(U / 2^32) from the exponent, a table of
+// log2(1 + i/256) and a five-term series in r = m / (1 + i/256) - 1 < 2^-8,
+// times inv = 2^58 / q.  Errors, in units of -log2: the integer NL's own
+// truncation x^5 / (5 ln 2) < 2^-41.7; the double series' r^6 / (6 ln 2) <
+// 2^-50; its roundings, on values up to 32, < 2^-47; the product's, relative
+// 2^-51 on at most 32.  Together below 2^-41.5, so |fg - NL(U) / q| < 2^-41.5
+// inv, and where fg is at least 2^-40 inv from every integer its floor is the
+// gap.  Otherwise the gap is the integer nearest to fg or the one below
+// (2^-41.5 inv < 2^-17), settled by one exact product.
+
+// (1 / (1 + i/256), log2(1 + i/256)) pairs, for a copy in LDS.
+struct IcGapTab {
+  double rl[512];
+};
+
+__host__ __device__ inline void ic_gap_tab_entry(IcGapTab *t, uint32_t i) {
+  t->rl[2 * i] = 256.0 / (256.0 + static_cast<double>(i));
+  t->rl[2 * i + 1] = static_cast<double>(kLog2C[i]) * 0x1p-64;
+}
+
+// Fills t (LDS); every thread of the workgroup calls it, the caller
+// synchronises.
+__device__ inline void ic_load_tables(IcGapTab *t) {
+  for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) ic_gap_tab_entry(t, i);
+}
+
+// 2^58 / q (0 for q = 0), what ic_gap_draw multiplies by.
+__host__ __device__ inline double ic_gap_inv(uint64_t q) {
+  return q ? 0x1p58 / static_cast<double>(q) : 0.0;
+}
+
+// The gap of U = hi + 1 when g is the integer nearest to NL(U) / q.
+__host__ __device__ inline uint32_t ic_gap_settle(uint32_t hi, uint64_t q, uint32_t g) {
+  if (q == 0) return 0;                                    // every edge a candidate
+  const uint64_t N = ic_neg_log2(static_cast<uint64_t>(hi) + 1);
+  return static_cast<uint64_t>(g) * q <= N ? g : g - 1;
+}
+
+// ic_gap(x, q), with inv = ic_gap_inv(q).
+__host__ __device__ inline uint32_t ic_gap_draw(uint64_t x, uint64_t q, double inv,
+                                                const IcGapTab *t) {
+  const uint32_t hi = static_cast<uint32_t>(x >> 32);
+  const double u = static_cast<double>(hi) + 1.0;          // U, exact
+  uint64_t bits;
+  __builtin_memcpy(&bits, &u, 8);
+  const uint32_t top = static_cast<uint32_t>(bits >> 32);
+  const uint32_t i = (top >> 12) & 255u;
+  const int e = static_cast<int>(top >> 20) - 1023;        // floor(log2 U), 0..32
+  bits = (bits & 0x000FFFFFFFFFFFFFull) | 0x3FF0000000000000ull;
+  double m;
+  __builtin_memcpy(&m, &bits, 8);                          // U / 2^e, in [1, 2)
+  const double r = __builtin_fma(m, t->rl[2 * i], -1.0);
+  // (-1)^(k+1) / (k ln 2), k = 1..5
+  double s = __builtin_fma(r, 0.28853900817779268, -0.36067376022224085);
+  s = __builtin_fma(r, s, 0.48089834696298783);
+  s = __builtin_fma(r, s, -0.72134752044448170);
+  s = __builtin_fma(r, s, 1.4426950408889634);
+  const double nl = static_cast<double>(32 - e) - __builtin_fma(r, s, t->rl[2 * i + 1]);
+  const double fg = nl * inv;
+  const double fl = __builtin_floor(fg);
+  const double off = __builtin_fabs(fg - fl - 0.5);        // 0.5: right between two integers
+  if (off < __builtin_fma(inv, -0x1p-40, 0.5)) return static_cast<uint32_t>(fl);
+  return ic_gap_settle(hi, q, static_cast<uint32_t>(__builtin_rint(fg < 0.0 ? 0.0 : fg)));
 }
 
 }  // namespace rip

@@ -132,14 +132,14 @@ ic_fused_kernel(IcParams P) {
   __shared__ uint32_t s_hn[2];   // deferred-hub lists
   __shared__ uint32_t s_union;
   __shared__ Affine s_p2[64];      // P^(2^j): jumps between gap blocks
-  __shared__ IcLogTables s_tab;
+  __shared__ IcGapTab s_tab;
   __shared__ uint32_t s_ebeg[BT];
   __shared__ uint32_t s_edeg[BT];
   __shared__ uint32_t s_eT[BT];    // the row's largest threshold
   __shared__ uint32_t s_eflags[BT];
   __shared__ uint32_t s_eufull[BT];
   __shared__ uint32_t s_eulast[BT];
-  __shared__ unsigned long long s_erq[BT];
+  __shared__ double s_einv[BT];
   __shared__ uint32_t s_epre[BT];
   __shared__ unsigned long long s_eq[BT];
   __shared__ unsigned long long s_ea[BT];
@@ -245,7 +245,7 @@ ic_fused_kernel(IcParams P) {
           s_eflags[tid] = r.flags;
           s_eufull[tid] = r.ufull;
           s_eulast[tid] = r.ulast;
-          s_erq[tid] = r.rq;
+          s_einv[tid] = r.inv;
           s_eq[tid] = r.q;
           s_ea[tid] = r.ja;
           s_eb[tid] = r.jb;
@@ -269,7 +269,8 @@ ic_fused_kernel(IcParams P) {
           unsigned long long mm = 0;
           Affine E{1, 0};
           uint32_t e0 = 0, len = 0, B = 0, T = 0, uskip = 0;
-          uint64_t q = 0, rq = 0;
+          uint64_t q = 0;
+          double inv = 0.0;
           bool uniform = true;
           if (rr < total) {
             uint32_t lo = 0, hi = cl;
@@ -290,7 +291,7 @@ ic_fused_kernel(IcParams P) {
             // a block without candidates costs one compare: the full or
             // the partial last block's skip threshold
             uskip = len == B ? s_eufull[ent] : s_eulast[ent];
-            rq = s_erq[ent];
+            inv = s_einv[ent];
             uniform = (fl & kRowUniform) != 0;
             mm = s_em[ent];
             // block k's first element: P^(2 B k) after the row's first
@@ -316,12 +317,12 @@ ic_fused_kernel(IcParams P) {
                 if ((x >> 32) + 1 <= uskip) pos = len;
                 continue;
               }
-              const uint64_t gap = ic_gap_fast(x, q, rq, &s_tab);
+              const uint32_t gap = ic_gap_draw(x, q, inv, &s_tab);
               if (gap >= len - pos) {
                 pos = len;
                 continue;
               }
-              pos += static_cast<uint32_t>(gap);
+              pos += gap;
               const uint32_t e = e0 + pos;
               const uint64_t a = P.step.a * x + P.step.b;   // acceptance element
               ++st_edges;

@@ -237,11 +237,12 @@ __global__ void __launch_bounds__(64) grid_seed_kernel(GridParams P, const uint3
 template <int BT>
 struct ExpandLds {
   Affine p2[64];
-  IcLogTables tab;
+  IcGapTab tab;
   uint32_t tmp[BT / 64];
   uint32_t g[kExpItems], beg[kExpItems], deg[kExpItems], T[kExpItems], fl[kExpItems];
   uint32_t uf[kExpItems], ul[kExpItems], pre[kExpItems], nch[kExpItems], dpre[kExpItems];
-  unsigned long long q[kExpItems], rq[kExpItems], ja[kExpItems], jb[kExpItems], m[kExpItems];
+  unsigned long long q[kExpItems], ja[kExpItems], jb[kExpItems], m[kExpItems];
+  double inv[kExpItems];
   uint32_t ucur;   // next unit of the chunk not claimed by a wave
   // the dense round's tasks: entry, block, first element, prefix of colours,
   // and per task and position the colours live there
@@ -266,7 +267,8 @@ __device__ void expand_chunk(const GridParams &P, const unsigned long long *cur,
   Affine *s_p2 = S.p2;
   uint32_t *s_tmp = S.tmp, *s_g = S.g, *s_beg = S.beg, *s_deg = S.deg, *s_T = S.T, *s_fl = S.fl;
   uint32_t *s_uf = S.uf, *s_ul = S.ul, *s_pre = S.pre, *s_nch = S.nch, *s_dpre = S.dpre;
-  unsigned long long *s_q = S.q, *s_rq = S.rq, *s_ja = S.ja, *s_jb = S.jb, *s_m = S.m;
+  unsigned long long *s_q = S.q, *s_ja = S.ja, *s_jb = S.jb, *s_m = S.m;
+  double *s_inv = S.inv;
   unsigned long long &st_cand = st.cand, &st_draws = st.draws, &st_exp = st.exp;
   unsigned long long &st_bytes = st.bytes, &st_live = st.live;
   uint32_t units = 0, ntask = 0;
@@ -289,7 +291,7 @@ __device__ void expand_chunk(const GridParams &P, const unsigned long long *cur,
       s_uf[tid] = r.ufull;
       s_ul[tid] = r.ulast;
       s_q[tid] = r.q;
-      s_rq[tid] = r.rq;
+      s_inv[tid] = r.inv;
       s_ja[tid] = r.ja;
       s_jb[tid] = r.jb;
       s_m[tid] = M;
@@ -324,12 +326,13 @@ __device__ void expand_chunk(const GridParams &P, const unsigned long long *cur,
   // discovered together.
   const uint32_t lane = lane_id();
   {
-    const Affine Pst = s_p2[0];
+    const Affine Pst = uniform_affine(s_p2[0]), P2 = uniform_affine(s_p2[1]);
     uint32_t nxt = 0, hi = 0;   // the wave's claimed units [nxt, hi) (wave-uniform)
     bool has = false, started = false;
     uint32_t g = 0, e0 = 0, len = 0, pos = 0, T = 0, uskip = 0;
     unsigned long long bit = 0;
-    uint64_t q = 0, rq = 0, x = 0;
+    uint64_t q = 0, x = 0;
+    double inv = 0.0;
     bool uniform = true;
     // kSparseSteps steps per lane, then their live edges discovered together
     for (bool finished = false; !finished;) {
@@ -374,7 +377,7 @@ __device__ void expand_chunk(const GridParams &P, const unsigned long long *cur,
               T = s_T[ent];
               uskip = len == B ? s_uf[ent] : s_ul[ent];
               q = s_q[ent];
-              rq = s_rq[ent];
+              inv = s_inv[ent];
               uniform = (fl & kRowUniform) != 0;
               // block k's first element: P^(2 B k) after the row's first
               Affine E{s_ja[ent], s_jb[ent]};
@@ -400,21 +403,21 @@ __device__ void expand_chunk(const GridParams &P, const unsigned long long *cur,
             if ((x >> 32) + 1 <= uskip) has = false;
           }
           if (has) {
-            const uint64_t gap = ic_gap_fast(x, q, rq, &S.tab);
+            const uint32_t gap = ic_gap_draw(x, q, inv, &S.tab);
             if (gap >= len - pos) {
               has = false;
             } else {
-              pos += static_cast<uint32_t>(gap);
+              pos += gap;
               const uint32_t e = e0 + pos;
-              const uint64_t a = Pst.a * x + Pst.b;        // acceptance element
               ++st_cand;
+              bool live = true;
               if (!uniform) {
                 ++st_draws;
                 st_bytes += 4;
+                live = ic_accept(Pst.a * x + Pst.b, T, P.val[e]);   // acceptance element
               }
-              const bool live = uniform || ic_accept(a, T, P.val[e]);
               ++pos;
-              x = Pst.a * a + Pst.b;                       // next gap element
+              x = P2.a * x + P2.b;                         // next gap element
               if (pos < len) ++st_draws;
               else has = false;
               if (live) {
@@ -483,9 +486,10 @@ __device__ void expand_chunk(const GridParams &P, const unsigned long long *cur,
       const uint32_t len = min(s_deg[ent] - (k << beta), B);
       const uint32_t e0 = s_beg[ent] + (k << beta);
       const uint32_t T = s_T[ent];
-      const uint64_t q = s_q[ent], rq = s_rq[ent];
+      const uint64_t q = s_q[ent];
+      const double inv = s_inv[ent];
       const bool uniform = (fl & kRowUniform) != 0;
-      const Affine Pst = s_p2[0];
+      const Affine Pst = uniform_affine(s_p2[0]), P2 = uniform_affine(s_p2[1]);
       const Affine E = S.tE[t];
       uint64_t x = E.a * P.z[64ull * g + c] + E.b;
       ++st_draws;
@@ -504,25 +508,24 @@ __device__ void expand_chunk(const GridParams &P, const unsigned long long *cur,
           cp[j] = 0;
           ca[j] = 0;
           if (more) {
-            const uint64_t gap = ic_gap_fast(x, q, rq, &S.tab);
+            const uint32_t gap = ic_gap_draw(x, q, inv, &S.tab);
             if (gap >= len - pos) {
               more = false;
             } else {
-              pos += static_cast<uint32_t>(gap);
-              const uint64_t a = Pst.a * x + Pst.b;    // acceptance element
+              pos += gap;
               ++st_cand;
               if (!uniform) {
                 ++st_draws;
                 st_bytes += 4;
+                ca[j] = Pst.a * x + Pst.b;             // acceptance element
               }
               cp[j] = pos;
-              ca[j] = a;
               nc = j + 1;
               ++pos;
               if (pos >= len) {
                 more = false;
               } else {
-                x = Pst.a * a + Pst.b;                 // next gap element
+                x = P2.a * x + P2.b;                   // next gap element
                 ++st_draws;
               }
             }
@@ -576,7 +579,7 @@ __device__ void expand_chunk(const GridParams &P, const unsigned long long *cur,
 // (at most kExpItems) from the level's counter.  Levels are enqueued ahead of
 // the host: a level whose frontier is empty costs its launch only.
 template <int BT>
-__global__ void __launch_bounds__(BT) grid_level_kernel(GridParams P, uint32_t L) {
+__global__ void __launch_bounds__(BT, 3) grid_level_kernel(GridParams P, uint32_t L) {
   __shared__ ExpandLds<BT> S;
   __shared__ unsigned long long s_chunk;
   const uint32_t tid = threadIdx.x;
@@ -619,7 +622,7 @@ __global__ void __launch_bounds__(BT) grid_level_kernel(GridParams P, uint32_t L
 // number in gctl[kGTail]; that level's length stays in the ring for the
 // level kernels.
 template <int BT>
-__global__ void __launch_bounds__(BT) grid_tail_kernel(GridParams P, uint32_t L0,
+__global__ void __launch_bounds__(BT, 3) grid_tail_kernel(GridParams P, uint32_t L0,
                                                        uint64_t tail_cap) {
   __shared__ ExpandLds<BT> S;
   __shared__ unsigned long long s_n;

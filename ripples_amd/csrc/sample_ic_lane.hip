@@ -107,7 +107,7 @@ enum : uint32_t { kIdle = 0, kPop = 1, kRow = 2, kDone = 3 };
 template <int BT>
 __global__ void __launch_bounds__(BT) ic_lane_kernel(LaneParams P) {
   __shared__ Affine s_p2[64];
-  __shared__ IcLogTables s_tab;
+  __shared__ IcGapTab s_tab;
   if (threadIdx.x == 0) fill_step_powers(P.step, s_p2);
   ic_load_tables(&s_tab);
   __syncthreads();
@@ -117,7 +117,7 @@ __global__ void __launch_bounds__(BT) ic_lane_kernel(LaneParams P) {
   unsigned long long *table = P.table + gl * (static_cast<uint64_t>(P.tmask) + 1);
   uint32_t *list = P.list + gl * P.cap;
   uint32_t epoch = P.epoch[gl];
-  const Affine Pst = s_p2[0];
+  const Affine Pst = uniform_affine(s_p2[0]), P2 = uniform_affine(s_p2[1]);
   // wave-uniform: the claimed range of sample indices and the output chunk
   uint64_t next = 0, hi = 0;
   bool exhausted = false;
@@ -128,7 +128,8 @@ __global__ void __launch_bounds__(BT) ic_lane_kernel(LaneParams P) {
   unsigned long long tag = 0;
   uint32_t head = 0, tail = 0;
   uint32_t rbegin = 0, deg = 0, T = 0, beta = 0, nblk = 0, k = 0, pos = 0, len = 0;
-  uint64_t q = 0, rq = 0, ufull = 0, ulast = 0, xb = 0, x = 0;
+  uint64_t q = 0, ufull = 0, ulast = 0, xb = 0, x = 0;
+  double inv = 0.0;
   bool uniform = true;
   unsigned long long st_cand = 0, st_draws = 0, st_exp = 0, st_bytes = 0, st_live = 0;
 
@@ -183,7 +184,7 @@ __global__ void __launch_bounds__(BT) ic_lane_kernel(LaneParams P) {
           q = rv.q;
           ufull = rv.ufull;
           ulast = rv.ulast;
-          rq = rv.rq;
+          inv = rv.inv;
           nblk = ((deg - 1) >> beta) + 1;
           k = 0;
           xb = rv.ja * z + rv.jb;                  // the row's first element
@@ -212,21 +213,21 @@ __global__ void __launch_bounds__(BT) ic_lane_kernel(LaneParams P) {
           state = kPop;
         }
       } else {
-        const uint64_t gap = ic_gap_fast(x, q, rq, &s_tab);
+        const uint32_t gap = ic_gap_draw(x, q, inv, &s_tab);
         if (gap >= len - pos) {
           pos = len;
         } else {
-          pos += static_cast<uint32_t>(gap);
+          pos += gap;
           const uint32_t e = rbegin + (k << beta) + pos;
-          const uint64_t a = Pst.a * x + Pst.b;      // acceptance element
           ++st_cand;
+          bool live = true;
           if (!uniform) {
             ++st_draws;
             st_bytes += 4;
+            live = ic_accept(Pst.a * x + Pst.b, T, P.val[e]);   // acceptance element
           }
-          const bool live = uniform || ic_accept(a, T, P.val[e]);
           ++pos;
-          x = Pst.a * a + Pst.b;                     // next gap element
+          x = P2.a * x + P2.b;                       // next gap element
           if (pos < len) ++st_draws;
           if (live) {
             ++st_live;

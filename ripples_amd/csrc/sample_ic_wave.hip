@@ -122,7 +122,7 @@ __device__ inline bool lds_find(const uint32_t *t, uint32_t mask, uint32_t v) {
 template <typename Visit>
 __device__ inline bool expand_row(const VertexRec *vrec, const uint32_t *ids,
                                   const uint32_t *val, uint32_t v, uint64_t z,
-                                  const Affine *p2, const IcLogTables *tab, uint32_t *list,
+                                  const Affine *p2, const IcGapTab *tab, uint32_t *list,
                                   uint32_t &tail, uint32_t cap,
                                   unsigned long long &st_cand, unsigned long long &st_draws,
                                   unsigned long long &st_bytes, unsigned long long &st_live,
@@ -141,9 +141,9 @@ __device__ inline bool expand_row(const VertexRec *vrec, const uint32_t *ids,
   const uint64_t q = uniform_u64(rv.q);
   const uint64_t ufull = uniform_u32(rv.ufull);
   const uint64_t ulast = uniform_u32(rv.ulast);
-  const uint64_t rq = uniform_u64(rv.rq);
+  const double inv = rv.inv;
   const uint32_t nblk = ((deg - 1) >> beta) + 1;
-  const Affine P = p2[0];
+  const Affine P = uniform_affine(p2[0]), P2 = uniform_affine(p2[1]);
   const uint64_t x0 = uniform_u64(rv.ja) * z + uniform_u64(rv.jb);  // row's first element
   // this lane's first block: P^(2B lane) from the binary digits of lane
   Affine jl{1, 0};
@@ -169,25 +169,25 @@ __device__ inline bool expand_row(const VertexRec *vrec, const uint32_t *ids,
       if (pos < len) {
         if (!first) ++st_draws;
         first = false;
-        const uint64_t gap = ic_gap_fast(x, q, rq, tab);
+        const uint32_t gap = ic_gap_draw(x, q, inv, tab);
         if (gap >= len - pos) {
           pos = len;
         } else {
-          pos += static_cast<uint32_t>(gap);
+          pos += gap;
           e = rbegin + (k << beta) + pos;
-          const uint64_t a = aff_apply(P, x);     // acceptance element
           ++st_cand;
+          live = true;
           if (!uniform) {
             ++st_draws;
             st_bytes += 4;
+            live = ic_accept(aff_apply(P, x), T, val[e]);   // acceptance element
           }
-          live = uniform || ic_accept(a, T, val[e]);
           if (live) {
             ++st_live;
             st_bytes += 4;
           }
           ++pos;
-          x = aff_apply(P, a);                     // next gap element
+          x = aff_apply(P2, x);                    // next gap element
         }
       }
       const uint64_t lm = __ballot(live);
@@ -226,7 +226,7 @@ constexpr uint32_t kUnitBatch = 4;
 template <typename Visit>
 __device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *val, bool have,
                                          const VertexRec &rv, uint64_t z,
-                                         const Affine *p2, const IcLogTables *tab,
+                                         const Affine *p2, const IcGapTab *tab,
                                          uint32_t *list, uint32_t &tail, uint32_t cap,
                                          unsigned long long &st_cand,
                                          unsigned long long &st_draws,
@@ -240,10 +240,11 @@ __device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *va
   const bool single = __ballot(nblk > 1) == 0;     // a lane's unit is its own row
   const uint32_t incl = single ? 0u : wave_inclusive_scan(nblk);
   const uint32_t total = single ? 64u : uniform_u32(__shfl(incl, 63, 64));
-  const Affine P = p2[0];
+  const Affine P = uniform_affine(p2[0]), P2 = uniform_affine(p2[1]);
   for (uint32_t u0 = 0; u0 < total; u0 += 64) {
     uint32_t e0 = rv.begin, len = 0, T = rv.thr;
-    uint64_t q = rv.q, rq = rv.rq, x = x0;
+    uint64_t q = rv.q, x = x0;
+    double inv = rv.inv;
     bool uniform = (rv.flags & kRowUniform) != 0;
     bool skip = true;
     if (single) {
@@ -269,7 +270,7 @@ __device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *va
       const uint32_t ufull = __shfl(rv.ufull, src, 64), ulast = __shfl(rv.ulast, src, 64);
       T = __shfl(rv.thr, src, 64);
       q = __shfl(rv.q, src, 64);
-      rq = __shfl(rv.rq, src, 64);
+      inv = __shfl(rv.inv, src, 64);
       x = __shfl(x0, src, 64);
       uniform = (flags & kRowUniform) != 0;
       if (u < total) {
@@ -294,19 +295,19 @@ __device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *va
         ce[i] = 0;
         th[i] = 0;
         if (more) {
-          const uint64_t gap = ic_gap_fast(x, q, rq, tab);
+          const uint32_t gap = ic_gap_draw(x, q, inv, tab);
           if (gap >= len - pos) {
             more = false;
           } else {
-            pos += static_cast<uint32_t>(gap);
-            const uint64_t a = aff_apply(P, x);    // acceptance element
+            pos += gap;
             ce[i] = e0 + pos;
             // kept iff the edge's threshold t passes this (ic_accept:
-            // hi32(a) T < t 2^32)
-            th[i] = static_cast<uint32_t>(((a >> 32) * T) >> 32);
+            // hi32(a) T < t 2^32 for the acceptance element a)
+            if (!uniform)
+              th[i] = static_cast<uint32_t>(((aff_apply(P, x) >> 32) * T) >> 32);
             nc = i + 1;
             if (++pos < len) {
-              x = aff_apply(P, a);                 // next gap element
+              x = aff_apply(P2, x);                // next gap element
               ++st_draws;
             } else {
               more = false;
@@ -353,7 +354,7 @@ __device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *va
 // one row per step over its gap blocks (expand_row, the plain form), with
 // the first vertices of each sample marked in LDS.
 template <int BT, bool VP>
-__global__ void __launch_bounds__(BT) ic_wave_kernel(WaveParams P) {
+__global__ void __launch_bounds__(BT, 4) ic_wave_kernel(WaveParams P) {
   constexpr int NW = BT / 64;
   constexpr uint32_t kBuf = VP && kWaveLdsSlots > kSortCap ? kWaveLdsSlots : kSortCap;
   __shared__ uint32_t s_sort[NW][kBuf];
@@ -368,7 +369,7 @@ __global__ void __launch_bounds__(BT) ic_wave_kernel(WaveParams P) {
   // of a chunk that cannot take the next set stays a gap in the pool's data
   unsigned long long out_cur = 0, out_end = 0;
   __shared__ Affine s_p2[64];                 // P^(2^j): jumps between gap blocks
-  __shared__ IcLogTables s_tab;
+  __shared__ IcGapTab s_tab;
   if (threadIdx.x == 0) fill_step_powers(P.step, s_p2);
   ic_load_tables(&s_tab);
   __syncthreads();
@@ -534,7 +535,7 @@ __global__ void __launch_bounds__(BT) ic_big_kernel(BigParams P) {
   uint32_t *sum = P.sum + wave * P.swords;
   uint32_t *list = P.list + wave * P.n;
   __shared__ Affine s_p2[64];
-  __shared__ IcLogTables s_tab;
+  __shared__ IcGapTab s_tab;
   if (threadIdx.x == 0) fill_step_powers(P.step, s_p2);
   ic_load_tables(&s_tab);
   __syncthreads();
