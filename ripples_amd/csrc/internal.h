@@ -142,10 +142,20 @@ struct SelectScratch {
   unsigned long long *d_soff = nullptr;  // cap_sets + 1: each set's first pair
   void *d_stemp = nullptr;               // the sort's temporary storage
   size_t stemp_bytes = 0;
+  // plain pools (select_top.hip): the counts' buckets, the candidates and the
+  // sets that hold them
+  uint64_t cap_part = 0, cap_top_sets = 0, cap_members = 0;
+  uint32_t top_n = 0;
+  uint32_t *d_part = nullptr;          // bucket tables and members by bucket
+  uint8_t *d_top = nullptr;            // the rounds' state
+  uint16_t *d_rank = nullptr;          // n: rank among the candidates
+  uint32_t *d_cand = nullptr;          // candidates, counts, index starts and cursors, tie tiles
+  uint8_t *d_rec = nullptr;            // cap_top_sets records of the candidates each set holds
+  uint16_t *d_members = nullptr;       // cap_members: ranks of the sets that hold many
   uint32_t *d_kill = nullptr;          // cap_kill: dense pools' kill list
   uint64_t cap_kill = 0;
   uint8_t *d_covered = nullptr;        // cap_sets
-  unsigned long long *d_keys = nullptr;  // per-seed argmax keys (k)
+  unsigned long long *d_keys = nullptr;  // per-seed argmax keys (k); plain pools: the seeds
   unsigned long long *d_partial = nullptr;  // kArgmaxBlocks per-block maxima
   uint32_t cap_k = 0;
   // The k rounds of argmax + kill as one HIP graph, captured for graph_k
@@ -399,6 +409,12 @@ uint64_t coverage_run(rip_pool *p, uint64_t num_sets, const uint32_t *seeds,
 // buffers: no device memory is allocated or freed
 uint64_t coverage_run_noalloc(rip_pool *p, uint64_t num_sets, const uint32_t *seeds,
                               uint32_t num_seeds);
+
+// select_top.hip: occurrence counts of a plain pool's sets, and greedy
+// selection among the vertices of largest count
+void count_plain(rip_pool *p, uint64_t num_sets, uint64_t total, const uint8_t *covered);
+uint32_t select_top(rip_pool *p, uint64_t num_sets, uint64_t total, uint32_t k, uint32_t *seeds,
+                    uint64_t *covered, bool *finished);
 
 // scan.hip: exclusive scan of uint32 values into uint64 prefixes (n + 1 out)
 // select_sort.hip: sorts `count` (key, value) pairs by the low `bits` bits

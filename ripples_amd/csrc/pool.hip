@@ -267,6 +267,12 @@ void pool_destroy(rip_pool *p) {
   dev_free(p->sel.d_pval);
   dev_free(p->sel.d_soff);
   dev_free(p->sel.d_stemp);
+  dev_free(p->sel.d_part);
+  dev_free(p->sel.d_top);
+  dev_free(p->sel.d_rank);
+  dev_free(p->sel.d_cand);
+  dev_free(p->sel.d_rec);
+  dev_free(p->sel.d_members);
   dev_free(p->sel.d_kill);
   dev_free(p->sel.d_covered);
   dev_free(p->sel.d_keys);

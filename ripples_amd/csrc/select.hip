@@ -4,14 +4,17 @@
 // streaming_find_most_influential.h:607-643) with lowest-id ties as
 // GPUMaxElement (src/gpu/find_most_influential.cc:65-72):
 //   1. counts[v] = number of sets containing v          (counting.h:65-97)
-//   2. inverted index vertex -> sets by counting sort
-//   3. k times: argmax of counts (key = count<<32 | ~v, so the largest key is
-//      the largest count with the lowest id), then a kill pass that visits
-//      only the sets containing the new seed, marks the uncovered ones
+//   2. plain pools: rounds among the vertices of largest count
+//      (select_top.hip), which finish nearly every selection
+//   3. otherwise, k times: argmax of counts (key = count<<32 | ~v, so the
+//      largest key is the largest count with the lowest id), then a kill pass
+//      over the uncovered sets containing the new seed -- found through an
+//      inverted index (plain pools whose candidates share their sets) or by a
+//      scan (dense pools and pools with column sets) -- that marks them
 //      covered and decrements the counts of their members.
 // Every set is killed at most once, so the kill passes cost O(T) over all k
 // seeds, where the reference recounts every uncovered set per seed
-// (gpu/find_most_influential.h:98-120).  The 2k kernels of the seed loop run
+// (gpu/find_most_influential.h:98-120).  The kernels of the seed loop of 3 run
 // as one HIP graph with no host synchronisation; the host reads the k keys
 // once.
 #include <algorithm>
@@ -19,38 +22,13 @@
 
 #include "device_util.h"
 #include "internal.h"
+#include "select_common.h"
 
 namespace rip {
 namespace {
 
 constexpr uint32_t kBT = 256;
 constexpr uint32_t kArgmaxBlocks = 1024;  // most blocks of an argmax pass
-
-// Each lane of a wave holds one run (off, len) of `data`; the wave visits
-// every element of the 64 runs once, lanes taking elements of any run:
-// f(value, run index).
-template <typename F>
-__device__ inline void for_each_run_element(unsigned long long off, uint32_t len,
-                                            const uint32_t *data, uint32_t *s_pre,
-                                            unsigned long long *s_off, F &&f) {
-  const uint32_t lane = lane_id();
-  s_off[lane] = off;
-  const uint32_t incl = wave_inclusive_scan(len);
-  s_pre[lane + 1] = incl;
-  if (lane == 0) s_pre[0] = 0;
-  const uint32_t total = __shfl(incl, 63, 64);
-  __builtin_amdgcn_wave_barrier();
-  for (uint32_t i = lane; i < total; i += 64) {
-    uint32_t lo = 0, hi = 64;
-    while (lo < hi) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (s_pre[mid + 1] <= i) lo = mid + 1;
-      else hi = mid;
-    }
-    f(data[s_off[lo] + (i - s_pre[lo])], lo);
-  }
-  __builtin_amdgcn_wave_barrier();
-}
 
 // Each wave walks 64 consecutive sets; lanes take elements of any of them.
 template <typename F>
@@ -72,15 +50,6 @@ __device__ inline void for_each_element(const unsigned long long *set_off,
 }
 
 __global__ void __launch_bounds__(kBT)
-count_kernel(const unsigned long long *set_off, const uint32_t *set_len,
-             const uint32_t *data, uint64_t num_sets, uint32_t *counts) {
-  __shared__ uint32_t s_pre[kBT / 64][65];
-  __shared__ unsigned long long s_off[kBT / 64][64];
-  for_each_element(set_off, set_len, data, num_sets, s_pre, s_off,
-                   [&](uint32_t v, uint64_t) { atomicAdd(&counts[v], 1u); });
-}
-
-__global__ void __launch_bounds__(kBT)
 fill_inverted_kernel(const unsigned long long *set_off, const uint32_t *set_len,
                      const uint32_t *data, uint64_t num_sets,
                      unsigned long long *cursor, uint32_t *inv) {
@@ -96,8 +65,8 @@ fill_inverted_kernel(const unsigned long long *set_off, const uint32_t *set_len,
 // ------------------------------------------------------------ sorted index
 // Sparse pools of kSortMinPairs to kSortMaxPairs elements build the inverted
 // index by sorting their (vertex, set) pairs by vertex: no atomic per
-// element, where the count and fill passes above make one each (and the hub
-// vertices of R-MAT graphs share their counters).  Below the minimum the
+// element, where the fill pass above makes one each (and the hub vertices of
+// R-MAT graphs share their cursors).  Below the minimum the
 // sort's fixed costs (its buffers, a scan) outweigh the atomics: IMM on
 // R-MAT scale 20 LT (pools of up to 3.5M elements) took 19 ms with the sort
 // against 16 ms without; at 60M elements the index takes 2.1 ms against 13.9.
@@ -315,14 +284,6 @@ __global__ void zero_word_kernel(unsigned long long *w) { *w = 0; }
 __global__ void clear_keys_kernel(const Args *a, uint32_t k) {
   for (uint32_t i = threadIdx.x; i < k; i += blockDim.x) a->keys[i] = 0;
   if (threadIdx.x == 0) a->ctl[kCtlCovered] = 0;
-}
-
-__device__ inline unsigned long long wave_max_u64(unsigned long long x) {
-  for (int d = 32; d > 0; d >>= 1) {
-    const unsigned long long y = __shfl_xor(x, d, 64);
-    x = y > x ? y : x;
-  }
-  return x;
 }
 
 __device__ inline unsigned long long block_max_u64(unsigned long long x,
@@ -742,11 +703,6 @@ void ensure_select_scratch(rip_pool *p, uint64_t num_sets, uint64_t inv_elems,
   if (!s.d_partial) s.d_partial = dev_alloc<unsigned long long>(kArgmaxBlocks);
 }
 
-uint32_t grid_for(uint64_t work, uint32_t per_block, uint32_t cap) {
-  uint64_t g = (work + per_block - 1) / per_block;
-  return static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(g, cap)));
-}
-
 constexpr uint64_t kDenseMinElements = 1ull << 22;
 
 uint32_t ranges_of(uint32_t n) { return (n + kDenseRange - 1) / kDenseRange; }
@@ -802,55 +758,49 @@ const uint32_t *inverted_by_sort(rip_pool *p, uint64_t num_sets, uint64_t total)
 }
 
 // counts over sets [0, num_sets) and the scratch a selection needs; returns
-// whether the pool takes the dense path.  *sorted_inv (selections only): the
-// inverted index when it was built here by sorting, else nullptr.
-bool build_counts(rip_pool *p, uint64_t num_sets, uint32_t k, Need need,
-                  const uint32_t **sorted_inv = nullptr) {
-  if (sorted_inv) *sorted_inv = nullptr;
+// whether the pool takes the dense path.  *members: set members in its lists.
+bool build_counts(rip_pool *p, uint64_t num_sets, uint32_t k, Need need, uint64_t *members) {
   RIP_REQUIRE(num_sets <= p->num_sets, -1, "select: num_sets beyond the pool");
   const uint32_t n = p->g->n;
   hipStream_t st = p->stream;
   RIP_HIP(hipSetDevice(p->g->device));
-  // total element count
-  hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(1), 0, st, p->d_ctl + kCtlWords - 1);
-  launch_sum_u32(p->d_len, num_sets, p->d_ctl + kCtlWords - 1, st);
-  unsigned long long total = 0;
-  RIP_HIP(hipMemcpyAsync(&total, p->d_ctl + kCtlWords - 1, sizeof(total),
-                         hipMemcpyDeviceToHost, st));
-  RIP_HIP(hipStreamSynchronize(st));
   // pools with column sets take the dense kernels, whose seed rounds scan
   // every uncovered set and so also test the column sets' hot members
   const bool cols = p->groups > 0;
+  // total element count: known for the whole of a pool without columns
+  unsigned long long total = p->num_elements;
+  if (cols || num_sets != p->num_sets) {
+    hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(1), 0, st, p->d_ctl + kCtlWords - 1);
+    launch_sum_u32(p->d_len, num_sets, p->d_ctl + kCtlWords - 1, st);
+    RIP_HIP(hipMemcpyAsync(&total, p->d_ctl + kCtlWords - 1, sizeof(total),
+                           hipMemcpyDeviceToHost, st));
+    RIP_HIP(hipStreamSynchronize(st));
+  }
+  *members = total;
   const bool dense = cols ? num_sets > 0 : is_dense(n, num_sets, total);
   const bool sel = need == Need::Select;
   ensure_select_scratch(p, sel ? num_sets : 0, sel && !dense ? total : 0,
                         sel && dense ? num_sets : 0, k);
   SelectScratch &s = p->sel;
+  if (!dense) {
+    count_plain(p, num_sets, total, nullptr);
+    return false;
+  }
   hipLaunchKernelGGL(fill_u32_kernel, dim3(grid_for(n, kBT, 2048)), dim3(kBT), 0, st,
                      s.d_counts, static_cast<uint64_t>(n), 0u);
-  if (dense) {
-    const uint32_t ranges = ranges_of(n);
-    hipLaunchKernelGGL(dense_count_kernel, dim3(dense_chunks(ranges, num_sets) * ranges),
-                       dim3(kDenseBT), 0, st, p->d_off, p->d_len, p->d_data, num_sets, n,
-                       ranges, s.d_counts);
-    if (cols) {
-      hipLaunchKernelGGL(group_active_kernel, dim3(grid_for(p->groups, kBT, 1024)), dim3(kBT), 0,
-                         st, p->d_gsample, p->groups, num_sets, s.d_gactive, s.d_gkill);
-      hipLaunchKernelGGL(hot_count_kernel, dim3(grid_for(p->g->hot_n, kBT, 8192)), dim3(kBT), 0,
-                         st, p->d_colptr, s.d_gactive, p->groups, p->g->d_hot_vertex,
-                         p->g->hot_n, s.d_counts);
-    }
-  } else if (num_sets) {
-    if (sel && sorted_inv && total >= kSortMinPairs && total <= kSortMaxPairs) {
-      *sorted_inv = inverted_by_sort(p, num_sets, total);
-    } else {
-      hipLaunchKernelGGL(count_kernel, dim3(grid_for(num_sets, 64 * (kBT / 64), 8192)),
-                         dim3(kBT), 0, st, p->d_off, p->d_len, p->d_data, num_sets,
-                         s.d_counts);
-    }
+  const uint32_t ranges = ranges_of(n);
+  hipLaunchKernelGGL(dense_count_kernel, dim3(dense_chunks(ranges, num_sets) * ranges),
+                     dim3(kDenseBT), 0, st, p->d_off, p->d_len, p->d_data, num_sets, n,
+                     ranges, s.d_counts);
+  if (cols) {
+    hipLaunchKernelGGL(group_active_kernel, dim3(grid_for(p->groups, kBT, 1024)), dim3(kBT), 0,
+                       st, p->d_gsample, p->groups, num_sets, s.d_gactive, s.d_gkill);
+    hipLaunchKernelGGL(hot_count_kernel, dim3(grid_for(p->g->hot_n, kBT, 8192)), dim3(kBT), 0,
+                       st, p->d_colptr, s.d_gactive, p->groups, p->g->d_hot_vertex,
+                       p->g->hot_n, s.d_counts);
   }
   RIP_HIP(hipGetLastError());
-  return dense;
+  return true;
 }
 
 // Captures clear + k seed rounds on the pool's stream as an executable graph:
@@ -906,29 +856,55 @@ void capture_rounds(rip_pool *p, uint32_t k, bool dense, bool cols) {
 
 }  // namespace
 
-uint32_t select_run(rip_pool *p, uint64_t num_sets, uint32_t k, uint32_t *seeds,
+// The full inverted index of plain sets [0, num_sets) (total members): by
+// sorting their pairs or, for smaller pools, by counting and atomics.
+// Returns where it is; d_counts is overwritten.
+static const uint32_t *inverted_index(rip_pool *p, uint64_t num_sets, uint64_t total) {
+  SelectScratch &s = p->sel;
+  hipStream_t st = p->stream;
+  const uint32_t n = p->g->n;
+  if (total >= kSortMinPairs && total <= kSortMaxPairs) return inverted_by_sort(p, num_sets, total);
+  count_plain(p, num_sets, total, nullptr);
+  exclusive_scan_u32(s.d_counts, s.d_inv_start, n, st);
+  hipLaunchKernelGGL(copy_u64_kernel, dim3(grid_for(n, kBT, 2048)), dim3(kBT), 0, st,
+                     s.d_cursor, s.d_inv_start, static_cast<uint64_t>(n));
+  if (num_sets)
+    hipLaunchKernelGGL(fill_inverted_kernel, dim3(grid_for(num_sets, 64 * (kBT / 64), 8192)),
+                       dim3(kBT), 0, st, p->d_off, p->d_len, p->d_data, num_sets, s.d_cursor,
+                       s.d_inv);
+  return s.d_inv;
+}
+
+uint32_t select_run(rip_pool *p, uint64_t num_sets, uint32_t k_total, uint32_t *seeds,
                     uint64_t *covered) {
   const uint32_t n = p->g->n;
   hipStream_t st = p->stream;
-  const uint32_t *sorted_inv = nullptr;
-  const bool dense = build_counts(p, num_sets, std::max<uint32_t>(k, 1), Need::Select,
-                                  &sorted_inv);
+  uint64_t total = 0;
+  const bool dense = build_counts(p, num_sets, std::max<uint32_t>(k_total, 1), Need::Select, &total);
   SelectScratch &s = p->sel;
-  if (!dense && !sorted_inv) {
-    exclusive_scan_u32(s.d_counts, s.d_inv_start, n, st);
-    hipLaunchKernelGGL(copy_u64_kernel, dim3(grid_for(n, kBT, 2048)), dim3(kBT), 0, st,
-                       s.d_cursor, s.d_inv_start, static_cast<uint64_t>(n));
-    if (num_sets)
-      hipLaunchKernelGGL(fill_inverted_kernel,
-                         dim3(grid_for(num_sets, 64 * (kBT / 64), 8192)), dim3(kBT), 0, st,
-                         p->d_off, p->d_len, p->d_data, num_sets, s.d_cursor, s.d_inv);
-  }
   hipLaunchKernelGGL(fill_u8_kernel, dim3(grid_for(num_sets, kBT, 2048)), dim3(kBT), 0, st,
                      s.d_covered, num_sets);
+  // plain pools: the rounds run on the vertices of largest count
+  uint32_t done = 0;
+  uint64_t done_cov = 0;
+  const uint32_t *inv = s.d_inv;
+  if (!dense && k_total) {
+    bool finished = false;
+    if (total <= kSortMaxPairs)
+      done = select_top(p, num_sets, total, k_total, seeds, &done_cov, &finished);
+    if (finished) {
+      if (covered) *covered = done_cov;
+      return done;
+    }
+    // the rest over all vertices, from the full index
+    inv = inverted_index(p, num_sets, total);
+    count_plain(p, num_sets, total, done ? s.d_covered : nullptr);
+  }
+  const uint32_t k = k_total - done;
   // the seed rounds run as one graph; this call's buffers travel in d_args
   // (`args` stays alive until the stream is synchronised below)
   const bool cols = p->groups > 0;
-  const Args args{s.d_counts, s.d_inv_start, sorted_inv ? sorted_inv : s.d_inv, p->d_off,
+  const Args args{s.d_counts, s.d_inv_start, inv, p->d_off,
                   p->d_len, p->d_data,
                   s.d_covered, s.d_keys, p->d_ctl, s.d_kill, s.d_partial, num_sets, n,
                   p->d_gref, p->d_colptr, p->g->d_hot_index, p->g->d_hot_vertex, s.d_gkill,
@@ -950,12 +926,12 @@ uint32_t select_run(rip_pool *p, uint64_t num_sets, uint32_t k, uint32_t *seeds,
   RIP_HIP(hipMemcpyAsync(&cov, p->d_ctl + kCtlCovered, sizeof(cov),
                          hipMemcpyDeviceToHost, st));
   RIP_HIP(hipStreamSynchronize(st));
-  uint32_t got = 0;
+  uint32_t got = done;
   for (uint32_t i = 0; i < k; ++i) {
     if ((keys[i] >> 32) == 0) break;
     seeds[got++] = 0xFFFFFFFFu - static_cast<uint32_t>(keys[i]);
   }
-  if (covered) *covered = cov;
+  if (covered) *covered = done_cov + cov;
   return got;
 }
 
@@ -1102,7 +1078,8 @@ uint64_t coverage_run_noalloc(rip_pool *p, uint64_t num_sets, const uint32_t *se
 }
 
 void count_run(rip_pool *p, uint64_t num_sets, uint32_t *counts_host) {
-  build_counts(p, num_sets, 1, Need::Counts);
+  uint64_t total = 0;
+  build_counts(p, num_sets, 1, Need::Counts, &total);
   RIP_HIP(hipMemcpyAsync(counts_host, p->sel.d_counts, sizeof(uint32_t) * p->g->n,
                          hipMemcpyDeviceToHost, p->stream));
   RIP_HIP(hipStreamSynchronize(p->stream));
