@@ -65,18 +65,21 @@ typedef struct {
                             are found again by a scan of the pending masks */
   uint32_t wave_stage;   /* IC AUTO: nonzero (or queue_cap 0) = samples passing queue_cap are
                             first run one per wave, 64 frontier vertices at a
-                            time, up to 4096 vertices, and only the larger
-                            ones go to the grid sampler; calls of up to 16,384
-                            samples start there, with no lanes before */
+                            time, up to 4096 vertices (1024 on graphs of up to
+                            2^20 vertices), and only the larger ones go on;
+                            calls of up to 16,384 samples start there, with no
+                            lanes before */
 } rip_tune;
 
 /* IC sampler kinds (all give the same sets):
  *   AUTO    one reverse BFS per lane (64 samples per wave); samples passing
  *           queue_cap vertices go to one BFS per wave expanding 64 queued
  *           vertices at a time (the wave stage; not with a queue_cap given
- *           and wave_stage 0), and past 4096 vertices to the grid sampler:
- *           64-sample colour groups, many groups per batch, one BFS level of
- *           all of them per kernel
+ *           and wave_stage 0), and larger ones to a workgroup each with its
+ *           visited vertices in LDS (graphs of up to 2^20 vertices, no colors
+ *           or frontier_cap given) or to the grid sampler: 64-sample colour
+ *           groups, many groups per batch, one BFS level of all of them per
+ *           kernel
  *   WAVE    one reverse BFS per wave for every sample (the plain form), sets
  *           passing 4096 vertices finished by a bitmap-visited BFS per wave
  *   COLOUR  64-sample colour groups for every sample
@@ -247,10 +250,11 @@ int rip_pool_coverage_noalloc(rip_pool *p, uint64_t num_sets, const uint32_t *se
  * LT: the walk kernel), measured with HIP events on the pool's
  * stream, and the number of kernel launches of the call. */
 int rip_pool_last_kernel_ms(const rip_pool *p, double *ms, uint32_t *launches);
-/* The grid sampler's share of the last rip_pool_sample call (IC, AUTO: the
- * samples that outgrew a lane): the summed device time of its BFS level
- * kernels (HIP events on the pool's stream), how many levels ran (0 when no
- * sample reached it), and the work counters of its kernels (RIP_STAT_*
+/* The large sets' share of the last rip_pool_sample call (IC, AUTO: the
+ * samples that outgrew lanes and waves): the summed device time of the grid
+ * sampler's BFS level kernels, or the time of the one-sample-per-workgroup
+ * kernels (HIP events on the pool's stream), how many levels, or such kernels,
+ * ran (0 when no sample came that far), and the work counters of its kernels (RIP_STAT_*
  * order, as rip_pool_last_stats) into stats[0 .. count). */
 int rip_pool_last_grid(const rip_pool *p, double *ms, uint32_t *levels, uint64_t *stats,
                        uint32_t count);

@@ -164,22 +164,29 @@ void graph_ensure_hot(rip_graph *g, hipStream_t st) {
   std::vector<uint32_t> index(n, kNotHot), vertex(order.begin(), order.begin() + hot);
   std::sort(vertex.begin(), vertex.end());
   for (uint32_t h = 0; h < hot; ++h) index[vertex[h]] = h;
+  std::vector<uint32_t> mask((static_cast<size_t>(n) + 31) / 32, 0u);
+  for (const uint32_t v : vertex) mask[v >> 5] |= 1u << (v & 31u);
   uint32_t *d_index = dev_alloc<uint32_t>(n);
-  uint32_t *d_vertex = nullptr;
+  uint32_t *d_vertex = nullptr, *d_mask = nullptr;
   try {
     d_vertex = dev_alloc<uint32_t>(hot);
+    d_mask = dev_alloc<uint32_t>(mask.size());
     RIP_HIP(hipMemcpyAsync(d_index, index.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice,
                            st));
     RIP_HIP(hipMemcpyAsync(d_vertex, vertex.data(), sizeof(uint32_t) * hot,
+                           hipMemcpyHostToDevice, st));
+    RIP_HIP(hipMemcpyAsync(d_mask, mask.data(), sizeof(uint32_t) * mask.size(),
                            hipMemcpyHostToDevice, st));
     RIP_HIP(hipStreamSynchronize(st));
   } catch (...) {
     dev_free(d_index);
     dev_free(d_vertex);
+    dev_free(d_mask);
     throw;
   }
   g->d_hot_index = d_index;
   g->d_hot_vertex = d_vertex;
+  g->d_hot_mask = d_mask;
   g->hot_n = hot;
 }
 
@@ -341,6 +348,7 @@ void graph_destroy(rip_graph *g) {
   dev_free(g->d_vrec);
   dev_free(g->d_hot_index);
   dev_free(g->d_hot_vertex);
+  dev_free(g->d_hot_mask);
   dev_free(g->d_ids);
   dev_free(g->d_val);
   dev_free(g->ic.d_vp);
@@ -361,6 +369,7 @@ void graph_destroy(rip_graph *g) {
   dev_free(g->wave.d_over);
   dev_free(g->wave.d_lsort);
   grid_scratch_free(g->grid);
+  team_scratch_free(g->team);
   dev_free(g->lt.d_long_ids);
   dev_free(g->lt.d_spill);
   dev_free(g->d_bp);

@@ -82,6 +82,16 @@ struct GridScratch {
   unsigned long long *h_ctl = nullptr;
 };
 
+// Scratch of the team IC sampler (sample_ic_team.hip): per resident workgroup
+// a BFS queue of n vertices; per sample of a batch its visited bitmap, size
+// and hot members; per colour group of the batch its output tables.
+struct TeamScratch {
+  uint64_t queue_words = 0, row_words = 0, samples = 0;
+  uint32_t *d_queue = nullptr;
+  uint32_t *d_rows = nullptr;
+  uint32_t *d_tables = nullptr;
+};
+
 // Forward CSR and per-workgroup scratch of the spread simulator, built on
 // first use (spread.hip).
 struct FwdGraph {
@@ -197,6 +207,7 @@ struct rip_graph {
   uint32_t hot_n = 0;
   uint32_t *d_hot_index = nullptr;   // n: index among the hot vertices, or kNotHot
   uint32_t *d_hot_vertex = nullptr;  // hot_n: the hot vertices, ascending
+  uint32_t *d_hot_mask = nullptr;    // n bits: who is hot
   // Sampler settings chosen by the autotuner (tune.cpp), used by sampling
   // calls that pass none.
   rip_tune tuned{};
@@ -211,6 +222,7 @@ struct rip_graph {
   rip::IcSlots ic;
   rip::WaveScratch wave;
   rip::GridScratch grid;
+  rip::TeamScratch team;
   rip::LtScratch lt;
   rip::FwdGraph fwd;
 };
@@ -247,10 +259,12 @@ struct rip_pool {
   rip::SelectScratch sel;
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;
   hipEvent_t ev3 = nullptr, ev4 = nullptr;  // around each grid-sampler level
-  double grid_ms = 0.0;       // last sampling call: the grid sampler's level kernels
+  double grid_ms = 0.0;       // last sampling call: the grid sampler's level kernels, or the
+                              // team sampler's kernels
   uint32_t grid_levels = 0;   // and how many ran
   double wave_ms = 0.0;       // last sampling call: the wave stage's kernel (AUTO)
   bool wave_ran = false;
+  bool team_ran = false;      // the team sampler: its kernels lie between ev3 and ev4
   uint64_t wave_stats[RIP_STAT_COUNT] = {};  // last_stats as they stood after it
   double last_kernel_ms = 0.0;
   double last_call_ms = 0.0;
@@ -377,6 +391,12 @@ void ic_big_launch(rip_pool *p, uint64_t first, uint64_t count);
 uint32_t ic_grid_launch(rip_pool *p, uint64_t first, uint64_t count, const uint32_t *ids,
                         bool columns, uint32_t frontier_cap, uint32_t colors);
 void grid_scratch_free(GridScratch &s);
+
+// sample_ic_team.hip: the same samples, one per workgroup with its visited
+// vertices in LDS, for graphs of up to kTeamMaxNodes vertices.
+constexpr uint32_t kTeamMaxNodes = 1u << 20;   // bits: 128 KiB of the CU's 160 KiB of LDS
+uint32_t ic_team_launch(rip_pool *p, uint64_t first, uint64_t count, const uint32_t *ids);
+void team_scratch_free(TeamScratch &s);
 
 // sample_ic_lane.hip: one BFS per lane over samples [first, first + count);
 // returns how many outgrew a lane's queue, their indices (relative to first)

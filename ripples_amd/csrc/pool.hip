@@ -519,6 +519,7 @@ void pool_sample(rip_pool *p, uint64_t count, const rip_tune *tune) {
     p->grid_levels = 0;
     p->wave_ms = 0.0;
     p->wave_ran = false;
+    p->team_ran = false;
     hipLaunchKernelGGL(set_ctl_kernel, dim3(1), dim3(1), 0, p->stream, p->d_ctl,
                        static_cast<unsigned long long>(p->used_data));
     pool_clear_gref(p, first, first + count);
@@ -551,6 +552,11 @@ void pool_sample(rip_pool *p, uint64_t count, const rip_tune *tune) {
       float ms = 0.0f, call = 0.0f;
       RIP_HIP(hipEventElapsedTime(&ms, p->ev0, p->ev1));
       RIP_HIP(hipEventElapsedTime(&call, p->ev0, p->ev2));
+      if (p->team_ran) {
+        float team = 0.0f;
+        RIP_HIP(hipEventElapsedTime(&team, p->ev3, p->ev4));
+        p->grid_ms = team;
+      }
       p->last_kernel_ms = ms;
       p->last_call_ms = call;
       p->last_launches = launches;

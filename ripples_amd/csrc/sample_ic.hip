@@ -655,6 +655,19 @@ uint32_t ic_launch(rip_pool *p, uint64_t first, uint64_t count,
   return 2;
 }
 
+// The samples that outgrew lanes and waves: a workgroup each with the visited
+// bits in LDS where they fit, else the grid sampler's colour groups (also
+// where the caller sets what only those have).  IMM with U[0,0.1] weights:
+// 41.8 ms with the grid and 17.2 with a workgroup each at 65,536 vertices,
+// 49.5 and 20.8 at 262,144.
+static uint32_t large_sets(rip_pool *p, uint64_t first, uint64_t count, const uint32_t *ids,
+                           const rip_tune *tune) {
+  const uint32_t colors = tune ? tune->colors : 0u, frontier_cap = tune ? tune->frontier_cap : 0u;
+  if (p->g->n <= kTeamMaxNodes && colors == 0 && frontier_cap == 0)
+    return ic_team_launch(p, first, count, ids);
+  return ic_grid_launch(p, first, count, ids, true, frontier_cap, colors ? colors : 64u);
+}
+
 // Calls of at most this many samples skip the lanes: a lane takes about
 // 0.4 ms to walk a sample of 64 vertices, whatever the launch holds, where a
 // wave of the stage takes under 0.1 ms.  IMM on 1,000 vertices (weighted
@@ -674,9 +687,7 @@ uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &
     const uint64_t big = ic_wave_launch(p, first, count, nullptr, cfg.out_chunk, true, true, true);
     launches += 2;
     if (big == 0) return launches;
-    return launches + ic_grid_launch(p, first, big, p->g->wave.d_big, true,
-                                     tune ? tune->frontier_cap : 0u,
-                                     tune && tune->colors ? tune->colors : 64u);
+    return launches + large_sets(p, first, big, p->g->wave.d_big, tune);
   }
   uint64_t wave_count = count;
   const uint32_t *wave_ids = nullptr;
@@ -689,8 +700,6 @@ uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &
     if (wave_count == 0) return launches;
     wave_ids = p->g->wave.d_over;
     if (cfg.sampler == RIP_SAMPLER_AUTO) {
-      const uint32_t frontier_cap = tune ? tune->frontier_cap : 0u;
-      const uint32_t colors = tune && tune->colors ? tune->colors : 64u;
       if (ic_wave_stage(tune)) {
         // one BFS per wave, 64 frontier vertices at a time, for the samples
         // up to the wave list; the grid sampler takes the larger ones
@@ -698,10 +707,9 @@ uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &
                                             true, true);
         launches += 2;
         if (big == 0) return launches;
-        return launches + ic_grid_launch(p, first, big, p->g->wave.d_big, true, frontier_cap,
-                                         colors);
+        return launches + large_sets(p, first, big, p->g->wave.d_big, tune);
       }
-      return launches + ic_grid_launch(p, first, wave_count, wave_ids, true, frontier_cap, colors);
+      return launches + large_sets(p, first, wave_count, wave_ids, tune);
     }
   }
   const uint64_t big = ic_wave_launch(p, first, wave_count, wave_ids, cfg.out_chunk, !lanes);

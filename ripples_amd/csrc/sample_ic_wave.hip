@@ -23,6 +23,7 @@
 
 #include "device_util.h"
 #include "ic_common.h"
+#include "ic_expand.h"
 #include "ic_gap.h"
 #include "internal.h"
 
@@ -206,150 +207,6 @@ __device__ inline bool expand_row(const VertexRec *vrec, const uint32_t *ids,
   return true;
 }
 
-// Candidates a lane collects before their edges are read together.
-constexpr uint32_t kUnitBatch = 4;
-
-// Expands up to 64 queued vertices of the sample whose element 0 is z at
-// once, lane l holding the record rv of one (when `have`).  The rows' gap
-// blocks are the units of work: 64 units at a time, one per lane, found by a
-// wave scan of the block counts when some row has several (a hub's blocks
-// spread over the lanes instead of queueing in one).  A lane draws up to
-// kUnitBatch candidates of its block (arithmetic only), then the wave reads
-// their thresholds and in-neighbours together, so a unit waits for one trip
-// to memory, not one per candidate; the live ones go through visit() and the
-// first visits are appended to list[tail ...].  Against one draw per lane and
-// step, a whole row per lane: the stage's kernels of an IMM run on R-MAT scale
-// 22 weighted cascade took 13.5 ms instead of 15.6 (rows of one block there;
-// hub rows of U[0,0.1] graphs have hundreds).  Every lane of the wave must
-// call it.  Returns false when the live edges of a step could take the list
-// past cap.
-template <typename Visit>
-__device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *val, bool have,
-                                         const VertexRec &rv, uint64_t z,
-                                         const Affine *p2, const IcGapTab *tab,
-                                         uint32_t *list, uint32_t &tail, uint32_t cap,
-                                         unsigned long long &st_cand,
-                                         unsigned long long &st_draws,
-                                         unsigned long long &st_bytes,
-                                         unsigned long long &st_live, Visit &&visit) {
-  const uint32_t lane = lane_id();
-  const bool row = have && rv.thr != 0;            // else no edge of the row can be live
-  const uint32_t rdeg = rv.end - rv.begin;
-  const uint32_t nblk = row ? ((rdeg - 1) >> ((rv.flags >> kBetaShift) & 31u)) + 1 : 0u;
-  const uint64_t x0 = rv.ja * z + rv.jb;           // the row's first element
-  const bool single = __ballot(nblk > 1) == 0;     // a lane's unit is its own row
-  const uint32_t incl = single ? 0u : wave_inclusive_scan(nblk);
-  const uint32_t total = single ? 64u : uniform_u32(__shfl(incl, 63, 64));
-  const Affine P = uniform_affine(p2[0]), P2 = uniform_affine(p2[1]);
-  for (uint32_t u0 = 0; u0 < total; u0 += 64) {
-    uint32_t e0 = rv.begin, len = 0, T = rv.thr;
-    uint64_t q = rv.q, x = x0;
-    double inv = rv.inv;
-    bool uniform = (rv.flags & kRowUniform) != 0;
-    bool skip = true;
-    if (single) {
-      if (row) {
-        len = rdeg;                                // one block, at most its full length
-        const uint32_t beta = (rv.flags >> kBetaShift) & 31u;
-        skip = (x >> 32) + 1 <= (len == (1u << beta) ? rv.ufull : rv.ulast);
-      }
-    } else {
-      // unit u is block k of the row of lane j, the first whose inclusive
-      // prefix passes u
-      const uint32_t u = u0 + lane;
-      uint32_t j = 0;
-#pragma unroll
-      for (uint32_t s = 32; s > 0; s >>= 1) {
-        const uint32_t v = __shfl(incl, static_cast<int>(j + s - 1), 64);
-        if (v <= u) j += s;
-      }
-      const int src = static_cast<int>(min(j, 63u));
-      const uint32_t k = u - (__shfl(incl, src, 64) - __shfl(nblk, src, 64));
-      const uint32_t begin = __shfl(rv.begin, src, 64), deg = __shfl(rdeg, src, 64);
-      const uint32_t flags = __shfl(rv.flags, src, 64);
-      const uint32_t ufull = __shfl(rv.ufull, src, 64), ulast = __shfl(rv.ulast, src, 64);
-      T = __shfl(rv.thr, src, 64);
-      q = __shfl(rv.q, src, 64);
-      inv = __shfl(rv.inv, src, 64);
-      x = __shfl(x0, src, 64);
-      uniform = (flags & kRowUniform) != 0;
-      if (u < total) {
-        const uint32_t beta = (flags >> kBetaShift) & 31u;
-        e0 = begin + (k << beta);
-        len = min(deg - (k << beta), 1u << beta);
-        // block k's first element: 2 B k elements after the row's first
-        for (uint32_t kk = k, bit = beta + 1; kk; kk >>= 1, ++bit)
-          if (kk & 1) x = aff_apply(p2[bit], x);
-        skip = (x >> 32) + 1 <= (len == (1u << beta) ? ufull : ulast);
-      }
-    }
-    // a block without candidates costs one compare
-    if (len) ++st_draws;
-    bool more = len != 0 && !skip;
-    uint32_t pos = 0;
-    while (__ballot(more)) {
-      uint32_t ce[kUnitBatch], th[kUnitBatch];
-      uint32_t nc = 0;
-#pragma unroll
-      for (uint32_t i = 0; i < kUnitBatch; ++i) {
-        ce[i] = 0;
-        th[i] = 0;
-        if (more) {
-          const uint32_t gap = ic_gap_draw(x, q, inv, tab);
-          if (gap >= len - pos) {
-            more = false;
-          } else {
-            pos += gap;
-            ce[i] = e0 + pos;
-            // kept iff the edge's threshold t passes this (ic_accept:
-            // hi32(a) T < t 2^32 for the acceptance element a)
-            if (!uniform)
-              th[i] = static_cast<uint32_t>(((aff_apply(P, x) >> 32) * T) >> 32);
-            nc = i + 1;
-            if (++pos < len) {
-              x = aff_apply(P2, x);                // next gap element
-              ++st_draws;
-            } else {
-              more = false;
-            }
-          }
-        }
-      }
-      uint32_t t[kUnitBatch], src[kUnitBatch];
-#pragma unroll
-      for (uint32_t i = 0; i < kUnitBatch; ++i) {
-        t[i] = 0xFFFFFFFFu;                        // rows sharing one threshold keep every candidate
-        src[i] = 0;
-        if (i < nc) {
-          src[i] = ids[ce[i]];
-          if (!uniform) t[i] = val[ce[i]];
-        }
-      }
-      st_cand += nc;
-      if (!uniform) {
-        st_draws += nc;
-        st_bytes += 4 * nc;
-      }
-#pragma unroll
-      for (uint32_t i = 0; i < kUnitBatch; ++i) {
-        const bool live = i < nc && t[i] > th[i];
-        const uint64_t lm = __ballot(live);
-        if (lm == 0) continue;
-        if (tail + __popcll(lm) > cap) return false;
-        if (live) {
-          ++st_live;
-          st_bytes += 4;
-        }
-        const bool fresh = live && visit(src[i]);
-        const uint64_t fm = __ballot(fresh);
-        if (fresh) list[tail + __popcll(fm & lanes_below())] = src[i];
-        tail += __popcll(fm);
-      }
-    }
-  }
-  return true;
-}
-
 // VP: expand 64 queued vertices at a time (expand_rows_units) instead of
 // one row per step over its gap blocks (expand_row, the plain form), with
 // the first vertices of each sample marked in LDS.
@@ -413,6 +270,21 @@ __global__ void __launch_bounds__(BT, 4) ic_wave_kernel(WaveParams P) {
       if (lds_find(ltab, kWaveLdsSlots - 1, src)) return false;
       return table_insert(table, tmask, tag, src);
     };
+    // the first visits among a batch's live edges join the list; false when
+    // they could take it past the cap
+    auto take_vp = [&](const bool (&live)[kUnitBatch], const uint32_t (&src)[kUnitBatch]) {
+#pragma unroll
+      for (uint32_t i = 0; i < kUnitBatch; ++i) {
+        const uint64_t lm = __ballot(live[i]);
+        if (lm == 0) continue;
+        if (tail + __popcll(lm) > P.cap) return false;
+        const bool fresh = live[i] && visit_vp(src[i]);
+        const uint64_t fm = __ballot(fresh);
+        if (fresh) list[tail + __popcll(fm & lanes_below())] = src[i];
+        tail += __popcll(fm);
+      }
+      return true;
+    };
     while (head < tail && !big) {
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
       if (VP) {
@@ -432,8 +304,8 @@ __global__ void __launch_bounds__(BT, 4) ic_wave_kernel(WaveParams P) {
         if (next) recn = P.vrec[vn];
         head = nhead;
         st_exp += take;
-        if (!expand_rows_units(P.ids, P.val, have, rec, z, s_p2, &s_tab, list, tail, P.cap,
-                               st_cand, st_draws, st_bytes, st_live, visit_vp))
+        if (!expand_rows_units(P.ids, P.val, have, rec, z, s_p2, &s_tab, st_cand, st_draws,
+                               st_bytes, st_live, take_vp))
           big = true;
         prec = recn;
         npre = nnext;
@@ -647,6 +519,12 @@ uint32_t wave_grid() {
 // Returns the number of samples left for the colour sampler (their local
 // indices are in g->wave.d_big).
 constexpr int kWaveBT = 256;
+// The stage's list where the team sampler takes the rest: a sample that
+// reaches a giant component is soon seen to, and the stage's work on it is
+// lost.  IMM with U[0,0.1] weights at 65,536 vertices took 23.9, 17.2, 15.9
+// and 15.7 ms with 4096, 2048, 1024 and 512; OPIM-C with weighted cascade at
+// 200,003 vertices 6.0 ms down to 1024 and 7.9 with 512.
+constexpr uint32_t kStageCapTeam = 1024;
 
 uint32_t ic_wave_blocks(uint64_t count) {
   return std::max<uint32_t>(
@@ -715,7 +593,7 @@ uint64_t ic_wave_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
   P.table = w.d_table;
   P.list = w.d_list;
   P.epoch = w.d_epoch;
-  P.cap = CAP;
+  P.cap = stage && g->n <= kTeamMaxNodes ? kStageCapTeam : CAP;
   P.tcap = TCAP;
   P.big_ids = w.d_big;
   P.set_off = p->d_off;

@@ -36,3 +36,42 @@ def test_automatic_setting_matches_oracle(name, count, orc):
         assert np.array_equal(off, eo) and np.array_equal(ver, ev)
     p.close()
     g.close()
+
+
+def folded_csr(n, scale, edge_factor, scheme, wscale, seed):
+    """R-MAT edges folded onto n vertices (any number of them)."""
+    s, d = R.rmat_edges(scale, edge_factor, seed=seed)
+    s, d = s.astype(np.int64) % n, d.astype(np.int64) % n
+    key = np.unique((s * n + d)[s != d])
+    return R.csr_from_edges(n, (key // n).astype(np.uint32), (key % n).astype(np.uint32), scheme,
+                            wscale, seed)
+
+
+@pytest.mark.parametrize("n,scale,ef,wscale,count", [
+    (65, 8, 8, 0.4, 700),             # bitmaps of three words, one hot vertex per lane
+    (1000, 10, 8, 0.3, 900),
+    (4097, 12, 16, 0.1, 257),         # more samples than CUs: workgroups of 512
+    (32768, 15, 16, 0.1, 200),
+    (70001, 16, 16, 0.1, 1500),       # many samples: workgroups of 256, columns
+    (262147, 18, 8, 0.2, 150),        # bitmaps past 32 KiB
+    (1 << 20, 20, 4, 0.5, 70),        # the largest bitmap
+    ((1 << 20) + 1, 20, 4, 0.5, 70),  # one vertex more: the grid sampler
+])
+def test_team_sampler_matches_oracle(n, scale, ef, wscale, count, orc):
+    """Samples past 64 vertices straight to a workgroup each; in two calls, so
+    the second appends and its groups are ragged."""
+    index, edges, w = folded_csr(n, scale, ef, R.W_UNIFORM, wscale, n)
+    g = R.Graph(index, edges, w, model=R.IC)
+    p = g.pool(5)
+    for c in (count // 3, count - count // 3):
+        p.generate_rrr_sets(c, tune={"queue_cap": 64})
+    off, ver = p.export()
+    eo, ev = orc.sample(R.IC, index, edges, w, 5, 0, count)
+    assert np.array_equal(off, eo) and np.array_equal(ver, ev)
+    assert p.size() == (count, len(ev))
+    assert np.array_equal(p.count_occurrences(), orc.count(n, eo, ev))
+    seeds, cov = p.find_most_influential_set(8)
+    es, ec = orc.select(n, eo, ev, 8)
+    assert seeds.tolist() == es.tolist() and cov == ec
+    p.close()
+    g.close()
