@@ -140,7 +140,12 @@ constexpr uint32_t kDenseBT = 512;
 constexpr uint32_t kDenseRange = 16384;        // u32 counters: 64 KiB of LDS
 constexpr uint32_t kDenseLong = 256;           // runs this long are read by the whole wave
 constexpr uint32_t kDenseBlocks = 2048;        // blocks per histogram pass
-constexpr unsigned long long kDenseDecMin = 1ull << 21;  // killed elements for LDS decrements
+// Killed elements from which the decrements go through LDS: one atomic per
+// element on counters all killed sets share takes about 2.5 us per thousand,
+// a histogram pass 0.02-0.15 ms.  IMM with U[0,0.1] weights (column pools) at
+// 65,536 vertices 17.0 ms with the line at 2^21 and 15.4 at 2^17, at 262,144
+// 20.7 and 15.5; 2^14 and 2^19 measured as 2^17.
+constexpr unsigned long long kDenseDecMin = 1ull << 17;
 constexpr uint32_t kScanGrid = 1024;
 
 // First i in [0, len) with a[i] >= x (len if none).
