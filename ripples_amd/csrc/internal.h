@@ -76,7 +76,8 @@ struct GridScratch {
   uint32_t *d_nb = nullptr;            // groups
   unsigned long long *d_fa = nullptr, *d_fb = nullptr;
   unsigned long long *d_gctl = nullptr, *d_union = nullptr;
-  unsigned long long *d_ring = nullptr;  // per-level frontier lengths and chunk counters
+  unsigned long long *d_ring = nullptr;  // per-level counters
+  unsigned long long *d_heavy = nullptr, *d_segs = nullptr;  // heavy items of a level, segments
   unsigned long long *d_out = nullptr;   // output tables of a sub-batch
   uint64_t out_words = 0;
   unsigned long long *h_ctl = nullptr;

@@ -20,15 +20,33 @@
 // so the groups of a batch cost 16 bytes per vertex each, which bounds the
 // batch by memory rather than by the number of workgroups: every level is
 // one persistent kernel over the frontier items (g, v) of all groups of the
-// batch, pulling chunks of items from a global counter.  A chunk's rows are
-// split into units of one colour and up to eight gap blocks, balanced over
-// the workgroup by a scan; a lane draws its unit's candidates one live edge
-// per step, and every live edge is one discovery: a read of vis (most edges
-// in a giant component reach vertices the colour has visited), then atomicOr
-// on vis and pend, and (g, u) joins the next frontier when its pend word was
-// zero.  A frontier longer than its buffer sets an overflow flag; the
-// vertices it could not list keep their pend bits, and a scan of pend finds
-// them once the listed frontier is done.
+// batch.  A wave takes 64 items, a lane each: its pending colours with one
+// exchange, its record, and the number of its units, a unit being one colour
+// and one gap block.  The wave's units are dealt out over its lanes 64 at a
+// time, the colours of a block side by side (they read the same few lines of
+// thresholds); a lane draws its block's candidates, reads their thresholds
+// together, and the live edges join a queue of the wave in LDS.  When the
+// queue holds 64 kDiscover of them they are discovered at once, kDiscover to a
+// lane and stage by stage: the in-neighbours, the vis words (most edges in a
+// giant component reach vertices the colour has visited), the atomicOr on
+// vis, on the union bitmap and on pend; (g, u) joins the next frontier when
+// its pend word was zero, through another queue in LDS.  Items of kHeavyUnits
+// units or more (hub rows pending for many colours) are cut into segments
+// that a second kernel of the level spreads over all waves.  A frontier longer
+// than its buffer sets an overflow flag; the vertices it could not list keep
+// their pend bits, and a scan of pend finds them once the listed frontier is
+// done.
+//
+// What bounds it: requests to memory, 16 waves a CU holding dozens each and
+// meeting no workgroup barrier.  20,000 sets of an R-MAT graph of 2^24
+// vertices with U[0,0.02] weights (1.8e9 live edges, 3.7e9 candidates): 94 ms
+// in these kernels, where random 8-byte loads (55e9/s) and atomics (20e9/s) of
+// the live and the fresh edges alone take about that long.  Chunks of rows
+// per workgroup, expanded in barriered phases, took 320 ms.  Batches of 2, 3,
+// 4, 6 and 8 discoveries a lane (pool call and selection): 222, 170, 145, 126
+// and 125 ms while every batch reserved its own frontier entries, 117 ms for 3
+// and 4 with the queue of entries, whose LDS costs larger batches the fourth
+// workgroup of a CU (126 ms).
 //
 // After the last level, one workgroup per group reads its union in vertex
 // order from the bitmaps (clearing them and vis), keeps the group's hot
@@ -39,33 +57,34 @@
 
 #include "device_util.h"
 #include "ic_common.h"
+#include "ic_expand.h"
 #include "ic_gap.h"
 #include "internal.h"
 
 namespace rip {
 namespace {
 
-constexpr int kExpBT = 256;          // expand kernel
-// frontier items per chunk of the expand kernel: half a workgroup, which
-// keeps the chunk's tables small enough in LDS for six workgroups per CU
-constexpr uint32_t kExpItems = 128;
-// rows pending for this many colours or more are expanded a block per wave,
-// lane c drawing colour c, so a live edge is one discovery for all colours
-constexpr uint32_t kDenseColours = 8;
-constexpr uint32_t kDenseSpan = 128;   // largest block of the dense path (edges)
-constexpr uint32_t kDenseSlots = 8;    // dense tasks per round of a workgroup
-constexpr uint32_t kDenseBatch = 4;    // candidates a dense lane reads thresholds for at once
-constexpr uint32_t kSparseSteps = 8;   // steps of a sparse lane between discoveries
+constexpr int kExpBT = 256;            // level and tail kernels
+constexpr uint32_t kDiscover = 3;      // queued edges a lane discovers at once
+constexpr uint32_t kQueue = 64 * (kDiscover + kUnitBatch);  // a wave's queue of live edges
+constexpr uint32_t kHeavyUnits = 2048; // units from which an item is cut up (8192: the same time)
+constexpr uint32_t kSegUnits = 1024;   // units of a segment
+constexpr uint32_t kOut = 128;         // a wave's queue of frontier entries
+constexpr uint32_t kMinTake = 8;       // fewest items a wave takes at a time
+constexpr int kGridWaves = 4;          // waves a SIMD holds (a quarter of LDS per workgroup)
 // level counters kept on the device (a ring), and levels enqueued per host
 // synchronisation: a BFS of hundreds of narrow levels costs a launch per
 // level, not a round trip
 constexpr uint32_t kRing = 64;
 constexpr uint32_t kLevelsPerSync = 16;
-// a frontier of at most this many items (one chunk) is expanded by one
-// workgroup that runs level after level with a barrier between them (no
-// launch per level): the long thin tails of deep samples.  Wider frontiers go
-// to the level kernels: one workgroup would take their chunks one by one.
-constexpr uint64_t kTailItems = kExpItems;
+// a frontier of at most this many items is expanded by one workgroup that
+// runs level after level with a barrier between them (no launch per level):
+// the long thin tails of deep samples (32 to 128 measured the same).
+constexpr uint64_t kTailItems = 128;
+
+// room for the heavy items of a level and their segments (8 and 8 MiB), no
+// more than a level may list; what finds none is expanded by its own wave
+constexpr uint32_t kHeavyCap = 1u << 19, kSegCap = 1u << 20;
 
 // control words of the grid scratch
 enum : int { kGOver = 0, kGLevels = 1, kGCount = 2, kGTail = 3, kGWords = 4 };
@@ -86,11 +105,13 @@ struct GridParams {
   unsigned long long *next_cnt;    // its length (counts every append, also past cap)
   uint64_t cap;                    // capacity of next
   unsigned long long *gctl;        // control words: overflow flag, level count
-  unsigned long long *ring;        // per level L: ring[L % kRing] frontier length,
-                                   // ring[kRing + L % kRing] chunk counter
+  unsigned long long *ring;        // per level L, words k kRing + L % kRing: frontier length,
+                                   // items taken, heavy items, their segments, segments taken
+  unsigned long long *heavy;       // heavy items of a level: (g << 32 | v, colours) pairs
+  unsigned long long *segs;        // their segments: heavy index << 32 | segment
+  uint32_t heavy_cap, seg_cap;
   unsigned long long *buf[2];      // level L reads buf[L % 2], writes buf[(L + 1) % 2]
   unsigned long long *ctl;         // the pool's control words (work counters)
-  uint32_t chunk;                  // frontier items a level kernel's workgroup takes at a time
 };
 
 // The j-th set bit of m (j < popcount(m)).
@@ -152,71 +173,6 @@ __device__ inline void grid_discover(const GridParams &P, bool live, uint32_t g,
   }
 }
 
-// grid_discover for K entries per lane (bits[k] == 0: no entry), stage by
-// stage over the entries: the K reads of vis, then the K atomics on vis, the
-// bitmaps and the pend words, so each lane keeps K independent requests in
-// flight instead of one chain; one frontier reservation per wave for all.
-// Entries of one lane may name the same (g, u): the atomics on vis settle
-// which of them finds each colour fresh, as between lanes.
-template <int K>
-__device__ inline void grid_discover_k(const GridParams &P, const uint32_t (&g)[K],
-                                       const uint32_t (&u)[K], const unsigned long long (&bits)[K]) {
-  uint64_t idx[K];
-  unsigned long long old[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    idx[k] = static_cast<uint64_t>(g[k]) * P.n + u[k];
-    old[k] = ~0ull;
-    if (bits[k])
-      old[k] = __hip_atomic_load(&P.vp[2 * idx[k]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    if (bits[k] & ~old[k]) old[k] = atomicOr(&P.vp[2 * idx[k]], bits[k]);
-    else old[k] = ~0ull;
-  }
-  unsigned long long fresh[K];
-  uint32_t o0[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    fresh[k] = bits[k] & ~old[k];
-    o0[k] = 1u;
-    if (fresh[k] && old[k] == 0)
-      o0[k] = atomicOr(&P.bm0[static_cast<uint64_t>(g[k]) * P.nw0 + (u[k] >> 5)], 1u << (u[k] & 31u));
-  }
-  // the pend atomics go out with the bitmap ones (neither waits on the
-  // other); the summary bits, which need the bitmap's old word, follow
-  unsigned long long pp[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) pp[k] = fresh[k] ? atomicOr(&P.vp[2 * idx[k] + 1], fresh[k]) : 1ull;
-  bool push[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    if (o0[k] == 0)
-      atomicOr(&P.bm1[static_cast<uint64_t>(g[k]) * P.nw1 + (u[k] >> 10)], 1u << ((u[k] >> 5) & 31u));
-    push[k] = pp[k] == 0;
-  }
-  uint64_t m[K];
-  uint32_t total = 0;
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    m[k] = __ballot(push[k]);
-    total += static_cast<uint32_t>(__popcll(m[k]));
-  }
-  if (total == 0) return;
-  unsigned long long base = 0;
-  if (lane_id() == 0) base = atomicAdd(P.next_cnt, static_cast<unsigned long long>(total));
-  base = __shfl(base, 0, 64);
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    if (push[k]) {
-      const unsigned long long at = base + __popcll(m[k] & lanes_below());
-      if (at < P.cap) P.next[at] = (static_cast<unsigned long long>(g[k]) << 32) | u[k];
-    }
-    base += __popcll(m[k]);
-  }
-}
-
 __device__ inline unsigned long long wave_or_u64(unsigned long long v) {
   for (int d = 32; d > 0; d >>= 1) v |= __shfl_xor(v, d, 64);
   return v;
@@ -232,449 +188,416 @@ __global__ void __launch_bounds__(64) grid_seed_kernel(GridParams P, const uint3
   grid_discover(P, has, g, root, 1ull << c);
 }
 
-// Shared memory of the expansion: the step powers and, per item of a chunk,
-// its row and pending colours with the prefix of its work.
+enum : int { kRFront = 0, kRTaken = 1, kRHeavy = 2, kRSegs = 3, kRSegTaken = 4, kRWords = 5 };
+
+__device__ inline unsigned long long *ring_word(const GridParams &P, int k, uint32_t L) {
+  return &P.ring[static_cast<uint32_t>(k) * kRing + L % kRing];
+}
+
+// A row to expand: the vertex's record, the group and its pending colours.
+struct Row {
+  uint64_t q, ja, jb;
+  unsigned long long M;
+  double inv;
+  uint32_t begin, deg, ufull, ulast, g;
+  uint32_t tf;      // thr | beta << 25 | (threshold shared by the row) << 30
+};
+static_assert(sizeof(Row) == 64 && kIcOne < 1u << 25 && kIcBetaMax < 32, "packed row");
+
+// A workgroup's tables, and per wave the rows being expanded and the queue of
+// live edges to discover (the edge, and group << 6 | colour) and that of the
+// next level's entries.
 template <int BT>
 struct ExpandLds {
   Affine p2[64];
   IcGapTab tab;
-  uint32_t tmp[BT / 64];
-  uint32_t g[kExpItems], beg[kExpItems], deg[kExpItems], T[kExpItems], fl[kExpItems];
-  uint32_t uf[kExpItems], ul[kExpItems], pre[kExpItems], nch[kExpItems], dpre[kExpItems];
-  unsigned long long q[kExpItems], ja[kExpItems], jb[kExpItems], m[kExpItems];
-  double inv[kExpItems];
-  uint32_t ucur;   // next unit of the chunk not claimed by a wave
-  // the dense round's tasks: entry, block, first element, prefix of colours,
-  // and per task and position the colours live there
-  uint32_t tent[kDenseSlots], tk[kDenseSlots], tpre[kDenseSlots];
-  Affine tE[kDenseSlots];
-  unsigned long long pos[kDenseSlots * kDenseSpan];
+  Row row[BT / 64][64];
+  uint32_t qe[BT / 64][kQueue], qg[BT / 64][kQueue];
+  unsigned long long qo[BT / 64][kOut];
 };
 
-struct ExpandStats {
-  unsigned long long cand = 0, draws = 0, exp = 0, bytes = 0, live = 0;
-};
-
-// Expands the frontier items cur[c0, c0 + cl), cl <= kExpItems: every thread of
-// the workgroup calls it.  A chunk's rows are split into units of one colour
-// and up to eight gap blocks (rows pending for few colours) or into wave
-// tasks of one block for every colour (rows pending for many).
+// A wave's side of the expansion; every lane of the wave calls each method.
 template <int BT>
-__device__ void expand_chunk(const GridParams &P, const unsigned long long *cur, uint64_t c0,
-                             uint32_t cl, ExpandLds<BT> &S, ExpandStats &st) {
-  const uint32_t tid = threadIdx.x;
-  __syncthreads();   // the previous chunk's waves are done with the tables
-  Affine *s_p2 = S.p2;
-  uint32_t *s_tmp = S.tmp, *s_g = S.g, *s_beg = S.beg, *s_deg = S.deg, *s_T = S.T, *s_fl = S.fl;
-  uint32_t *s_uf = S.uf, *s_ul = S.ul, *s_pre = S.pre, *s_nch = S.nch, *s_dpre = S.dpre;
-  unsigned long long *s_q = S.q, *s_ja = S.ja, *s_jb = S.jb, *s_m = S.m;
-  double *s_inv = S.inv;
-  unsigned long long &st_cand = st.cand, &st_draws = st.draws, &st_exp = st.exp;
-  unsigned long long &st_bytes = st.bytes, &st_live = st.live;
-  uint32_t units = 0, ntask = 0;
-  if (tid < cl) {
-    const unsigned long long item = cur[c0 + tid];
-    const uint32_t g = static_cast<uint32_t>(item >> 32), v = static_cast<uint32_t>(item);
-    // the colours still to expand at v; a repeated item finds none
-    const unsigned long long M =
-        atomicExch(&P.vp[2 * (static_cast<uint64_t>(g) * P.n + v) + 1], 0ull);
-    uint32_t nch = 0;
-    if (M) {
-      const VertexRec r = P.vrec[v];
-      ++st_exp;
-      st_bytes += kIcRecBytes;
-      s_g[tid] = g;
-      s_beg[tid] = r.begin;
-      s_deg[tid] = r.end - r.begin;
-      s_T[tid] = r.thr;
-      s_fl[tid] = r.flags;
-      s_uf[tid] = r.ufull;
-      s_ul[tid] = r.ulast;
-      s_q[tid] = r.q;
-      s_inv[tid] = r.inv;
-      s_ja[tid] = r.ja;
-      s_jb[tid] = r.jb;
-      s_m[tid] = M;
-      if (r.thr) {
-        const uint32_t beta = (r.flags >> kBetaShift) & 31u;
-        const uint32_t nblk = ((r.end - r.begin - 1) >> beta) + 1;
-        if (__popcll(M) >= kDenseColours && (1u << beta) <= kDenseSpan) {
-          ntask = nblk;   // a round task per block, a lane per (block, colour)
-        } else {
-          nch = nblk;   // a unit per (colour, block)
-          units = static_cast<uint32_t>(__popcll(M)) * nch;
-        }
-      }
-    }
-    s_nch[tid] = nch;
+struct Expander {
+  const GridParams &P;
+  ExpandLds<BT> &S;
+  const uint32_t wid, lane;
+  uint32_t qn = 0, on = 0;   // edges and frontier entries queued (wave-uniform)
+  // a lane's work: blocks drawn and gaps after a block's first, candidates
+  // and those whose threshold was read, live edges, rows
+  uint32_t gaps = 0, cand = 0, vals = 0, live = 0, exp = 0;
+
+  __device__ Expander(const GridParams &p, ExpandLds<BT> &s)
+      : P(p), S(s), wid(threadIdx.x >> 6), lane(lane_id()) {}
+
+  // Appends the wave's frontier entries to the next level's list.
+  __device__ void flush() {
+    unsigned long long base = 0;
+    if (lane == 0) base = atomicAdd(P.next_cnt, static_cast<unsigned long long>(on));
+    base = uniform_u64(base);
+    for (uint32_t i = lane; i < on; i += 64)
+      if (base + i < P.cap) P.next[base + i] = S.qo[wid][i];
+    on = 0;
   }
-  uint32_t total, dtotal;
-  const uint32_t pre = block_exclusive_scan<BT>(units, s_tmp, &total);
-  const uint32_t dpre = block_exclusive_scan<BT>(ntask, s_tmp, &dtotal);
-  if (tid < cl) {
-    s_pre[tid] = pre;
-    s_dpre[tid] = dpre;
-  }
-  if (tid == 0) S.ucur = 0;
-  __syncthreads();
-  // Rows pending for few colours: unit u is block k of colour j of entry
-  // ent.  Each wave claims 64 units at a time from the chunk's counter; a
-  // lane with no unit takes the next one, and every step each lane with a
-  // unit makes one draw (the block's first element and its first gap, or the
-  // next gap) and tests its candidate, so the lanes stay busy whatever the
-  // lengths of their units; the live edges of kSparseSteps steps are then
-  // discovered together.
-  const uint32_t lane = lane_id();
-  {
-    const Affine Pst = uniform_affine(s_p2[0]), P2 = uniform_affine(s_p2[1]);
-    uint32_t nxt = 0, hi = 0;   // the wave's claimed units [nxt, hi) (wave-uniform)
-    bool has = false, started = false;
-    uint32_t g = 0, e0 = 0, len = 0, pos = 0, T = 0, uskip = 0;
-    unsigned long long bit = 0;
-    uint64_t q = 0, x = 0;
-    double inv = 0.0;
-    bool uniform = true;
-    // kSparseSteps steps per lane, then their live edges discovered together
-    for (bool finished = false; !finished;) {
-      uint32_t kg[kSparseSteps], ku[kSparseSteps];
-      unsigned long long kb[kSparseSteps];
+
+  // Discovers the last 64 kDiscover queued edges, or all when they are fewer,
+  // stage by stage over a lane's kDiscover entries, so that each stage's
+  // requests are in flight together.  Entries may name the same (g, u): the
+  // atomics on vis settle which of them finds a colour fresh.
+  __device__ void discover() {
+    const uint32_t take = min(qn, 64u * kDiscover), q0 = qn - take;
+    uint32_t gc[kDiscover], u[kDiscover];
+    bool fresh[kDiscover], first[kDiscover], push[kDiscover];
 #pragma unroll
-      for (uint32_t j = 0; j < kSparseSteps; ++j) {
-        kg[j] = 0;
-        ku[j] = 0;
-        kb[j] = 0;
-        if (finished) continue;   // wave-uniform
-        const uint64_t idle = __ballot(!has);
-        if (idle) {
-          if (nxt >= hi) {
-            uint32_t c0 = 0;
-            if (lane == 0) c0 = atomicAdd(&S.ucur, 64u);
-            c0 = uniform_u32(__shfl(c0, 0, 64));
-            nxt = min(c0, total);
-            hi = min(c0 + 64u, total);
-          }
-          if (!has) {
-            const uint32_t u = nxt + static_cast<uint32_t>(__popcll(idle & lanes_below()));
-            if (u < hi) {
-              uint32_t lo = 0, up = cl;
-              while (lo < up) {
-                const uint32_t mid = (lo + up) >> 1;
-                if (s_pre[mid] <= u) lo = mid + 1;
-                else up = mid;
-              }
-              const uint32_t ent = lo - 1;   // the last entry starting at or before u
-              const uint32_t r = u - s_pre[ent];
-              const uint32_t nblk = s_nch[ent];
-              const uint32_t cj = r / nblk, k = r - cj * nblk;
-              g = s_g[ent];
-              const uint32_t c = nth_bit(s_m[ent], cj);
-              bit = 1ull << c;
-              const uint32_t fl = s_fl[ent];
-              const uint32_t beta = (fl >> kBetaShift) & 31u;
-              const uint32_t B = 1u << beta;
-              e0 = s_beg[ent] + (k << beta);
-              len = min(s_deg[ent] - (k << beta), B);
-              T = s_T[ent];
-              uskip = len == B ? s_uf[ent] : s_ul[ent];
-              q = s_q[ent];
-              inv = s_inv[ent];
-              uniform = (fl & kRowUniform) != 0;
-              // block k's first element: P^(2 B k) after the row's first
-              Affine E{s_ja[ent], s_jb[ent]};
-              for (uint32_t kk = k, b2 = beta + 1; kk; kk >>= 1, ++b2)
-                if (kk & 1) E = aff_then(E, s_p2[b2]);
-              x = E.a * P.z[64ull * g + c] + E.b;
-              pos = 0;
-              has = true;
-              started = false;
-            }
-          }
-          nxt = min(nxt + static_cast<uint32_t>(__popcll(idle)), hi);
-        }
-        if (__ballot(has) == 0) {
-          if (nxt >= total) finished = true;
-          continue;
-        }
-        if (has) {
-          if (!started) {
-            started = true;
-            ++st_draws;
-            // a block without candidates costs one compare
-            if ((x >> 32) + 1 <= uskip) has = false;
-          }
-          if (has) {
-            const uint32_t gap = ic_gap_draw(x, q, inv, &S.tab);
-            if (gap >= len - pos) {
-              has = false;
-            } else {
-              pos += gap;
-              const uint32_t e = e0 + pos;
-              ++st_cand;
-              bool live = true;
-              if (!uniform) {
-                ++st_draws;
-                st_bytes += 4;
-                live = ic_accept(Pst.a * x + Pst.b, T, P.val[e]);   // acceptance element
-              }
-              ++pos;
-              x = P2.a * x + P2.b;                         // next gap element
-              if (pos < len) ++st_draws;
-              else has = false;
-              if (live) {
-                kg[j] = g;
-                ku[j] = P.ids[e];
-                kb[j] = bit;
-                ++st_live;
-                st_bytes += 4;
-              }
-            }
-          }
-        }
-      }
-      grid_discover_k<kSparseSteps>(P, kg, ku, kb);
+    for (uint32_t i = 0; i < kDiscover; ++i) {
+      const uint32_t at = q0 + i * 64 + lane;
+      fresh[i] = at < qn;
+      gc[i] = fresh[i] ? S.qg[wid][at] : 0u;
+      u[i] = fresh[i] ? P.ids[S.qe[wid][at]] : 0u;
     }
+    auto vis = [&](uint32_t i) {
+      return &P.vp[2 * (static_cast<uint64_t>(gc[i] >> 6) * P.n + u[i])];
+    };
+    unsigned long long old[kDiscover];
+#pragma unroll
+    for (uint32_t i = 0; i < kDiscover; ++i) {
+      // vis is written by atomics, which complete in L2; the read goes there too
+      old[i] = fresh[i] ? __hip_atomic_load(vis(i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kDiscover; ++i) {
+      fresh[i] = fresh[i] && ((old[i] >> (gc[i] & 63u)) & 1ull) == 0;
+      if (fresh[i]) old[i] = atomicOr(vis(i), 1ull << (gc[i] & 63u));
+    }
+    // the bitmap's and the pend word's atomics go out together; the summary
+    // bit needs the bitmap's old word
+    uint32_t o0[kDiscover];
+    unsigned long long pend[kDiscover];
+#pragma unroll
+    for (uint32_t i = 0; i < kDiscover; ++i) {
+      fresh[i] = fresh[i] && ((old[i] >> (gc[i] & 63u)) & 1ull) == 0;
+      first[i] = fresh[i] && old[i] == 0;
+      o0[i] = 0;
+      pend[i] = 0;
+      if (first[i])
+        o0[i] = atomicOr(&P.bm0[static_cast<uint64_t>(gc[i] >> 6) * P.nw0 + (u[i] >> 5)],
+                         1u << (u[i] & 31u));
+      if (fresh[i]) pend[i] = atomicOr(vis(i) + 1, 1ull << (gc[i] & 63u));
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kDiscover; ++i) {
+      push[i] = fresh[i] && pend[i] == 0;
+      if (first[i] && o0[i] == 0)
+        atomicOr(&P.bm1[static_cast<uint64_t>(gc[i] >> 6) * P.nw1 + (u[i] >> 10)],
+                 1u << ((u[i] >> 5) & 31u));
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kDiscover; ++i) {
+      const uint64_t m = __ballot(push[i]);
+      const uint32_t k = static_cast<uint32_t>(__popcll(m));
+      if (on + k > kOut) flush();
+      if (push[i])
+        S.qo[wid][on + __popcll(m & lanes_below())] =
+            (static_cast<unsigned long long>(gc[i] >> 6) << 32) | u[i];
+      on += k;
+    }
+    qn = q0;
   }
-  // Rows pending for many colours (blocks of at most kDenseSpan edges): task
-  // t is block k of entry ent, kDenseSlots tasks at a time.  Phase 1: a lane
-  // per (task, colour) walks the colour's candidates of the block and ORs the
-  // colour's bit into the LDS mask of each live position; phase 2: a lane per
-  // position makes one discovery with all the colours live there.  The
-  // atomics of a phase-2 step are independent of each other (many in flight
-  // per wave), and colours reaching one edge together cost one.
-  for (uint32_t r0 = 0; r0 < dtotal; r0 += kDenseSlots) {
-    const uint32_t nt = min(kDenseSlots, dtotal - r0);
-    // phase 0: the round's tasks, their colours and first elements
-    uint32_t tu = 0;
-    if (tid < nt) {
-      const uint32_t t = r0 + tid;
-      uint32_t lo = 0, hi = cl;
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (s_dpre[mid] <= t) lo = mid + 1;
-        else hi = mid;
+
+  // Expands `units` units of each lane's row, from its unit rbase on; unit r
+  // of a row is block r / |M| for the r % |M|-th of its colours M.
+  __device__ void run(uint32_t units, uint64_t rbase) {
+    const uint32_t incl = wave_inclusive_scan(units);
+    const uint32_t total = uniform_u32(__shfl(incl, 63, 64));
+    const Affine A = uniform_affine(S.p2[0]), A2 = uniform_affine(S.p2[1]);
+    for (uint32_t u0 = 0; u0 < total; u0 += 64) {
+      const uint32_t u = u0 + lane;
+      uint32_t j = 0;   // the first lane whose inclusive prefix passes u
+#pragma unroll
+      for (uint32_t s = 32; s > 0; s >>= 1)
+        if (__shfl(incl, static_cast<int>(j + s - 1), 64) <= u) j += s;
+      const uint32_t before = __shfl(incl, static_cast<int>(j ? j - 1 : 0), 64);
+      uint32_t gc = 0, e0 = 0, len = 0, T = 0;
+      uint64_t x = 0, q = 0;
+      double inv = 0.0;
+      bool uniform = true, more = false;
+      if (u < total) {
+        const Row &R = S.row[wid][j];
+        const uint64_t r = rbase + (u - (j ? before : 0u));
+        const unsigned long long M = R.M;
+        const uint32_t ncol = static_cast<uint32_t>(__popcll(M));
+        const uint32_t k = r >> 32 ? static_cast<uint32_t>(r / ncol)
+                                   : static_cast<uint32_t>(r) / ncol;
+        const uint32_t c = nth_bit(M, static_cast<uint32_t>(r - static_cast<uint64_t>(k) * ncol));
+        const uint32_t tf = R.tf, beta = (tf >> 25) & 31u;
+        gc = (R.g << 6) | c;
+        // block k's first element: 2 B k elements after the row's first
+        x = R.ja * P.z[gc] + R.jb;
+        e0 = R.begin + (k << beta);
+        len = min(R.deg - (k << beta), 1u << beta);
+        T = tf & 0x1FFFFFFu;
+        q = R.q;
+        inv = R.inv;
+        uniform = (tf >> 30) != 0;
+        for (uint32_t kk = k, bit = beta + 1; kk; kk >>= 1, ++bit)
+          if (kk & 1) x = aff_apply(S.p2[bit], x);
+        ++gaps;
+        // a block without candidates costs one compare
+        more = (x >> 32) + 1 > (len == 1u << beta ? R.ufull : R.ulast);
       }
-      const uint32_t ent = lo - 1;   // the last entry starting at or before t
-      const uint32_t k = t - s_dpre[ent];
-      const uint32_t beta = (s_fl[ent] >> kBetaShift) & 31u;
-      Affine E{s_ja[ent], s_jb[ent]};
-      for (uint32_t kk = k, b2 = beta + 1; kk; kk >>= 1, ++b2)
-        if (kk & 1) E = aff_then(E, s_p2[b2]);
-      S.tent[tid] = ent;
-      S.tk[tid] = k;
-      S.tE[tid] = E;
-      tu = static_cast<uint32_t>(__popcll(s_m[ent]));
-    }
-    uint32_t units;
-    const uint32_t tpre = block_exclusive_scan<BT>(tu, s_tmp, &units);
-    if (tid < nt) S.tpre[tid] = tpre;
-    __syncthreads();
-    // phase 1
-    for (uint32_t u = tid; u < units; u += BT) {
-      uint32_t lo = 0, hi = nt;
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (S.tpre[mid] <= u) lo = mid + 1;
-        else hi = mid;
-      }
-      const uint32_t t = lo - 1;
-      const uint32_t ent = S.tent[t], k = S.tk[t];
-      const uint32_t c = nth_bit(s_m[ent], u - S.tpre[t]);
-      const uint32_t g = s_g[ent];
-      const uint32_t fl = s_fl[ent];
-      const uint32_t beta = (fl >> kBetaShift) & 31u;
-      const uint32_t B = 1u << beta;
-      const uint32_t len = min(s_deg[ent] - (k << beta), B);
-      const uint32_t e0 = s_beg[ent] + (k << beta);
-      const uint32_t T = s_T[ent];
-      const uint64_t q = s_q[ent];
-      const double inv = s_inv[ent];
-      const bool uniform = (fl & kRowUniform) != 0;
-      const Affine Pst = uniform_affine(s_p2[0]), P2 = uniform_affine(s_p2[1]);
-      const Affine E = S.tE[t];
-      uint64_t x = E.a * P.z[64ull * g + c] + E.b;
-      ++st_draws;
-      // a block without candidates costs one compare
-      if ((x >> 32) + 1 <= (len == B ? s_uf[ent] : s_ul[ent])) continue;
-      unsigned long long *pm = S.pos + t * kDenseSpan;
-      // candidates kDenseBatch at a time: their positions first (arithmetic
-      // only), then their thresholds read together, then the tests
       uint32_t pos = 0;
-      for (bool more = true; more;) {
-        uint32_t cp[kDenseBatch];
-        uint64_t ca[kDenseBatch];
+      while (__ballot(more)) {
+        uint32_t ce[kUnitBatch], th[kUnitBatch], t[kUnitBatch];
         uint32_t nc = 0;
 #pragma unroll
-        for (uint32_t j = 0; j < kDenseBatch; ++j) {
-          cp[j] = 0;
-          ca[j] = 0;
+        for (uint32_t i = 0; i < kUnitBatch; ++i) {
+          ce[i] = 0;
+          th[i] = 0;
           if (more) {
             const uint32_t gap = ic_gap_draw(x, q, inv, &S.tab);
             if (gap >= len - pos) {
               more = false;
             } else {
               pos += gap;
-              ++st_cand;
-              if (!uniform) {
-                ++st_draws;
-                st_bytes += 4;
-                ca[j] = Pst.a * x + Pst.b;             // acceptance element
-              }
-              cp[j] = pos;
-              nc = j + 1;
-              ++pos;
-              if (pos >= len) {
-                more = false;
+              ce[i] = e0 + pos;
+              // kept iff the edge's threshold passes this (ic_accept)
+              if (!uniform) th[i] = static_cast<uint32_t>(((aff_apply(A, x) >> 32) * T) >> 32);
+              nc = i + 1;
+              if (++pos < len) {
+                x = aff_apply(A2, x);                // next gap element
+                ++gaps;
               } else {
-                x = P2.a * x + P2.b;                   // next gap element
-                ++st_draws;
+                more = false;
               }
             }
           }
         }
-        uint32_t tv[kDenseBatch];
 #pragma unroll
-        for (uint32_t j = 0; j < kDenseBatch; ++j)
-          tv[j] = (!uniform && j < nc) ? P.val[e0 + cp[j]] : 0u;
+        for (uint32_t i = 0; i < kUnitBatch; ++i)
+          t[i] = i < nc && !uniform ? P.val[ce[i]] : 0xFFFFFFFFu;
+        cand += nc;
+        if (!uniform) vals += nc;
 #pragma unroll
-        for (uint32_t j = 0; j < kDenseBatch; ++j) {
-          if (j < nc && (uniform || ic_accept(ca[j], T, tv[j]))) {
-            atomicOr(&pm[cp[j]], 1ull << c);
-            ++st_live;
+        for (uint32_t i = 0; i < kUnitBatch; ++i) {
+          const bool on = i < nc && t[i] > th[i];
+          const uint64_t m = __ballot(on);
+          if (on) {
+            const uint32_t at = qn + static_cast<uint32_t>(__popcll(m & lanes_below()));
+            S.qe[wid][at] = ce[i];
+            S.qg[wid][at] = gc;
+            ++live;
           }
+          qn += static_cast<uint32_t>(__popcll(m));
         }
+        if (qn >= 64 * kDiscover) discover();
       }
     }
-    __syncthreads();
-    // phase 2: every thread takes KP positions and discovers them together
-    constexpr int KP = static_cast<int>(kDenseSlots * kDenseSpan / BT);
-    static_assert(KP * BT == kDenseSlots * kDenseSpan, "positions split evenly");
-    uint32_t dg[KP], du[KP];
-    unsigned long long dm[KP];
-#pragma unroll
-    for (int j = 0; j < KP; ++j) {
-      const uint32_t pi = static_cast<uint32_t>(j) * BT + tid;
-      const uint32_t t = pi / kDenseSpan, pos = pi % kDenseSpan;
-      dm[j] = 0;
-      dg[j] = 0;
-      du[j] = 0;
-      if (t < nt) {
-        dm[j] = S.pos[pi];
-        if (dm[j]) {
-          S.pos[pi] = 0;
-          const uint32_t ent = S.tent[t];
-          dg[j] = s_g[ent];
-          du[j] = P.ids[s_beg[ent] + (S.tk[t] << ((s_fl[ent] >> kBetaShift) & 31u)) + pos];
-          st_bytes += 4;
-        }
-      }
-    }
-    grid_discover_k<KP>(P, dg, du, dm);
-    __syncthreads();
   }
+
+  // Lane's row: vertex v of group g, pending for the colours M (0: none).
+  // Returns its units.
+  __device__ uint64_t load(uint32_t g, uint32_t v, unsigned long long M) {
+    if (!M) return 0;
+    const VertexRec rv = P.vrec[v];
+    if (!rv.thr) return 0;
+    const uint32_t beta = (rv.flags >> kBetaShift) & 31u;
+    S.row[wid][lane] = Row{rv.q, rv.ja, rv.jb, M, rv.inv, rv.begin, rv.end - rv.begin, rv.ufull,
+                           rv.ulast, g,
+                           rv.thr | beta << 25 | (rv.flags & kRowUniform ? 1u << 30 : 0u)};
+    return static_cast<uint64_t>(__popcll(M)) * (((rv.end - rv.begin - 1) >> beta) + 1);
+  }
+
+  // Leaves an item of `all` units to the level's heavy kernel; false when
+  // there is no room for it.
+  __device__ bool defer(uint32_t L, unsigned long long item, unsigned long long M, uint64_t all) {
+    const uint64_t nseg = (all + kSegUnits - 1) / kSegUnits;
+    const unsigned long long h = atomicAdd(ring_word(P, kRHeavy, L), 1ull);
+    if (h >= P.heavy_cap) return false;
+    P.heavy[2 * h] = item;
+    P.heavy[2 * h + 1] = M;
+    const unsigned long long s0 = atomicAdd(ring_word(P, kRSegs, L), nseg);
+    const bool fits = s0 + nseg <= P.seg_cap;
+    const uint64_t end = fits ? s0 + nseg : P.seg_cap;
+    for (uint64_t i = s0; i < end; ++i) P.segs[i] = fits ? (h << 32) | (i - s0) : ~0ull;
+    return fits;
+  }
+
+  // Up to 64 frontier items, one per lane, of level L; with `here` also the
+  // heavy ones are expanded by this wave.
+  __device__ void items(bool have, unsigned long long item, uint32_t L, bool here) {
+    const uint32_t g = static_cast<uint32_t>(item >> 32), v = static_cast<uint32_t>(item);
+    // the colours still to expand at v; a repeated item finds none
+    unsigned long long M = 0;
+    if (have) M = atomicExch(&P.vp[2 * (static_cast<uint64_t>(g) * P.n + v) + 1], 0ull);
+    if (M) ++exp;
+    const uint64_t all = load(g, v, M);
+    uint64_t left = 0;     // units of a heavy item to expand here
+    uint32_t units = static_cast<uint32_t>(all);
+    if (all >= kHeavyUnits) {
+      units = 0;
+      if (here || !defer(L, item, M, all)) left = all;
+    }
+    // the light items together, then the heavy ones one by one
+    uint64_t from = 0;
+    for (;;) {
+      run(units, from);
+      const uint64_t m = __ballot(left != 0);
+      if (!m) break;
+      const uint32_t j = __ffsll(static_cast<unsigned long long>(m)) - 1;
+      const uint64_t lj = uniform_u64(__shfl(left, static_cast<int>(j), 64));
+      const uint64_t aj = uniform_u64(__shfl(all, static_cast<int>(j), 64));
+      const uint32_t now = static_cast<uint32_t>(min(lj, static_cast<uint64_t>(1) << 30));
+      from = aj - lj;
+      units = lane == j ? now : 0u;
+      if (lane == j) left -= now;
+    }
+  }
+
+  __device__ void finish() {
+    while (qn) discover();
+    if (on) flush();
+  }
+
+  __device__ void report() {
+    report_stats(P.ctl, static_cast<unsigned long long>(kIcRecBytes) * exp + 4ull * vals + 4ull * live,
+                 cand, static_cast<unsigned long long>(gaps) + vals, exp, live);
+  }
+};
+
+template <int BT>
+__device__ inline void expand_tables(const GridParams &P, ExpandLds<BT> &S) {
+  if (threadIdx.x == 0) fill_step_powers(P.step, S.p2);
+  ic_load_tables(&S.tab);
+  __syncthreads();
 }
 
-// BFS level L: the frontier is buf[L % 2][0, n) with n = ring[L % kRing]
-// (its first cap entries when it overflowed, which raises the overflow
-// flag); every workgroup with a chunk to take pulls chunks of P.chunk items
-// (at most kExpItems) from the level's counter.  Levels are enqueued ahead of
-// the host: a level whose frontier is empty costs its launch only.
+// BFS level L: the frontier is buf[L % 2][0, n) with n the level's frontier
+// length (its first cap entries when it overflowed, which raises the overflow
+// flag); waves take up to 64 items at a time, fewer when the frontier would
+// leave waves without any.  Levels are enqueued ahead of the host: a level
+// whose frontier is empty costs its launches only.
 template <int BT>
-__global__ void __launch_bounds__(BT, 3) grid_level_kernel(GridParams P, uint32_t L) {
+__global__ void __launch_bounds__(BT, kGridWaves) grid_level_kernel(GridParams P, uint32_t L) {
+  constexpr uint32_t NW = BT / 64;
   __shared__ ExpandLds<BT> S;
-  __shared__ unsigned long long s_chunk;
-  const uint32_t tid = threadIdx.x;
-  const uint64_t raw = __hip_atomic_load(&P.ring[L % kRing], __ATOMIC_RELAXED,
+  const uint64_t raw = __hip_atomic_load(ring_word(P, kRFront, L), __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
   const uint64_t ncur = raw < P.cap ? raw : P.cap;
-  if (blockIdx.x == 0 && tid == 0 && ncur) {
+  if (blockIdx.x == 0 && threadIdx.x == 0 && ncur) {
     P.gctl[kGLevels] += 1;
     if (raw > P.cap) P.gctl[kGOver] = 1;
   }
-  const uint32_t chunk = P.chunk;
-  if (static_cast<uint64_t>(blockIdx.x) * chunk >= ncur) return;   // no chunk for it
-  GridParams Q = P;
-  Q.cur = P.buf[L & 1u];
-  Q.ncur = ncur;
-  Q.next = P.buf[(L + 1) & 1u];
-  Q.next_cnt = &P.ring[(L + 1) % kRing];
-  unsigned long long *head = &P.ring[kRing + L % kRing];
-  if (tid == 0) fill_step_powers(P.step, S.p2);
-  ic_load_tables(&S.tab);
-  for (uint32_t i = tid; i < kDenseSlots * kDenseSpan; i += BT) S.pos[i] = 0;  // phase 2 keeps it zero
-  ExpandStats st;
+  const uint64_t each = ncur / (static_cast<uint64_t>(gridDim.x) * NW);
+  const uint32_t take = each >= 64 ? 64u : max(kMinTake, static_cast<uint32_t>(each));
+  if (static_cast<uint64_t>(blockIdx.x) * NW * take >= ncur) return;   // no items for it
+  P.next = L & 1u ? P.buf[0] : P.buf[1];
+  P.next_cnt = ring_word(P, kRFront, L + 1);
+  const unsigned long long *cur = L & 1u ? P.buf[1] : P.buf[0];
+  expand_tables<BT>(P, S);
+  Expander<BT> E(P, S);
   for (;;) {
-    __syncthreads();
-    if (tid == 0) s_chunk = atomicAdd(head, static_cast<unsigned long long>(chunk));
-    __syncthreads();
-    const uint64_t c0 = s_chunk;
-    if (c0 >= ncur) break;
-    expand_chunk<BT>(Q, Q.cur, c0,
-                     static_cast<uint32_t>(min(static_cast<uint64_t>(chunk), ncur - c0)), S,
-                     st);
+    unsigned long long i0 = 0;
+    if (E.lane == 0) i0 = atomicAdd(ring_word(P, kRTaken, L), static_cast<unsigned long long>(take));
+    i0 = uniform_u64(i0);
+    if (i0 >= ncur) break;
+    const bool have = E.lane < take && i0 + E.lane < ncur;
+    E.items(have, have ? cur[i0 + E.lane] : 0ull, L, false);
   }
-  report_stats(P.ctl, st.bytes, st.cand, st.draws, st.exp, st.live);
+  E.finish();
+  E.report();
+}
+
+// The segments of level L's heavy items, one to a wave at a time.
+template <int BT>
+__global__ void __launch_bounds__(BT, kGridWaves) grid_heavy_kernel(GridParams P, uint32_t L) {
+  __shared__ ExpandLds<BT> S;
+  const uint64_t raw = __hip_atomic_load(ring_word(P, kRSegs, L), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+  const uint64_t nseg = raw < P.seg_cap ? raw : P.seg_cap;
+  if (static_cast<uint64_t>(blockIdx.x) * (BT / 64) >= nseg) return;
+  P.next = L & 1u ? P.buf[0] : P.buf[1];
+  P.next_cnt = ring_word(P, kRFront, L + 1);
+  expand_tables<BT>(P, S);
+  Expander<BT> E(P, S);
+  for (;;) {
+    unsigned long long i = 0;
+    if (E.lane == 0) i = atomicAdd(ring_word(P, kRSegTaken, L), 1ull);
+    i = uniform_u64(i);
+    if (i >= nseg) break;
+    const unsigned long long s = uniform_u64(P.segs[i]);
+    if (s == ~0ull) continue;
+    const unsigned long long item = P.heavy[2 * (s >> 32)], M = P.heavy[2 * (s >> 32) + 1];
+    const uint64_t all = E.load(static_cast<uint32_t>(item >> 32), static_cast<uint32_t>(item),
+                                E.lane == 0 ? M : 0ull);
+    const uint64_t a = (s & 0xFFFFFFFFull) * kSegUnits;
+    E.run(all > a ? static_cast<uint32_t>(min(all - a, static_cast<uint64_t>(kSegUnits))) : 0u, a);
+  }
+  E.finish();
+  E.report();
 }
 
 // Levels L0, L0 + 1, ... by one workgroup while the frontier holds between 1
 // and tail_cap items: each level zeroes the next level's length, expands its
-// items chunk by chunk and meets the next level at a barrier.  Stops at the
-// first level whose frontier is empty or longer than tail_cap and leaves its
-// number in gctl[kGTail]; that level's length stays in the ring for the
-// level kernels.
+// items, an even share to each wave, and meets the next level at a barrier.
+// Stops at the first level whose frontier is empty or longer than tail_cap and
+// leaves its number in gctl[kGTail]; that level's length stays in the ring for
+// the level kernels.
 template <int BT>
-__global__ void __launch_bounds__(BT, 3) grid_tail_kernel(GridParams P, uint32_t L0,
-                                                       uint64_t tail_cap) {
+__global__ void __launch_bounds__(BT, kGridWaves) grid_tail_kernel(GridParams P, uint32_t L0,
+                                                          uint64_t tail_cap) {
+  constexpr uint32_t NW = BT / 64;
   __shared__ ExpandLds<BT> S;
   __shared__ unsigned long long s_n;
   const uint32_t tid = threadIdx.x;
-  if (tid == 0) fill_step_powers(P.step, S.p2);
-  ic_load_tables(&S.tab);
-  for (uint32_t i = tid; i < kDenseSlots * kDenseSpan; i += BT) S.pos[i] = 0;
-  ExpandStats st;
+  expand_tables<BT>(P, S);
+  Expander<BT> E(P, S);
   uint32_t L = L0;
   for (;; ++L) {
-    __syncthreads();   // the previous level's appends are done
+    // the previous level's appends are done: the waves' own stores first
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
     if (tid == 0) {
-      const unsigned long long raw = __hip_atomic_load(&P.ring[L % kRing], __ATOMIC_RELAXED,
+      const unsigned long long raw = __hip_atomic_load(ring_word(P, kRFront, L), __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_AGENT);
       s_n = raw;
       if (raw != 0 && raw <= tail_cap) {
-        __hip_atomic_store(&P.ring[(L + 1) % kRing], 0ull, __ATOMIC_RELAXED,
+        __hip_atomic_store(ring_word(P, kRFront, L + 1), 0ull, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
         P.gctl[kGLevels] += 1;
       }
     }
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     const uint64_t ncur = s_n;
     if (ncur == 0 || ncur > tail_cap) break;
-    GridParams Q = P;
-    Q.cur = P.buf[L & 1u];
-    Q.ncur = ncur;
-    Q.next = P.buf[(L + 1) & 1u];
-    Q.next_cnt = &P.ring[(L + 1) % kRing];
-    for (uint64_t c0 = 0; c0 < ncur; c0 += kExpItems)
-      expand_chunk<BT>(Q, Q.cur, c0,
-                       static_cast<uint32_t>(min(static_cast<uint64_t>(kExpItems), ncur - c0)),
-                       S, st);
+    P.next = L & 1u ? P.buf[0] : P.buf[1];
+    P.next_cnt = ring_word(P, kRFront, L + 1);
+    const unsigned long long *cur = L & 1u ? P.buf[1] : P.buf[0];
+    const uint64_t share = min(64ull, (ncur + NW - 1) / NW);
+    for (uint64_t i0 = E.wid * share; i0 < ncur; i0 += NW * share) {
+      const bool have = E.lane < share && i0 + E.lane < ncur;
+      E.items(have, have ? cur[i0 + E.lane] : 0ull, L, true);
+    }
+    E.finish();
   }
   if (tid == 0) P.gctl[kGTail] = L;
-  report_stats(P.ctl, st.bytes, st.cand, st.draws, st.exp, st.live);
+  E.report();
 }
 
-// Zeroes the frontier lengths of levels a .. a + k - 1 and the chunk
-// counters of levels a - 1 .. a + k - 2 (ring indices mod kRing), or, with
-// `all`, the whole ring and the control words.
+// Zeroes the frontier lengths of levels a .. a + k - 1 and the other counters
+// of levels a - 1 .. a + k - 2 (ring indices mod kRing), or, with `all`, the
+// whole ring and the control words.
 __global__ void grid_ring_kernel(unsigned long long *ring, unsigned long long *gctl, uint32_t a,
                                  uint32_t k, uint32_t all) {
   const uint32_t i = threadIdx.x;
   if (all) {
-    if (i < 2 * kRing) ring[i] = 0;
+    for (uint32_t j = i; j < kRWords * kRing; j += blockDim.x) ring[j] = 0;
     if (i < kGWords) gctl[i] = 0;
     return;
   }
   if (i < k) {
     ring[(a + i) % kRing] = 0;
-    ring[kRing + (a + i - 1) % kRing] = 0;
+    for (uint32_t w = 1; w < kRWords; ++w) ring[w * kRing + (a + i - 1) % kRing] = 0;
   }
 }
 
@@ -1083,7 +1006,9 @@ static void grid_ensure(rip_graph *g, uint32_t groups, uint64_t fcap, hipStream_
     s.fcap = fcap;
   }
   if (!s.d_gctl) {
-    s.d_ring = dev_alloc<unsigned long long>(2 * kRing);
+    s.d_ring = dev_alloc<unsigned long long>(kRWords * kRing);
+    s.d_heavy = dev_alloc<unsigned long long>(2ull * kHeavyCap);
+    s.d_segs = dev_alloc<unsigned long long>(kSegCap);
     s.d_gctl = dev_alloc<unsigned long long>(kGWords);
     s.d_union = dev_alloc<unsigned long long>(256);
     RIP_HIP(hipHostMalloc(reinterpret_cast<void **>(&s.h_ctl), sizeof(unsigned long long) * 256,
@@ -1121,6 +1046,8 @@ void grid_scratch_free(GridScratch &s) {
   dev_free(s.d_gctl);
   dev_free(s.d_union);
   dev_free(s.d_ring);
+  dev_free(s.d_heavy);
+  dev_free(s.d_segs);
   dev_free(s.d_out);
   s.out_words = 0;
   if (s.h_ctl) (void)hipHostFree(s.h_ctl);
@@ -1168,6 +1095,10 @@ uint32_t ic_grid_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
   P.gctl = s.d_gctl;
   P.ctl = p->d_ctl;
   P.ring = s.d_ring;
+  P.heavy = s.d_heavy;
+  P.segs = s.d_segs;
+  P.heavy_cap = static_cast<uint32_t>(std::min<uint64_t>(kHeavyCap, lcap));
+  P.seg_cap = static_cast<uint32_t>(std::min<uint64_t>(kSegCap, lcap));
   P.buf[0] = s.d_fa;
   P.buf[1] = s.d_fb;
   const int per_cu = blocks_per_cu(reinterpret_cast<const void *>(&grid_level_kernel<kExpBT>),
@@ -1176,16 +1107,9 @@ uint32_t ic_grid_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
   uint32_t launches = 0;
   for (uint64_t b0 = 0; b0 < count; b0 += static_cast<uint64_t>(C) * G) {
     const uint32_t Gb = static_cast<uint32_t>(std::min<uint64_t>(G, (count - b0 + C - 1) / C));
-    // small batches on small graphs take their levels in chunks of 32 items:
-    // a level's hub rows, discovered together, sit in few chunks, and with
-    // chunks of 128 the workgroups holding them set the level's time.  On
-    // R-MAT scale 16 IC (n Gb of 4M-25M), IMM's sampling calls of 4K-8K sets
-    // took 10-11.6 ms with 128 and 6.3-8.6 ms with 32; with 32 on every batch,
-    // scale 18 (100,000 sets) and scale 24 (20,000 sets) ran 4-5% slower.
-    P.chunk = static_cast<uint64_t>(n) * Gb <= (1ull << 25) ? kExpItems / 4 : kExpItems;
     hipLaunchKernelGGL(grid_samples_kernel, dim3((64 * Gb + 255) / 256), dim3(256), 0, st,
                        p->seed, first, ids, b0, count, Gb, C, s.d_z, s.d_sid, s.d_nb);
-    hipLaunchKernelGGL(grid_ring_kernel, dim3(1), dim3(2 * kRing), 0, st, s.d_ring, s.d_gctl, 0u,
+    hipLaunchKernelGGL(grid_ring_kernel, dim3(1), dim3(256), 0, st, s.d_ring, s.d_gctl, 0u,
                        0u, 1u);
     // level 0: the roots, in buf[0]
     P.next = s.d_fa;
@@ -1226,10 +1150,13 @@ uint32_t ic_grid_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
         // kLevelsPerSync levels, then one look at the frontier length
         hipLaunchKernelGGL(grid_ring_kernel, dim3(1), dim3(kLevelsPerSync), 0, st, s.d_ring,
                            s.d_gctl, L + 1, kLevelsPerSync, 0u);
-        for (uint32_t i = 0; i < kLevelsPerSync; ++i)
+        for (uint32_t i = 0; i < kLevelsPerSync; ++i) {
           hipLaunchKernelGGL((grid_level_kernel<kExpBT>), dim3(exp_grid), dim3(kExpBT), 0, st, P,
                              L + i);
-        launches += 1 + kLevelsPerSync;
+          hipLaunchKernelGGL((grid_heavy_kernel<kExpBT>), dim3(exp_grid), dim3(kExpBT), 0, st, P,
+                             L + i);
+        }
+        launches += 1 + 2 * kLevelsPerSync;
       }
       RIP_HIP(hipGetLastError());
       RIP_HIP(hipEventRecord(p->ev4, st));

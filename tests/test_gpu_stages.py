@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import ripples_amd as R
+from graphs import transposed_csr
 
 pytestmark = pytest.mark.gpu
 
@@ -73,5 +74,43 @@ def test_team_sampler_matches_oracle(n, scale, ef, wscale, count, orc):
     seeds, cov = p.find_most_influential_set(8)
     es, ec = orc.select(n, eo, ev, 8)
     assert seeds.tolist() == es.tolist() and cov == ec
+    p.close()
+    g.close()
+
+
+def hubs_csr(deg):
+    """100 hubs that every other vertex has as in-neighbours, each with `deg`
+    in-edges, one of threshold 2^23 (blocks of 16 edges) and the rest next to
+    dead."""
+    n = 3000 + deg
+    hubs, rest = np.arange(100), np.arange(100, n)
+    s = [np.tile(hubs, len(rest))]
+    d = [np.repeat(rest, 100)]
+    w = [np.ones(100 * len(rest), np.float32)]
+    for h in hubs:
+        s.append(100 + (np.arange(deg) * 7 + 31 * h) % (deg + 1000))
+        d.append(np.full(deg, h))
+        w.append(np.full(deg, 1e-5, np.float32))
+        w[-1][(17 * h) % deg] = 0.5
+    return transposed_csr(n, np.concatenate(s), np.concatenate(d), np.concatenate(w))
+
+
+@pytest.mark.parametrize("deg,count,cap", [
+    (511, 64 * 3 + 5, 0),         # thin frontiers, rows next to the size that is cut up
+    (513, 64 * 3 + 5, 0),
+    (513, 64 * 200 + 1, 0),       # wide ones: hub rows of 2112 units in segments
+    (512, 64 * 200 + 1, 37),      # no room for most of the segments, nor the frontier
+    (16003, 64 * 3 + 5, 100),     # 64 segments a row
+])
+def test_grid_sampler_hub_rows_match_oracle(deg, count, cap, orc):
+    index, edges, w = hubs_csr(deg)
+    g = R.Graph(index, edges, w, model=R.IC)
+    p = g.pool(9)
+    p.generate_rrr_sets(count, tune={"queue_cap": 64, "colors": 64, "frontier_cap": cap})
+    for first in {0, max(0, count - 600)}:
+        part = min(count, 600)
+        off, ver = p.export(first, part)
+        eo, ev = orc.sample(R.IC, index, edges, w, 9, first, part)
+        assert np.array_equal(off, eo) and np.array_equal(ver, ev)
     p.close()
     g.close()
