@@ -270,6 +270,7 @@ void graph_create(rip_graph *g, int device, int model, uint32_t n, uint64_t m,
   g->m = m;
   g->max_degree = maxdeg;
   g->step = sample_step();
+  g->blocks = std::make_shared<BlockCache>(device);
   for (int b = 0; b < 33; ++b) g->deg_ge_pow2[b] = deg_ge[b];
 
   unsigned long long *d_index = nullptr;
@@ -379,6 +380,7 @@ void graph_destroy(rip_graph *g) {
   dev_free(g->fwd.d_dst);
   dev_free(g->fwd.d_val);
   dev_free(g->fwd.d_scratch);
+  if (g->blocks) g->blocks->close();
 }
 
 }  // namespace rip

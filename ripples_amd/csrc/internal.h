@@ -4,7 +4,11 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <list>
+#include <memory>
 #include <mutex>
+#include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "common.h"
@@ -20,6 +24,55 @@ struct rip_host_graph {
 };
 
 namespace rip {
+
+// blocks.cpp: the parts of a pool that take the driver long to make.
+struct StreamKit {
+  hipStream_t stream = nullptr;
+  hipEvent_t ev[5] = {};
+  unsigned long long *d_ctl = nullptr;  // kCtlWords control words
+  unsigned long long *h_ctl = nullptr;  // pinned host copy
+};
+void kit_create(StreamKit *k);          // on failure the caller destroys what there is
+void kit_destroy(StreamKit &k);
+
+// Device blocks and stream kits that the pools of one graph gave up, for the
+// next pool of the graph; bounded (blocks.cpp), freed when the graph goes and
+// when a device allocation fails.  A block or kit comes in only when no queued
+// work uses it, so any stream may take it.  Safe from several threads.
+class BlockCache {
+ public:
+  explicit BlockCache(int device);
+  ~BlockCache();
+  BlockCache(const BlockCache &) = delete;
+  BlockCache &operator=(const BlockCache &) = delete;
+  void *take(size_t bytes);              // contents undefined
+  void give(void *p, bool keep);         // keep false: straight to the driver
+  bool take_kit(StreamKit *kit);         // false: none idle
+  bool give_kit(const StreamKit &kit);   // false: not taken
+  void release();                        // frees the idle blocks
+  void close();                          // and the kits, and keeps no more
+  size_t idle_bytes();
+  int device() const { return device_; }
+
+ private:
+  struct Block {
+    void *p;
+    size_t bytes;
+  };
+  const int device_;
+  uint64_t limit_ = 0;
+  std::mutex mu_;
+  std::list<Block> idle_;                // longest idle first
+  size_t idle_bytes_ = 0;
+  std::unordered_map<void *, size_t> lent_;
+  std::vector<StreamKit> kits_;
+  bool closed_ = false;
+};
+
+// hipMalloc on the current device; idle blocks are freed before it gives up.
+void *device_malloc(size_t bytes);
+// Free memory of the current device, counting idle blocks.
+uint64_t device_free_bytes();
 
 // Scratch of the fused IC sampler: one slot per resident colour group.
 struct IcSlots {
@@ -226,6 +279,7 @@ struct rip_graph {
   rip::TeamScratch team;
   rip::LtScratch lt;
   rip::FwdGraph fwd;
+  std::shared_ptr<rip::BlockCache> blocks;  // what its pools gave up
 };
 
 namespace rip {
@@ -236,6 +290,9 @@ constexpr uint32_t kColBlock = 16;  // column groups per device allocation
 
 struct rip_pool {
   rip_graph *g = nullptr;
+  std::shared_ptr<rip::BlockCache> blocks;  // the graph's
+  bool keep_blocks = true;    // what the pool gives up may wait there
+  bool quiet = false;         // no queued work on the stream (pool_destroy)
   uint64_t seed = 0;
   hipStream_t stream = nullptr;
   uint64_t num_sets = 0;
@@ -441,10 +498,9 @@ uint32_t select_top(rip_pool *p, uint64_t num_sets, uint64_t total, uint32_t k, 
 // select_sort.hip: sorts `count` (key, value) pairs by the low `bits` bits
 // of the key in the double buffers (k0, k1), (v0, v1); returns the buffer
 // holding the result (0 or 1).  *temp grows to the sort's temporary storage.
-int sort_pairs_u32(uint32_t *k0, uint32_t *k1, uint32_t *v0, uint32_t *v1, uint64_t count,
-                   uint32_t bits, void **temp, size_t *temp_bytes, hipStream_t st);
-void exclusive_scan_u32(const uint32_t *d_in, unsigned long long *d_out,
-                        uint64_t n, hipStream_t stream);
+int sort_pairs_u32(rip_pool *p, uint32_t *k0, uint32_t *k1, uint32_t *v0, uint32_t *v1,
+                   uint64_t count, uint32_t bits, void **temp, size_t *temp_bytes);
+void exclusive_scan_u32(rip_pool *p, const uint32_t *d_in, unsigned long long *d_out, uint64_t n);
 
 // tune.cpp: the candidate settings that draw `probe` samples fastest on g
 // (or, unless force, those found before for a graph of the same model and
@@ -473,19 +529,29 @@ void csr_from_edges(uint32_t n, uint64_t m, const uint32_t *src,
 template <typename T>
 T *dev_alloc(size_t count) {
   if (count == 0) count = 1;
-  void *p = nullptr;
-  hipError_t e = hipMalloc(&p, count * sizeof(T));
-  if (e != hipSuccess)
-    throw Error(-2, std::string("hipMalloc of ") +
-                        std::to_string(count * sizeof(T)) +
-                        " bytes failed: " + hipGetErrorString(e));
-  return static_cast<T *>(p);
+  return static_cast<T *>(device_malloc(count * sizeof(T)));
 }
 
 template <typename T>
 void dev_free(T *&p) {
   if (p) (void)hipFree(p);
   p = nullptr;
+}
+
+// The same for a pool's buffers, through its graph's idle blocks.  A block is
+// given up once the pool's stream, the only one that uses it, is idle.
+template <typename T>
+T *pool_alloc(rip_pool *p, size_t count) {
+  return static_cast<T *>(p->blocks->take((count ? count : 1) * sizeof(T)));
+}
+
+template <typename T>
+void pool_free(rip_pool *p, T *&b) {
+  if (b) {
+    const bool idle = p->quiet || hipStreamSynchronize(p->stream) == hipSuccess;
+    p->blocks->give(b, p->keep_blocks && idle);
+  }
+  b = nullptr;
 }
 
 // spread.hip

@@ -192,8 +192,9 @@ __global__ void __launch_bounds__(kHotBT) hot_extract_kernel(unsigned long long 
 
 }  // namespace
 
-void exclusive_scan_u32(const uint32_t *d_in, unsigned long long *d_out,
-                        uint64_t n, hipStream_t stream) {
+void exclusive_scan_u32(rip_pool *p, const uint32_t *d_in, unsigned long long *d_out,
+                        uint64_t n) {
+  hipStream_t stream = p->stream;
   if (n == 0) {
     const unsigned long long zero = 0;
     RIP_HIP(hipMemcpyAsync(d_out, &zero, sizeof(zero), hipMemcpyHostToDevice, stream));
@@ -201,15 +202,14 @@ void exclusive_scan_u32(const uint32_t *d_in, unsigned long long *d_out,
     return;
   }
   const uint64_t tiles = (n + kScanTile - 1) / kScanTile;
-  unsigned long long *tmp = dev_alloc<unsigned long long>(tiles);
+  unsigned long long *tmp = pool_alloc<unsigned long long>(p, tiles);
   hipLaunchKernelGGL(scan_tile_sums, dim3(static_cast<uint32_t>(tiles)), dim3(kScanBT),
                      0, stream, d_in, n, tmp);
   hipLaunchKernelGGL(scan_tile_prefix, dim3(1), dim3(kScanBT), 0, stream, tmp, tiles);
   hipLaunchKernelGGL(scan_apply, dim3(static_cast<uint32_t>(tiles)), dim3(kScanBT), 0,
                      stream, d_in, n, tmp, d_out);
   hipError_t e = hipGetLastError();
-  RIP_HIP(hipStreamSynchronize(stream));
-  dev_free(tmp);
+  pool_free(p, tmp);
   RIP_HIP(e);
 }
 
@@ -229,69 +229,75 @@ void pool_create(rip_pool *p, rip_graph *g, uint64_t seed) {
 }
 
 void pool_create_resources(rip_pool *p) {
-  RIP_HIP(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking));
-  RIP_HIP(hipEventCreate(&p->ev0));
-  RIP_HIP(hipEventCreate(&p->ev1));
-  RIP_HIP(hipEventCreate(&p->ev2));
-  RIP_HIP(hipEventCreate(&p->ev3));
-  RIP_HIP(hipEventCreate(&p->ev4));
-  p->d_ctl = dev_alloc<unsigned long long>(kCtlWords);
-  // pinned, so reading the control words back after a launch is one DMA
-  // rather than a copy staged through a driver buffer
-  RIP_HIP(hipHostMalloc(reinterpret_cast<void **>(&p->h_ctl),
-                        sizeof(unsigned long long) * kCtlWords, hipHostMallocDefault));
+  p->blocks = p->g->blocks;
+  StreamKit kit;
+  if (!p->blocks->take_kit(&kit)) {
+    try {
+      kit_create(&kit);
+    } catch (...) {
+      kit_destroy(kit);
+      throw;
+    }
+  }
+  p->stream = kit.stream;
+  p->ev0 = kit.ev[0];
+  p->ev1 = kit.ev[1];
+  p->ev2 = kit.ev[2];
+  p->ev3 = kit.ev[3];
+  p->ev4 = kit.ev[4];
+  p->d_ctl = kit.d_ctl;
+  p->h_ctl = kit.h_ctl;
   RIP_HIP(hipMemsetAsync(p->d_ctl, 0, sizeof(unsigned long long) * kCtlWords, p->stream));
   RIP_HIP(hipStreamSynchronize(p->stream));
 }
 
 void pool_destroy(rip_pool *p) {
-  if (!p || !p->g) return;
+  if (!p || !p->g || !p->blocks) return;
   (void)hipSetDevice(p->g->device);
-  if (p->stream) (void)hipStreamSynchronize(p->stream);
-  dev_free(p->d_off);
-  dev_free(p->d_len);
-  dev_free(p->d_data);
-  dev_free(p->d_ctl);
-  dev_free(p->d_gref);
-  dev_free(p->d_colptr);
-  dev_free(p->d_gsample);
-  for (auto *b : p->col_blocks) dev_free(b);
+  // blocks and the kit may serve another pool only when the stream is idle
+  const bool idle = !p->stream || hipStreamSynchronize(p->stream) == hipSuccess;
+  if (!idle) p->keep_blocks = false;
+  p->quiet = true;
+  pool_free(p, p->d_off);
+  pool_free(p, p->d_len);
+  pool_free(p, p->d_data);
+  pool_free(p, p->d_gref);
+  pool_free(p, p->d_colptr);
+  pool_free(p, p->d_gsample);
+  for (auto *b : p->col_blocks) pool_free(p, b);
   p->col_blocks.clear();
   p->groups = p->cap_groups = 0;
-  dev_free(p->sel.d_counts);
-  dev_free(p->sel.d_inv_start);
-  dev_free(p->sel.d_cursor);
-  dev_free(p->sel.d_inv);
-  dev_free(p->sel.d_pkey[0]);
-  dev_free(p->sel.d_pkey[1]);
-  dev_free(p->sel.d_pval);
-  dev_free(p->sel.d_soff);
-  dev_free(p->sel.d_stemp);
-  dev_free(p->sel.d_part);
-  dev_free(p->sel.d_top);
-  dev_free(p->sel.d_rank);
-  dev_free(p->sel.d_cand);
-  dev_free(p->sel.d_rec);
-  dev_free(p->sel.d_members);
-  dev_free(p->sel.d_kill);
-  dev_free(p->sel.d_covered);
-  dev_free(p->sel.d_keys);
-  dev_free(p->sel.d_partial);
-  dev_free(p->sel.d_args);
-  dev_free(p->sel.d_gactive);
-  dev_free(p->sel.d_gkill);
-  dev_free(p->sel.d_kgroups);
+  pool_free(p, p->sel.d_counts);
+  pool_free(p, p->sel.d_inv_start);
+  pool_free(p, p->sel.d_cursor);
+  pool_free(p, p->sel.d_inv);
+  pool_free(p, p->sel.d_pkey[0]);
+  pool_free(p, p->sel.d_pkey[1]);
+  pool_free(p, p->sel.d_pval);
+  pool_free(p, p->sel.d_soff);
+  pool_free(p, p->sel.d_stemp);
+  pool_free(p, p->sel.d_part);
+  pool_free(p, p->sel.d_top);
+  pool_free(p, p->sel.d_rank);
+  pool_free(p, p->sel.d_cand);
+  pool_free(p, p->sel.d_rec);
+  pool_free(p, p->sel.d_members);
+  pool_free(p, p->sel.d_kill);
+  pool_free(p, p->sel.d_covered);
+  pool_free(p, p->sel.d_keys);
+  pool_free(p, p->sel.d_partial);
+  pool_free(p, p->sel.d_args);
+  pool_free(p, p->sel.d_gactive);
+  pool_free(p, p->sel.d_gkill);
+  pool_free(p, p->sel.d_kgroups);
   if (p->sel.graph) (void)hipGraphExecDestroy(p->sel.graph);
-  if (p->h_ctl) (void)hipHostFree(p->h_ctl);
-  p->h_ctl = nullptr;
-  if (p->ev0) (void)hipEventDestroy(p->ev0);
-  if (p->ev1) (void)hipEventDestroy(p->ev1);
-  if (p->ev2) (void)hipEventDestroy(p->ev2);
-  if (p->ev3) (void)hipEventDestroy(p->ev3);
-  if (p->ev4) (void)hipEventDestroy(p->ev4);
+  StreamKit kit{p->stream, {p->ev0, p->ev1, p->ev2, p->ev3, p->ev4}, p->d_ctl, p->h_ctl};
+  if (!p->keep_blocks || !kit.stream || !p->blocks->give_kit(kit)) kit_destroy(kit);
+  p->d_ctl = p->h_ctl = nullptr;
   p->ev0 = p->ev1 = p->ev2 = p->ev3 = p->ev4 = nullptr;
-  if (p->stream) (void)hipStreamDestroy(p->stream);
   p->stream = nullptr;
+  p->quiet = false;
+  p->blocks.reset();
   p->sel = SelectScratch{};
   p->cap_sets = p->cap_data = p->used_data = p->num_sets = p->num_elements = 0;
 }
@@ -299,14 +305,14 @@ void pool_destroy(rip_pool *p) {
 void pool_reserve_sets(rip_pool *p, uint64_t cap) {
   if (cap <= p->cap_sets) return;
   cap = std::max(cap, 2 * p->cap_sets);
-  auto *off = dev_alloc<unsigned long long>(cap);
+  auto *off = pool_alloc<unsigned long long>(p, cap);
   uint32_t *len = nullptr, *gref = nullptr;
   try {
-    len = dev_alloc<uint32_t>(cap);
-    if (p->d_gref) gref = dev_alloc<uint32_t>(cap);
+    len = pool_alloc<uint32_t>(p, cap);
+    if (p->d_gref) gref = pool_alloc<uint32_t>(p, cap);
   } catch (...) {
-    dev_free(off);
-    dev_free(len);
+    pool_free(p, off);
+    pool_free(p, len);
     throw;
   }
   if (p->num_sets) {
@@ -319,9 +325,9 @@ void pool_reserve_sets(rip_pool *p, uint64_t cap) {
                              hipMemcpyDeviceToDevice, p->stream));
   }
   RIP_HIP(hipStreamSynchronize(p->stream));
-  dev_free(p->d_off);
-  dev_free(p->d_len);
-  dev_free(p->d_gref);
+  pool_free(p, p->d_off);
+  pool_free(p, p->d_len);
+  pool_free(p, p->d_gref);
   p->d_off = off;
   p->d_len = len;
   p->d_gref = gref;
@@ -359,7 +365,7 @@ uint64_t pool_device_bytes(const rip_pool *p) {
 void pool_reserve_groups(rip_pool *p, uint32_t need) {
   graph_ensure_hot(p->g, p->stream);
   if (!p->d_gref) {
-    p->d_gref = dev_alloc<uint32_t>(std::max<uint64_t>(p->cap_sets, 1));
+    p->d_gref = pool_alloc<uint32_t>(p, std::max<uint64_t>(p->cap_sets, 1));
     pool_clear_gref(p, 0, std::max<uint64_t>(p->cap_sets, 1));
   }
   if (need <= p->cap_groups) return;
@@ -371,14 +377,14 @@ void pool_reserve_groups(rip_pool *p, uint32_t need) {
                            hipMemcpyDeviceToHost, p->stream));
   RIP_HIP(hipStreamSynchronize(p->stream));
   for (uint32_t b = p->cap_groups; b < cap; b += kColBlock) {
-    unsigned long long *blk = dev_alloc<unsigned long long>(kColBlock * hot);
+    unsigned long long *blk = pool_alloc<unsigned long long>(p, kColBlock * hot);
     p->col_blocks.push_back(blk);
     for (uint32_t i = 0; i < kColBlock; ++i) ptrs[b + i] = blk + i * hot;
   }
-  unsigned long long **colptr = dev_alloc<unsigned long long *>(cap);
+  unsigned long long **colptr = pool_alloc<unsigned long long *>(p, cap);
   uint32_t *gsample = nullptr;
   try {
-    gsample = dev_alloc<uint32_t>(64ull * cap);
+    gsample = pool_alloc<uint32_t>(p, 64ull * cap);
     RIP_HIP(hipMemcpyAsync(colptr, ptrs.data(), sizeof(void *) * cap, hipMemcpyHostToDevice,
                            p->stream));
     if (p->cap_groups)
@@ -386,12 +392,12 @@ void pool_reserve_groups(rip_pool *p, uint32_t need) {
                              hipMemcpyDeviceToDevice, p->stream));
     RIP_HIP(hipStreamSynchronize(p->stream));
   } catch (...) {
-    dev_free(colptr);
-    dev_free(gsample);
+    pool_free(p, colptr);
+    pool_free(p, gsample);
     throw;
   }
-  dev_free(p->d_colptr);
-  dev_free(p->d_gsample);
+  pool_free(p, p->d_colptr);
+  pool_free(p, p->d_gsample);
   p->d_colptr = colptr;
   p->d_gsample = gsample;
   p->cap_groups = cap;
@@ -448,12 +454,12 @@ static void copy_sync(rip_pool *p, void *dst, const void *src, size_t bytes, hip
 
 void pool_reserve_data(rip_pool *p, uint64_t cap) {
   if (cap <= p->cap_data) return;
-  auto *data = dev_alloc<uint32_t>(cap);
+  auto *data = pool_alloc<uint32_t>(p, cap);
   if (p->used_data)
     RIP_HIP(hipMemcpyAsync(data, p->d_data, sizeof(uint32_t) * p->used_data,
                            hipMemcpyDeviceToDevice, p->stream));
   RIP_HIP(hipStreamSynchronize(p->stream));
-  dev_free(p->d_data);
+  pool_free(p, p->d_data);
   p->d_data = data;
   p->cap_data = cap;
 }
@@ -642,11 +648,11 @@ void pool_export(rip_pool *p, uint64_t first, uint64_t count, uint64_t *offsets,
         gent.push_back(gref[i]);
       }
   }
-  auto *pre = dev_alloc<unsigned long long>(count + 1);
+  auto *pre = pool_alloc<unsigned long long>(p, count + 1);
   uint32_t *out = nullptr, *d_ent = nullptr, *hot = nullptr;
   unsigned long long *hsz = nullptr;
   try {
-    exclusive_scan_u32(p->d_len + first, pre, count, p->stream);
+    exclusive_scan_u32(p, p->d_len + first, pre, count);
     std::vector<uint64_t> coff(count + 1);
     copy_sync(p, coff.data(), pre, sizeof(uint64_t) * (count + 1), hipMemcpyDeviceToHost);
     const uint64_t cold_total = coff[count];
@@ -654,8 +660,8 @@ void pool_export(rip_pool *p, uint64_t first, uint64_t count, uint64_t *offsets,
     const uint64_t ng = gidx.size();
     std::vector<unsigned long long> hoff(ng + 1, 0);
     if (ng) {
-      d_ent = dev_alloc<uint32_t>(ng);
-      hsz = dev_alloc<unsigned long long>(ng + 1);
+      d_ent = pool_alloc<uint32_t>(p, ng);
+      hsz = pool_alloc<unsigned long long>(p, ng + 1);
       copy_sync(p, d_ent, gent.data(), sizeof(uint32_t) * ng, hipMemcpyHostToDevice);
       hipLaunchKernelGGL(hot_size_kernel, dim3(static_cast<uint32_t>(ng)), dim3(kHotBT), 0,
                          p->stream, p->d_colptr, d_ent, p->g->hot_n, hsz);
@@ -679,7 +685,7 @@ void pool_export(rip_pool *p, uint64_t first, uint64_t count, uint64_t *offsets,
     const uint64_t total = offsets[count];
     if (vertices) {
       RIP_REQUIRE(total <= cap, -1, "export: vertices buffer too small");
-      out = dev_alloc<uint32_t>(cold_total);
+      out = pool_alloc<uint32_t>(p, cold_total);
       const uint64_t waves = (count + 63) / 64;
       if (waves) {
         hipLaunchKernelGGL(gather_sets, dim3(static_cast<uint32_t>((waves + 3) / 4)),
@@ -689,7 +695,7 @@ void pool_export(rip_pool *p, uint64_t first, uint64_t count, uint64_t *offsets,
       }
       std::vector<uint32_t> hot_h;
       if (ng) {
-        hot = dev_alloc<uint32_t>(hoff[ng]);
+        hot = pool_alloc<uint32_t>(p, hoff[ng]);
         copy_sync(p, hsz, hoff.data(), sizeof(unsigned long long) * (ng + 1),
                           hipMemcpyHostToDevice);
         hipLaunchKernelGGL(hot_extract_kernel, dim3(static_cast<uint32_t>(ng)), dim3(kHotBT), 0,
@@ -723,18 +729,18 @@ void pool_export(rip_pool *p, uint64_t first, uint64_t count, uint64_t *offsets,
       }
     }
   } catch (...) {
-    dev_free(pre);
-    dev_free(out);
-    dev_free(d_ent);
-    dev_free(hsz);
-    dev_free(hot);
+    pool_free(p, pre);
+    pool_free(p, out);
+    pool_free(p, d_ent);
+    pool_free(p, hsz);
+    pool_free(p, hot);
     throw;
   }
-  dev_free(pre);
-  dev_free(out);
-  dev_free(d_ent);
-  dev_free(hsz);
-  dev_free(hot);
+  pool_free(p, pre);
+  pool_free(p, out);
+  pool_free(p, d_ent);
+  pool_free(p, hsz);
+  pool_free(p, hot);
 }
 
 }  // namespace rip

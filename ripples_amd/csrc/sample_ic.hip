@@ -543,8 +543,7 @@ IcLaunch ic_tune(const rip_pool *p, const rip_tune *tune) {
   RIP_REQUIRE(c.block == 256 || c.block == 512 || c.block == 1024, -1,
               "tune: block must be 256, 512 or 1024");
   if (c.slots == 0) {
-    size_t free_b = 0, total_b = 0;
-    RIP_HIP(hipMemGetInfo(&free_b, &total_b));
+    const size_t free_b = device_free_bytes();
     const size_t per = slot_bytes_for(p->g, c.heavy_degree);
     // keep the sampler scratch within an eighth of the memory it may use
     // (free plus what it already holds), 24 GiB at most

@@ -957,8 +957,7 @@ uint64_t group_bytes(uint32_t n) {
 // Groups per batch and frontier capacity for `count` samples.
 static void grid_plan(const rip_graph *g, uint64_t count, uint32_t colors, uint32_t *groups,
                       uint64_t *fcap) {
-  size_t free_b = 0, total_b = 0;
-  RIP_HIP(hipMemGetInfo(&free_b, &total_b));
+  const uint64_t free_b = device_free_bytes();
   const GridScratch &s = g->grid;
   const uint64_t held = s.n == g->n ? s.groups * group_bytes(g->n) + 16ull * s.fcap : 0;
   // the scratch stays within an eighth of the memory it may use, 32 GiB at most

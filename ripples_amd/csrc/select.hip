@@ -663,49 +663,49 @@ void ensure_select_scratch(rip_pool *p, uint64_t num_sets, uint64_t inv_elems,
   SelectScratch &s = p->sel;
   const uint32_t n = p->g->n;
   if (s.n != n) {
-    dev_free(s.d_counts);
-    dev_free(s.d_inv_start);
-    dev_free(s.d_cursor);
-    s.d_counts = dev_alloc<uint32_t>(n);
-    s.d_inv_start = dev_alloc<unsigned long long>(static_cast<uint64_t>(n) + 1);
-    s.d_cursor = dev_alloc<unsigned long long>(n);
+    pool_free(p, s.d_counts);
+    pool_free(p, s.d_inv_start);
+    pool_free(p, s.d_cursor);
+    s.d_counts = pool_alloc<uint32_t>(p, n);
+    s.d_inv_start = pool_alloc<unsigned long long>(p, static_cast<uint64_t>(n) + 1);
+    s.d_cursor = pool_alloc<unsigned long long>(p, n);
     s.n = n;
   }
   if (s.cap_sets < num_sets) {
-    dev_free(s.d_covered);
-    dev_free(s.d_soff);
+    pool_free(p, s.d_covered);
+    pool_free(p, s.d_soff);
     s.cap_sets = std::max<uint64_t>(num_sets, s.cap_sets + s.cap_sets / 2);
-    s.d_covered = dev_alloc<uint8_t>(s.cap_sets);
-    s.d_soff = dev_alloc<unsigned long long>(s.cap_sets + 1);
+    s.d_covered = pool_alloc<uint8_t>(p, s.cap_sets);
+    s.d_soff = pool_alloc<unsigned long long>(p, s.cap_sets + 1);
   }
   if (s.cap_elems < inv_elems) {
-    dev_free(s.d_inv);
+    pool_free(p, s.d_inv);
     s.cap_elems = std::max<uint64_t>(inv_elems, s.cap_elems + s.cap_elems / 2);
-    s.d_inv = dev_alloc<uint32_t>(s.cap_elems);
+    s.d_inv = pool_alloc<uint32_t>(p, s.cap_elems);
   }
   if (s.cap_kill < kill_sets) {
-    dev_free(s.d_kill);
+    pool_free(p, s.d_kill);
     s.cap_kill = std::max<uint64_t>(kill_sets, s.cap_kill + s.cap_kill / 2);
-    s.d_kill = dev_alloc<uint32_t>(s.cap_kill);
+    s.d_kill = pool_alloc<uint32_t>(p, s.cap_kill);
   }
   if (s.cap_k < k) {
-    dev_free(s.d_keys);
+    pool_free(p, s.d_keys);
     s.cap_k = k;
-    s.d_keys = dev_alloc<unsigned long long>(k);
+    s.d_keys = pool_alloc<unsigned long long>(p, k);
   }
   if (s.cap_groups < p->groups) {
-    dev_free(s.d_gactive);
-    dev_free(s.d_gkill);
-    dev_free(s.d_kgroups);
+    pool_free(p, s.d_gactive);
+    pool_free(p, s.d_gkill);
+    pool_free(p, s.d_kgroups);
     s.cap_groups = 0;
     const uint32_t cap = std::max<uint32_t>(p->groups, p->cap_groups);
-    s.d_gactive = dev_alloc<unsigned long long>(cap);
-    s.d_gkill = dev_alloc<unsigned long long>(cap);
-    s.d_kgroups = dev_alloc<uint32_t>(cap);
+    s.d_gactive = pool_alloc<unsigned long long>(p, cap);
+    s.d_gkill = pool_alloc<unsigned long long>(p, cap);
+    s.d_kgroups = pool_alloc<uint32_t>(p, cap);
     s.cap_groups = cap;
   }
-  if (!s.d_args) s.d_args = dev_alloc<Args>(1);
-  if (!s.d_partial) s.d_partial = dev_alloc<unsigned long long>(kArgmaxBlocks);
+  if (!s.d_args) s.d_args = pool_alloc<Args>(p, 1);
+  if (!s.d_partial) s.d_partial = pool_alloc<unsigned long long>(p, kArgmaxBlocks);
 }
 
 constexpr uint64_t kDenseMinElements = 1ull << 22;
@@ -737,23 +737,23 @@ const uint32_t *inverted_by_sort(rip_pool *p, uint64_t num_sets, uint64_t total)
   const uint32_t n = p->g->n;
   if (s.cap_pairs < total) {
     const uint64_t cap = std::max<uint64_t>(total, s.cap_pairs + s.cap_pairs / 2);
-    dev_free(s.d_pkey[0]);
-    dev_free(s.d_pkey[1]);
-    dev_free(s.d_pval);
+    pool_free(p, s.d_pkey[0]);
+    pool_free(p, s.d_pkey[1]);
+    pool_free(p, s.d_pval);
     s.cap_pairs = 0;
-    s.d_pkey[0] = dev_alloc<uint32_t>(cap);
-    s.d_pkey[1] = dev_alloc<uint32_t>(cap);
-    s.d_pval = dev_alloc<uint32_t>(cap);
+    s.d_pkey[0] = pool_alloc<uint32_t>(p, cap);
+    s.d_pkey[1] = pool_alloc<uint32_t>(p, cap);
+    s.d_pval = pool_alloc<uint32_t>(p, cap);
     s.cap_pairs = cap;
   }
-  exclusive_scan_u32(p->d_len, s.d_soff, num_sets, st);
+  exclusive_scan_u32(p, p->d_len, s.d_soff, num_sets);
   hipLaunchKernelGGL(pairs_kernel, dim3(grid_for(num_sets, 64 * (kBT / 64), 8192)), dim3(kBT), 0,
                      st, p->d_off, p->d_len, p->d_data, num_sets, s.d_soff, s.d_pkey[0], s.d_inv);
   RIP_HIP(hipGetLastError());
   uint32_t bits = 1;
   while (bits < 32 && (static_cast<uint64_t>(n) - 1) >> bits) ++bits;
-  const int at = sort_pairs_u32(s.d_pkey[0], s.d_pkey[1], s.d_inv, s.d_pval, total, bits,
-                                &s.d_stemp, &s.stemp_bytes, st);
+  const int at = sort_pairs_u32(p, s.d_pkey[0], s.d_pkey[1], s.d_inv, s.d_pval, total, bits,
+                                &s.d_stemp, &s.stemp_bytes);
   hipLaunchKernelGGL(starts_kernel, dim3(grid_for(total + 1, kBT, 4096)), dim3(kBT), 0, st,
                      s.d_pkey[at], total, n, s.d_inv_start);
   hipLaunchKernelGGL(counts_from_starts_kernel, dim3(grid_for(n, kBT, 2048)), dim3(kBT), 0, st,
@@ -870,7 +870,7 @@ static const uint32_t *inverted_index(rip_pool *p, uint64_t num_sets, uint64_t t
   const uint32_t n = p->g->n;
   if (total >= kSortMinPairs && total <= kSortMaxPairs) return inverted_by_sort(p, num_sets, total);
   count_plain(p, num_sets, total, nullptr);
-  exclusive_scan_u32(s.d_counts, s.d_inv_start, n, st);
+  exclusive_scan_u32(p, s.d_counts, s.d_inv_start, n);
   hipLaunchKernelGGL(copy_u64_kernel, dim3(grid_for(n, kBT, 2048)), dim3(kBT), 0, st,
                      s.d_cursor, s.d_inv_start, static_cast<uint64_t>(n));
   if (num_sets)

@@ -8,17 +8,17 @@
 
 namespace rip {
 
-int sort_pairs_u32(uint32_t *k0, uint32_t *k1, uint32_t *v0, uint32_t *v1, uint64_t count,
-                   uint32_t bits, void **temp, size_t *temp_bytes, hipStream_t st) {
+int sort_pairs_u32(rip_pool *p, uint32_t *k0, uint32_t *k1, uint32_t *v0, uint32_t *v1,
+                   uint64_t count, uint32_t bits, void **temp, size_t *temp_bytes) {
+  hipStream_t st = p->stream;
   rocprim::double_buffer<uint32_t> keys(k0, k1), vals(v0, v1);
   size_t need = 0;
   RIP_HIP(rocprim::radix_sort_pairs(nullptr, need, keys, vals, static_cast<size_t>(count), 0u,
                                     bits, st));
   if (*temp_bytes < need) {
-    dev_free(*temp);
-    *temp = nullptr;
+    pool_free(p, *temp);
     *temp_bytes = 0;
-    *temp = dev_alloc<uint8_t>(need);
+    *temp = pool_alloc<uint8_t>(p, need);
     *temp_bytes = need;
   }
   size_t have = *temp_bytes;

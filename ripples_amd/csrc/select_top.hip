@@ -691,9 +691,9 @@ void count_plain(rip_pool *p, uint64_t num_sets, uint64_t total, const uint8_t *
   const uint64_t words = 3ull * (buckets + 1) + static_cast<uint64_t>(blocks) * buckets +
                          (total + 1) / 2;
   if (s.cap_part < words) {
-    dev_free(s.d_part);
+    pool_free(p, s.d_part);
     s.cap_part = 0;
-    s.d_part = dev_alloc<uint32_t>(words);
+    s.d_part = pool_alloc<uint32_t>(p, words);
     s.cap_part = words;
   }
   uint32_t *bcnt = s.d_part, *bstart = bcnt + buckets + 1, *sstart = bstart + buckets + 1;
@@ -725,29 +725,29 @@ uint32_t select_top(rip_pool *p, uint64_t num_sets, uint64_t total, uint32_t k, 
   const uint32_t n = p->g->n;
   const uint32_t ntiles = (n + kTile - 1) / kTile;
   const uint64_t nwords = (static_cast<uint64_t>(n) + 63) / 64;
-  if (!s.d_top) s.d_top = dev_alloc<uint8_t>(sizeof(TopState));
+  if (!s.d_top) s.d_top = pool_alloc<uint8_t>(p, sizeof(TopState));
   if (s.top_n != n) {
-    dev_free(s.d_rank);
-    dev_free(s.d_cand);
+    pool_free(p, s.d_rank);
+    pool_free(p, s.d_cand);
     s.top_n = 0;
     // ranks, then the bitmap of the candidates
-    s.d_rank = dev_alloc<uint16_t>(4 * nwords + 4 * ((n + 3ull) / 4));
+    s.d_rank = pool_alloc<uint16_t>(p, 4 * nwords + 4 * ((n + 3ull) / 4));
     // candidates, their counts, starts and cursors; the tiles' two counts
-    s.d_cand = dev_alloc<uint32_t>(4ull * (kTopMax + 1) + 2ull * ntiles);
+    s.d_cand = pool_alloc<uint32_t>(p, 4ull * (kTopMax + 1) + 2ull * ntiles);
     s.top_n = n;
   }
   if (s.cap_top_sets < num_sets) {
-    dev_free(s.d_rec);
+    pool_free(p, s.d_rec);
     const uint64_t cap = std::max<uint64_t>(num_sets, s.cap_top_sets + s.cap_top_sets / 2);
     s.cap_top_sets = 0;
-    s.d_rec = dev_alloc<uint8_t>(sizeof(SetRec) * cap);
+    s.d_rec = pool_alloc<uint8_t>(p, sizeof(SetRec) * cap);
     s.cap_top_sets = cap;
   }
   if (s.cap_members < total) {
-    dev_free(s.d_members);
+    pool_free(p, s.d_members);
     const uint64_t cap = std::max<uint64_t>(total, s.cap_members + s.cap_members / 2);
     s.cap_members = 0;
-    s.d_members = dev_alloc<uint16_t>(cap);
+    s.d_members = pool_alloc<uint16_t>(p, cap);
     s.cap_members = cap;
   }
   TopState *ts = reinterpret_cast<TopState *>(s.d_top);

@@ -301,6 +301,8 @@ void worker_loop(rip_server *s) {
     try {
       RIP_HIP(hipSetDevice(g->device));
       if (!e->created) {
+        // under a budget an evicted pool gives its memory back
+        e->pool.keep_blocks = s->budget == 0;
         pool_create(&e->pool, g, e->seed);
         e->created = true;
       } else if (e->reseed) {

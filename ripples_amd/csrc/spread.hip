@@ -430,8 +430,7 @@ void spread_run(rip_graph *g, const uint32_t *seeds, uint32_t nseeds, uint64_t s
   const bool lds = bitmaps <= kSpreadLds;
   // 32-bit words per workgroup: queue, bitmaps outside LDS; LT: sums, candidates
   const uint64_t per_wg = ((ic ? n : 4 * n) + (lds ? 0 : bitmaps / 4) + 1) / 2 * 2;
-  size_t free_b = 0, total_b = 0;
-  RIP_HIP(hipMemGetInfo(&free_b, &total_b));
+  const uint64_t free_b = device_free_bytes();
   const uint64_t held = g->fwd.wgs * g->fwd.per_wg * 4;
   const uint64_t budget = std::min<uint64_t>((free_b + held) / 8, 16ull << 30);
   uint64_t wgs = std::max<uint64_t>(1, std::min<uint64_t>({count, 1024, budget / (per_wg * 4)}));
