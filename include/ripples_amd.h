@@ -64,8 +64,8 @@ typedef struct {
                             level may list (0 = automatic); vertices past it
                             are found again by a scan of the pending masks */
   uint32_t wave_stage;   /* IC AUTO: nonzero (or queue_cap 0) = samples passing queue_cap are
-                            first run one per wave, 64 frontier vertices at a
-                            time, up to 4096 vertices (1024 on graphs of up to
+                            first run several per wave, 64 frontier vertices at
+                            a time, up to 4096 vertices (1024 on graphs of up to
                             2^20 vertices), and only the larger ones go on;
                             calls of up to 16,384 samples start there, with no
                             lanes before */
@@ -73,9 +73,9 @@ typedef struct {
 
 /* IC sampler kinds (all give the same sets):
  *   AUTO    one reverse BFS per lane (64 samples per wave); samples passing
- *           queue_cap vertices go to one BFS per wave expanding 64 queued
- *           vertices at a time (the wave stage; not with a queue_cap given
- *           and wave_stage 0), and larger ones to a workgroup each with its
+ *           queue_cap vertices go to waves that hold up to four each and expand
+ *           64 queued vertices at a time (the wave stage; not with a queue_cap
+ *           given and wave_stage 0), and larger ones to a workgroup each with its
  *           visited vertices in LDS (graphs of up to 2^20 vertices, no colors
  *           or frontier_cap given) or to the grid sampler: 64-sample colour
  *           groups, many groups per batch, one BFS level of all of them per

@@ -369,6 +369,7 @@ void graph_destroy(rip_graph *g) {
   dev_free(g->wave.d_lepoch);
   dev_free(g->wave.d_over);
   dev_free(g->wave.d_lsort);
+  stage_scratch_free(g->wave);
   grid_scratch_free(g->grid);
   team_scratch_free(g->team);
   dev_free(g->lt.d_long_ids);

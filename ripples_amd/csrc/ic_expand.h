@@ -1,5 +1,5 @@
-// Row expansion shared by the IC samplers that take 64 vertices of one sample
-// at a time (wave stage, team sampler).
+// Row expansion shared by the IC samplers that take 64 queued vertices at a
+// time (wave stage, team sampler).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -13,26 +13,69 @@
 
 namespace rip {
 
-// Candidates a lane collects before their edges are read together (a block
-// draws two or three; four spill the team kernel's registers and measured 3%
-// slower there, two 4%).
+// Candidates a lane draws before their edges are read together (a block has
+// two or three; in the team kernel four measured 3% slower and two 4%).
 constexpr uint32_t kUnitBatch = 3;
 
-// Expands up to 64 queued vertices of the sample whose element 0 is z at
-// once, lane l holding the record rv of one (when `have`).  The rows' gap
-// blocks are the units of work: 64 units at a time, one per lane, found by a
-// wave scan of the block counts when some row has several (a hub's blocks
-// spread over the lanes instead of queueing in one).  A lane draws up to
+// Draws of up to K candidates of a gap block, for lanes with `more` set: the
+// next element x, pos of the block's len edges passed.  e[i] gets the i-th
+// candidate's position in the block and h[i] what its threshold must pass (0
+// for `uniform` rows, which keep every candidate); returns how many there
+// are, with x, pos and more moved on.  K elements and their gaps are computed
+// whether or not the block ends before them, apart from each other: one draw
+// is a chain of some forty dependent instructions, which is what a wave waits
+// for when it draws them one by one.
+template <int K>
+__device__ inline uint32_t ic_draw_block(uint64_t &x, uint32_t &pos, bool &more, uint32_t len,
+                                         uint32_t T, uint64_t q, double inv, bool uniform,
+                                         const Affine &A, const Affine &A2, const IcGapTab *tab,
+                                         uint32_t (&e)[K], uint32_t (&h)[K]) {
+  uint64_t xs[K];
+  double fg[K];
+  uint32_t gap[K];
+  xs[0] = x;
+#pragma unroll
+  for (int i = 1; i < K; ++i) xs[i] = aff_apply(A2, xs[i - 1]);
+#pragma unroll
+  for (int i = 0; i < K; ++i) fg[i] = ic_gap_real(xs[i], inv, tab);
+  bool sure = true;
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    sure = sure && ic_gap_sure(fg[i], inv);
+    gap[i] = static_cast<uint32_t>(__builtin_floor(fg[i]));
+  }
+  if (more && !sure) {
+#pragma unroll 1
+    for (int i = 0; i < K; ++i)
+      if (!ic_gap_sure(fg[i], inv)) gap[i] = ic_gap_near(xs[i], q, fg[i]);
+  }
+  uint32_t n = 0;
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    const bool is = more && gap[i] < len - pos;
+    e[i] = is ? pos + gap[i] : 0u;
+    h[i] = is && !uniform ? static_cast<uint32_t>(((aff_apply(A, xs[i]) >> 32) * T) >> 32) : 0u;
+    if (is) pos = e[i] + 1;
+    n += is ? 1u : 0u;
+    more = is && pos < len;
+  }
+  x = aff_apply(A2, xs[K - 1]);
+  return n;
+}
+
+// Expands up to 64 queued vertices at once, lane l holding the record rv of
+// one (when `have`), the element 0 z of its sample and the caller's tag of it.
+// The rows' gap blocks are the units of work: 64 units at a time, one per lane,
+// found by a wave scan of the block counts when some row has several (a hub's
+// blocks spread over the lanes instead of queueing in one).  A lane draws up to
 // kUnitBatch candidates of its block (arithmetic only), then the wave reads
-// their thresholds and in-neighbours together, so a unit waits for one trip
-// to memory, not one per candidate; take(live, src) gets every batch.  Against one draw per lane and
-// step, a whole row per lane: the stage's kernels of an IMM run on R-MAT scale
-// 22 weighted cascade took 13.5 ms instead of 15.6 (rows of one block there;
-// hub rows of U[0,0.1] graphs have hundreds).  Every lane of the wave must
-// call it.  Returns false as soon as take() does.
-template <typename Take>
+// their thresholds and in-neighbours together, so a unit waits for one trip to
+// memory, not one per candidate; take(live, src, tag) gets every batch (without
+// kIds the edges in place of their in-neighbours, which are not read).  Every
+// lane of the wave must call it.  Returns false as soon as take() does.
+template <bool kIds, typename Take>
 __device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *val, bool have,
-                                         const VertexRec &rv, uint64_t z,
+                                         const VertexRec &rv, uint64_t z, uint32_t tag,
                                          const Affine *p2, const IcGapTab *tab,
                                          unsigned long long &st_cand,
                                          unsigned long long &st_draws,
@@ -52,6 +95,7 @@ __device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *va
     uint64_t q = rv.q, x = x0;
     double inv = rv.inv;
     bool uniform = (rv.flags & kRowUniform) != 0;
+    uint32_t utag = tag;
     bool skip = true;
     if (single) {
       if (row) {
@@ -78,6 +122,7 @@ __device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *va
       q = __shfl(rv.q, src, 64);
       inv = __shfl(rv.inv, src, 64);
       x = __shfl(x0, src, 64);
+      utag = __shfl(tag, src, 64);
       uniform = (flags & kRowUniform) != 0;
       if (u < total) {
         const uint32_t beta = (flags >> kBetaShift) & 31u;
@@ -95,40 +140,17 @@ __device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *va
     uint32_t pos = 0;
     while (__ballot(more)) {
       uint32_t ce[kUnitBatch], th[kUnitBatch];
-      uint32_t nc = 0;
-#pragma unroll
-      for (uint32_t i = 0; i < kUnitBatch; ++i) {
-        ce[i] = 0;
-        th[i] = 0;
-        if (more) {
-          const uint32_t gap = ic_gap_draw(x, q, inv, tab);
-          if (gap >= len - pos) {
-            more = false;
-          } else {
-            pos += gap;
-            ce[i] = e0 + pos;
-            // kept iff the edge's threshold t passes this (ic_accept:
-            // hi32(a) T < t 2^32 for the acceptance element a)
-            if (!uniform)
-              th[i] = static_cast<uint32_t>(((aff_apply(P, x) >> 32) * T) >> 32);
-            nc = i + 1;
-            if (++pos < len) {
-              x = aff_apply(P2, x);                // next gap element
-              ++st_draws;
-            } else {
-              more = false;
-            }
-          }
-        }
-      }
+      const uint32_t nc = ic_draw_block<kUnitBatch>(x, pos, more, len, T, q, inv, uniform, P, P2, tab,
+                                                    ce, th);
+      st_draws += nc - (nc != 0 && pos == len ? 1u : 0u);
       uint32_t t[kUnitBatch], src[kUnitBatch];
 #pragma unroll
       for (uint32_t i = 0; i < kUnitBatch; ++i) {
         t[i] = 0xFFFFFFFFu;                        // rows sharing one threshold keep every candidate
         src[i] = 0;
         if (i < nc) {
-          src[i] = ids[ce[i]];
-          if (!uniform) t[i] = val[ce[i]];
+          src[i] = kIds ? ids[e0 + ce[i]] : e0 + ce[i];
+          if (!uniform) t[i] = val[e0 + ce[i]];
         }
       }
       st_cand += nc;
@@ -145,7 +167,7 @@ __device__ inline bool expand_rows_units(const uint32_t *ids, const uint32_t *va
           st_bytes += 4;
         }
       }
-      if (!take(live, src)) return false;
+      if (!take(live, src, utag)) return false;
     }
   }
   return true;

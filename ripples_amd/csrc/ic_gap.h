@@ -208,9 +208,8 @@ __host__ __device__ inline uint32_t ic_gap_settle(uint32_t hi, uint64_t q, uint3
   return static_cast<uint64_t>(g) * q <= N ? g : g - 1;
 }
 
-// ic_gap(x, q), with inv = ic_gap_inv(q).
-__host__ __device__ inline uint32_t ic_gap_draw(uint64_t x, uint64_t q, double inv,
-                                                const IcGapTab *t) {
+// NL(U) / q in double precision, U = hi32(x) + 1.
+__host__ __device__ inline double ic_gap_real(uint64_t x, double inv, const IcGapTab *t) {
   const uint32_t hi = static_cast<uint32_t>(x >> 32);
   const double u = static_cast<double>(hi) + 1.0;          // U, exact
   uint64_t bits;
@@ -228,11 +227,27 @@ __host__ __device__ inline uint32_t ic_gap_draw(uint64_t x, uint64_t q, double i
   s = __builtin_fma(r, s, -0.72134752044448170);
   s = __builtin_fma(r, s, 1.4426950408889634);
   const double nl = static_cast<double>(32 - e) - __builtin_fma(r, s, t->rl[2 * i + 1]);
-  const double fg = nl * inv;
-  const double fl = __builtin_floor(fg);
-  const double off = __builtin_fabs(fg - fl - 0.5);        // 0.5: right between two integers
-  if (off < __builtin_fma(inv, -0x1p-40, 0.5)) return static_cast<uint32_t>(fl);
-  return ic_gap_settle(hi, q, static_cast<uint32_t>(__builtin_rint(fg < 0.0 ? 0.0 : fg)));
+  return nl * inv;
+}
+
+// Whether floor(fg) is the gap, fg = ic_gap_real: off is 0.5 right between
+// two integers.
+__host__ __device__ inline bool ic_gap_sure(double fg, double inv) {
+  const double off = __builtin_fabs(fg - __builtin_floor(fg) - 0.5);
+  return off < __builtin_fma(inv, -0x1p-40, 0.5);
+}
+
+__host__ __device__ inline uint32_t ic_gap_near(uint64_t x, uint64_t q, double fg) {
+  return ic_gap_settle(static_cast<uint32_t>(x >> 32), q,
+                       static_cast<uint32_t>(__builtin_rint(fg < 0.0 ? 0.0 : fg)));
+}
+
+// ic_gap(x, q), with inv = ic_gap_inv(q).
+__host__ __device__ inline uint32_t ic_gap_draw(uint64_t x, uint64_t q, double inv,
+                                                const IcGapTab *t) {
+  const double fg = ic_gap_real(x, inv, t);
+  if (ic_gap_sure(fg, inv)) return static_cast<uint32_t>(__builtin_floor(fg));
+  return ic_gap_near(x, q, fg);
 }
 
 }  // namespace rip

@@ -105,6 +105,13 @@ struct WaveScratch {
   uint32_t *d_blist = nullptr;
   // lane kernel: per lane a visited table of 2 cap entries, a list of cap
   // vertices and an epoch; samples that outgrew a lane, sets to sort
+  // wave stage: per wave and slot a visited table of 2 cap entries and a list
+  // of cap vertices; sets to sort
+  uint64_t stage_waves = 0;
+  uint32_t *d_shtab = nullptr;
+  uint32_t *d_slist = nullptr;
+  uint64_t cap_ssort = 0;
+  uint32_t *d_ssort = nullptr;
   uint64_t lane_lanes = 0;
   uint32_t lane_cap = 0;
   unsigned long long *d_ltable = nullptr;
@@ -429,12 +436,18 @@ uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &
 // sample_ic_wave.hip: one BFS per wave over samples first + i, i in
 // [0, count), or first + ids[i]; returns how many samples outgrew the wave's
 // list, their indices (relative to first) in g->wave.d_big.  record_events:
-// bracket the kernel with the pool's ev0 / ev1.  vertex_parallel: expand 64
-// queued vertices at a time, a lane each, instead of one row per step.
-// stage: the wave stage of AUTO, timed into p->wave_ms / p->wave_stats.
+// bracket the kernel with the pool's ev0 / ev1.
 uint64_t ic_wave_launch(rip_pool *p, uint64_t first, uint64_t count, const uint32_t *ids,
-                        uint32_t out_chunk, bool record_events, bool vertex_parallel = false,
-                        bool stage = false);
+                        uint32_t out_chunk, bool record_events);
+// Workgroups (of 256) of a wave launch for `count` samples, and the pool
+// elements a wave reserves at a time.
+uint32_t ic_wave_blocks(uint64_t count);
+uint32_t ic_chunk(const rip_pool *p, uint64_t count, uint32_t out_chunk, uint64_t waves);
+// sample_ic_stage.hip: the same for the wave stage of AUTO, several samples
+// per wave, timed into p->wave_ms / p->wave_stats.
+uint64_t ic_stage_launch(rip_pool *p, uint64_t first, uint64_t count, const uint32_t *ids,
+                         uint32_t out_chunk, bool record_events);
+void stage_scratch_free(WaveScratch &w);
 // Most pool elements an IC sampling call of `count` samples can leave
 // unused (the rest of each wave's last output chunk).
 uint64_t ic_output_slack(const rip_pool *p, uint64_t count, const rip_tune *tune);

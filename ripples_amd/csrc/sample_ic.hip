@@ -683,7 +683,7 @@ uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &
   uint32_t launches = 0;
   if (count <= kWaveDirectMax && ic_wave_stage(tune)) {
     // few samples: one wave each from the start, with no lanes before
-    const uint64_t big = ic_wave_launch(p, first, count, nullptr, cfg.out_chunk, true, true, true);
+    const uint64_t big = ic_stage_launch(p, first, count, nullptr, cfg.out_chunk, true);
     launches += 2;
     if (big == 0) return launches;
     return launches + large_sets(p, first, big, p->g->wave.d_big, tune);
@@ -702,8 +702,7 @@ uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &
       if (ic_wave_stage(tune)) {
         // one BFS per wave, 64 frontier vertices at a time, for the samples
         // up to the wave list; the grid sampler takes the larger ones
-        const uint64_t big = ic_wave_launch(p, first, wave_count, wave_ids, cfg.out_chunk, false,
-                                            true, true);
+        const uint64_t big = ic_stage_launch(p, first, wave_count, wave_ids, cfg.out_chunk, false);
         launches += 2;
         if (big == 0) return launches;
         return launches + large_sets(p, first, big, p->g->wave.d_big, tune);

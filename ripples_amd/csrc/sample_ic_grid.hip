@@ -348,33 +348,12 @@ struct Expander {
       uint32_t pos = 0;
       while (__ballot(more)) {
         uint32_t ce[kUnitBatch], th[kUnitBatch], t[kUnitBatch];
-        uint32_t nc = 0;
-#pragma unroll
-        for (uint32_t i = 0; i < kUnitBatch; ++i) {
-          ce[i] = 0;
-          th[i] = 0;
-          if (more) {
-            const uint32_t gap = ic_gap_draw(x, q, inv, &S.tab);
-            if (gap >= len - pos) {
-              more = false;
-            } else {
-              pos += gap;
-              ce[i] = e0 + pos;
-              // kept iff the edge's threshold passes this (ic_accept)
-              if (!uniform) th[i] = static_cast<uint32_t>(((aff_apply(A, x) >> 32) * T) >> 32);
-              nc = i + 1;
-              if (++pos < len) {
-                x = aff_apply(A2, x);                // next gap element
-                ++gaps;
-              } else {
-                more = false;
-              }
-            }
-          }
-        }
+        const uint32_t nc = ic_draw_block<kUnitBatch>(x, pos, more, len, T, q, inv, uniform, A, A2,
+                                                      &S.tab, ce, th);
+        gaps += nc - (nc != 0 && pos == len ? 1u : 0u);
 #pragma unroll
         for (uint32_t i = 0; i < kUnitBatch; ++i)
-          t[i] = i < nc && !uniform ? P.val[ce[i]] : 0xFFFFFFFFu;
+          t[i] = i < nc && !uniform ? P.val[e0 + ce[i]] : 0xFFFFFFFFu;
         cand += nc;
         if (!uniform) vals += nc;
 #pragma unroll
@@ -383,7 +362,7 @@ struct Expander {
           const uint64_t m = __ballot(on);
           if (on) {
             const uint32_t at = qn + static_cast<uint32_t>(__popcll(m & lanes_below()));
-            S.qe[wid][at] = ce[i];
+            S.qe[wid][at] = e0 + ce[i];
             S.qg[wid][at] = gc;
             ++live;
           }

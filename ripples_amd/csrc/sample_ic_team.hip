@@ -70,7 +70,7 @@ __global__ void __launch_bounds__(BT, 4) ic_team_kernel(TeamParams P) {
   for (uint32_t w = tid; w < P.nw; w += BT) s_bits[w] = 0;
   unsigned long long st_cand = 0, st_draws = 0, st_exp = 0, st_bytes = 0, st_live = 0;
   // marks a batch's live edges' sources; the first visits join the queue
-  auto take = [&](const bool (&live)[kUnitBatch], const uint32_t (&src)[kUnitBatch]) {
+  auto take = [&](const bool (&live)[kUnitBatch], const uint32_t (&src)[kUnitBatch], uint32_t) {
     bool fresh[kUnitBatch];
     uint64_t m[kUnitBatch];
     uint32_t total = 0;
@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(BT, 4) ic_team_kernel(TeamParams P) {
         VertexRec rec{};
         if (have) rec = P.vrec[queue[b + lane]];
         st_exp += have ? 1u : 0u;
-        expand_rows_units(P.ids, P.val, have, rec, z, s_p2, &s_tab, st_cand, st_draws, st_bytes,
+        expand_rows_units<true>(P.ids, P.val, have, rec, z, 0u, s_p2, &s_tab, st_cand, st_draws, st_bytes,
                           st_live, take);
       }
       __syncthreads();

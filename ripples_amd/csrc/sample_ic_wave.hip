@@ -14,16 +14,14 @@
 //   list[CAP]    BFS queue and output list (FIFO in discovery order)
 // Expansion of a vertex: lane l draws the candidates of the row's gap
 // blocks l, l + 64, ... (one compare for a full block without candidates);
-// only live edges read their in-neighbour and touch the table (in the
-// vertex-parallel form, an LDS table first).  The finished list is sorted in
-// LDS (bitonic, 1024 entries per wave, 2048 in the vertex-parallel form) or,
-// if longer, in its HBM buffer.  Samples whose sets outgrow CAP are listed for
-// the large-set kernels.
+// only live edges read their in-neighbour and touch the table.  The finished
+// list is sorted in LDS (bitonic, 1024 entries per wave) or, if longer, in its
+// HBM buffer.  Samples whose sets outgrow CAP are listed for the large-set
+// kernels.
 #include <algorithm>
 
 #include "device_util.h"
 #include "ic_common.h"
-#include "ic_expand.h"
 #include "ic_gap.h"
 #include "internal.h"
 
@@ -31,15 +29,6 @@ namespace rip {
 namespace {
 
 constexpr uint32_t kSortCap = 1024;
-// Vertex-parallel form: the first kWaveLdsLimit vertices of a sample are
-// marked in a per-wave LDS table of kWaveLdsSlots 32-bit slots (vertex + 1,
-// 0 empty), cleared per sample; only later ones go to the wave's HBM table.
-// Most sets of this stage end below the limit, so most of its visited checks
-// never leave the CU.  The slots double as the wave's sort buffer once the
-// BFS is done.
-constexpr uint32_t kWaveLdsSlots = 2048;
-constexpr uint32_t kWaveLdsLimit = kWaveLdsSlots / 2;
-
 struct WaveParams {
   const VertexRec *vrec;
   const uint32_t *ids;
@@ -81,34 +70,6 @@ __device__ inline bool table_insert(unsigned long long *table, uint32_t mask,
       if (static_cast<uint32_t>(cur) == v) return false;
       break;  // occupied by another vertex of this sample
     }
-    h = (h + 1) & mask;
-  }
-}
-
-// Insert v into a wave's LDS table (power-of-two slots, fewer entries than
-// slots); true if it was not there yet.
-__device__ inline bool lds_insert(uint32_t *t, uint32_t mask, uint32_t v) {
-  const uint32_t want = v + 1u;
-  uint32_t h = hash_vertex(v) & mask;
-  for (;;) {
-    uint32_t cur = __hip_atomic_load(&t[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-    if (cur == 0) {
-      cur = atomicCAS(&t[h], 0u, want);
-      if (cur == 0) return true;
-    }
-    if (cur == want) return false;
-    h = (h + 1) & mask;
-  }
-}
-
-// Whether v is in a wave's LDS table.
-__device__ inline bool lds_find(const uint32_t *t, uint32_t mask, uint32_t v) {
-  const uint32_t want = v + 1u;
-  uint32_t h = hash_vertex(v) & mask;
-  for (;;) {
-    const uint32_t cur = __hip_atomic_load(&t[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-    if (cur == want) return true;
-    if (cur == 0) return false;
     h = (h + 1) & mask;
   }
 }
@@ -207,14 +168,10 @@ __device__ inline bool expand_row(const VertexRec *vrec, const uint32_t *ids,
   return true;
 }
 
-// VP: expand 64 queued vertices at a time (expand_rows_units) instead of
-// one row per step over its gap blocks (expand_row, the plain form), with
-// the first vertices of each sample marked in LDS.
-template <int BT, bool VP>
+template <int BT>
 __global__ void __launch_bounds__(BT, 4) ic_wave_kernel(WaveParams P) {
   constexpr int NW = BT / 64;
-  constexpr uint32_t kBuf = VP && kWaveLdsSlots > kSortCap ? kWaveLdsSlots : kSortCap;
-  __shared__ uint32_t s_sort[NW][kBuf];
+  __shared__ uint32_t s_sort[NW][kSortCap];
   const uint32_t lane = lane_id();
   const uint32_t wid = threadIdx.x >> 6;
   const uint64_t wave = static_cast<uint64_t>(blockIdx.x) * NW + wid;
@@ -243,80 +200,20 @@ __global__ void __launch_bounds__(BT, 4) ic_wave_kernel(WaveParams P) {
     const unsigned long long tag = static_cast<unsigned long long>(epoch) << 32;
     const uint64_t z = sample_z(P.seed, s);
     const uint32_t root = uniform_index(z, P.n);
-    uint32_t *ltab = s_sort[wid];
-    if (VP) {
-      for (uint32_t i = 4 * lane; i < kWaveLdsSlots; i += 256)
-        *reinterpret_cast<uint4 *>(&ltab[i]) = make_uint4(0, 0, 0, 0);
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    }
     if (lane == 0) {
-      if (VP)
-        lds_insert(ltab, kWaveLdsSlots - 1, root);
-      else
-        table_insert(table, tmask, tag, root);
+      table_insert(table, tmask, tag, root);
       list[0] = root;
     }
     uint32_t head = 0, tail = 1;
     bool big = false;
-    // vertex-parallel rounds: the records of the next round's first npre
-    // vertices, loaded with the current round's where the queue held them
-    uint32_t npre = 0;
-    VertexRec prec{};
-    // a visit call adds at most 64 vertices: while the sample stays within
-    // the LDS limit they go to the LDS table, then to the HBM table (after a
-    // look in the LDS one)
-    auto visit_vp = [&](uint32_t src) {
-      if (tail + 64u <= kWaveLdsLimit) return lds_insert(ltab, kWaveLdsSlots - 1, src);
-      if (lds_find(ltab, kWaveLdsSlots - 1, src)) return false;
-      return table_insert(table, tmask, tag, src);
-    };
-    // the first visits among a batch's live edges join the list; false when
-    // they could take it past the cap
-    auto take_vp = [&](const bool (&live)[kUnitBatch], const uint32_t (&src)[kUnitBatch]) {
-#pragma unroll
-      for (uint32_t i = 0; i < kUnitBatch; ++i) {
-        const uint64_t lm = __ballot(live[i]);
-        if (lm == 0) continue;
-        if (tail + __popcll(lm) > P.cap) return false;
-        const bool fresh = live[i] && visit_vp(src[i]);
-        const uint64_t fm = __ballot(fresh);
-        if (fresh) list[tail + __popcll(fm & lanes_below())] = src[i];
-        tail += __popcll(fm);
-      }
-      return true;
-    };
     while (head < tail && !big) {
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-      if (VP) {
-        const uint32_t take = min(tail - head, 64u);
-        const bool have = lane < take;
-        const uint32_t nhead = head + take;
-        // the next round's vertices already queued: their records load with
-        // this round's, off the next round's chain of dependent loads
-        const uint32_t nnext = min(tail - nhead, 64u);
-        const bool now = have && lane >= npre;
-        const bool next = lane < nnext;
-        const uint32_t v = now ? list[head + lane] : 0u;
-        const uint32_t vn = next ? list[nhead + lane] : 0u;
-        VertexRec rec = prec;
-        if (now) rec = P.vrec[v];
-        VertexRec recn{};
-        if (next) recn = P.vrec[vn];
-        head = nhead;
-        st_exp += take;
-        if (!expand_rows_units(P.ids, P.val, have, rec, z, s_p2, &s_tab, st_cand, st_draws,
-                               st_bytes, st_live, take_vp))
-          big = true;
-        prec = recn;
-        npre = nnext;
-      } else {
-        const uint32_t v = uniform_u32(list[head++]);
-        ++st_exp;
-        if (!expand_row(P.vrec, P.ids, P.val, v, z, s_p2, &s_tab, list, tail, P.cap, st_cand,
-                        st_draws, st_bytes, st_live,
-                        [&](uint32_t src) { return table_insert(table, tmask, tag, src); }))
-          big = true;
-      }
+      const uint32_t v = uniform_u32(list[head++]);
+      ++st_exp;
+      if (!expand_row(P.vrec, P.ids, P.val, v, z, s_p2, &s_tab, list, tail, P.cap, st_cand,
+                      st_draws, st_bytes, st_live,
+                      [&](uint32_t src) { return table_insert(table, tmask, tag, src); }))
+        big = true;
     }
     if (big) {
       if (lane == 0) {
@@ -331,7 +228,7 @@ __global__ void __launch_bounds__(BT, 4) ic_wave_kernel(WaveParams P) {
     while (cap2 < len) cap2 <<= 1;
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     const uint32_t *sorted;
-    if (cap2 <= kBuf) {
+    if (cap2 <= kSortCap) {
       uint32_t *a = s_sort[wid];
       for (uint32_t i = lane; i < len; i += 64) a[i] = list[i];
       wave_bitonic(a, len, cap2);
@@ -511,7 +408,7 @@ __global__ void reset_big_kernel(unsigned long long *ctl) { ctl[kCtlBigCounter] 
 template <int BT>
 uint32_t wave_grid() {
   return static_cast<uint32_t>(
-      blocks_per_cu(reinterpret_cast<const void *>(&ic_wave_kernel<BT, false>), BT) * cu_count());
+      blocks_per_cu(reinterpret_cast<const void *>(&ic_wave_kernel<BT>), BT) * cu_count());
 }
 
 }  // namespace
@@ -519,13 +416,6 @@ uint32_t wave_grid() {
 // Returns the number of samples left for the colour sampler (their local
 // indices are in g->wave.d_big).
 constexpr int kWaveBT = 256;
-// The stage's list where the team sampler takes the rest: a sample that
-// reaches a giant component is soon seen to, and the stage's work on it is
-// lost.  IMM with U[0,0.1] weights at 65,536 vertices took 23.9, 17.2, 15.9
-// and 15.7 ms with 4096, 2048, 1024 and 512; OPIM-C with weighted cascade at
-// 200,003 vertices 6.0 ms down to 1024 and 7.9 with 512.
-constexpr uint32_t kStageCapTeam = 1024;
-
 uint32_t ic_wave_blocks(uint64_t count) {
   return std::max<uint32_t>(
       1, std::min<uint64_t>(wave_grid<kWaveBT>(),
@@ -556,8 +446,7 @@ __global__ void reset_wave_kernel(unsigned long long *ctl) {
 }
 
 uint64_t ic_wave_launch(rip_pool *p, uint64_t first, uint64_t count, const uint32_t *ids,
-                        uint32_t out_chunk, bool record_events, bool vertex_parallel,
-                        bool stage) {
+                        uint32_t out_chunk, bool record_events) {
   constexpr int BT = kWaveBT;
   constexpr uint32_t CAP = 4096, TCAP = 8192;
   rip_graph *g = p->g;
@@ -593,7 +482,7 @@ uint64_t ic_wave_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
   P.table = w.d_table;
   P.list = w.d_list;
   P.epoch = w.d_epoch;
-  P.cap = stage && g->n <= kTeamMaxNodes ? kStageCapTeam : CAP;
+  P.cap = CAP;
   P.tcap = TCAP;
   P.big_ids = w.d_big;
   P.set_off = p->d_off;
@@ -605,22 +494,10 @@ uint64_t ic_wave_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
   P.sample_ids = ids;
   hipLaunchKernelGGL(reset_wave_kernel, dim3(1), dim3(1), 0, p->stream, p->d_ctl);
   if (record_events) RIP_HIP(hipEventRecord(p->ev0, p->stream));
-  if (stage) RIP_HIP(hipEventRecord(p->ev3, p->stream));
-  if (vertex_parallel)
-    hipLaunchKernelGGL((ic_wave_kernel<BT, true>), dim3(blocks), dim3(BT), 0, p->stream, P);
-  else
-    hipLaunchKernelGGL((ic_wave_kernel<BT, false>), dim3(blocks), dim3(BT), 0, p->stream, P);
+  hipLaunchKernelGGL((ic_wave_kernel<BT>), dim3(blocks), dim3(BT), 0, p->stream, P);
   RIP_HIP(hipGetLastError());
   if (record_events) RIP_HIP(hipEventRecord(p->ev1, p->stream));
-  if (stage) RIP_HIP(hipEventRecord(p->ev4, p->stream));
   pool_read_ctl(p, record_events);
-  if (stage) {
-    float ms = 0.0f;
-    RIP_HIP(hipEventElapsedTime(&ms, p->ev3, p->ev4));
-    p->wave_ms = ms;
-    p->wave_ran = true;
-    for (int i = 0; i < RIP_STAT_COUNT; ++i) p->wave_stats[i] = p->h_ctl[kCtlStatBytes + i];
-  }
   return p->h_ctl[kCtlLongCount];
 }
 

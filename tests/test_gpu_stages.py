@@ -114,3 +114,43 @@ def test_grid_sampler_hub_rows_match_oracle(deg, count, cap, orc):
         assert np.array_equal(off, eo) and np.array_equal(ver, ev)
     p.close()
     g.close()
+
+
+def cycles_csr(lengths, reps, isolated):
+    """Cycles whose edges are all live in both directions (a set is its root's
+    whole cycle) and isolated vertices."""
+    s, d, at = [], [], 0
+    for length in np.tile(lengths, reps):
+        v = at + np.arange(length)
+        u = at + (np.arange(length) + 1) % length
+        s += [v, u]
+        d += [u, v]
+        at += length
+    s, d = np.concatenate(s), np.concatenate(d)
+    return transposed_csr(at + isolated, s, d, np.ones(len(s), np.float32))
+
+
+SHORT = [3, 15, 16, 17, 18, 31, 63, 64, 65, 66, 95, 96, 97, 127, 128, 129, 255, 256, 257]
+LONG = SHORT + [191, 192, 193, 383, 384, 385, 511, 512, 513, 767, 768, 769, 1023, 1024, 1025]
+WIDE = LONG + [1535, 1536, 2047, 2048, 2049, 4095, 4096, 4097]
+
+
+@pytest.mark.parametrize("lengths,reps,isolated,count", [
+    (LONG, 3, 100, 1),
+    (LONG, 3, 100, 4000),              # a sample per wave
+    (LONG, 3, 100, 16384),             # two
+    (SHORT, 40, 100, 45000),           # lanes first, four per wave behind them
+    (WIDE, 6, 1 << 20, 1500),          # past 2^20 vertices: sets of up to 4096
+    (WIDE, 6, 1 << 20, 17000),
+])
+def test_wave_stage_set_lengths_match_oracle(lengths, reps, isolated, count, orc):
+    index, edges, w = cycles_csr(lengths, reps, isolated)
+    g = R.Graph(index, edges, w, model=R.IC)
+    p = g.pool(3)
+    for first in (0, count):           # the second call finds the scratch of the first
+        p.generate_rrr_sets(count)
+        off, ver = p.export(first, count)
+        eo, ev = orc.sample(R.IC, index, edges, w, 3, first, count)
+        assert np.array_equal(off, eo) and np.array_equal(ver, ev)
+    p.close()
+    g.close()
