@@ -53,8 +53,9 @@ typedef struct {
   uint32_t queue_cap;    /* IC lane sampler: vertices one lane's sample may
                             reach before the wave sampler takes it over:
                             64, 256, 1024, 2048 or 4096.  0 = automatic: AUTO
-                            runs the wave stage below behind lanes of 64
-                            vertices, LANE takes 1024 */
+                            runs the wave stage below, LANE takes 1024.  With
+                            the wave stage behind them lanes hand over at 16
+                            vertices, whatever is given */
   uint32_t heavy_degree; /* IC: rows this long wait for the hub phase */
   uint32_t sampler;      /* IC: RIP_SAMPLER_AUTO, _WAVE or _COLOUR */
   uint32_t out_chunk;    /* LT and IC wave sampler: pool elements a wave
@@ -67,7 +68,7 @@ typedef struct {
                             first run several per wave, 64 frontier vertices at
                             a time, up to 4096 vertices (1024 on graphs of up to
                             2^20 vertices), and only the larger ones go on;
-                            calls of up to 16,384 samples start there, with no
+                            calls of up to 4,096 samples start there, with no
                             lanes before */
 } rip_tune;
 

@@ -473,7 +473,8 @@ void team_scratch_free(TeamScratch &s);
 // returns how many outgrew a lane's queue, their indices (relative to first)
 // in g->wave.d_over.  Brackets its main kernel with the pool's ev0 / ev1.
 constexpr uint32_t kLaneCapDefault = 1024;
-constexpr uint32_t kLaneCapStaged = 64;   // with the wave stage behind the lanes
+constexpr uint32_t kLaneCapStaged = 64;   // with the wave stage behind them (which then
+                                          // start at 16 vertices: sample_ic_lane.hip)
 // Whether an AUTO call runs the wave stage: asked for, or no queue_cap given.
 bool ic_wave_stage(const rip_tune *tune);
 uint32_t ic_lane_cap(const rip_tune *tune);

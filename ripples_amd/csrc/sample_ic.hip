@@ -667,15 +667,15 @@ static uint32_t large_sets(rip_pool *p, uint64_t first, uint64_t count, const ui
   return ic_grid_launch(p, first, count, ids, true, frontier_cap, colors ? colors : 64u);
 }
 
-// Calls of at most this many samples skip the lanes: a lane takes about
-// 0.4 ms to walk a sample of 64 vertices, whatever the launch holds, where a
-// wave of the stage takes under 0.1 ms.  IMM on 1,000 vertices (weighted
-// cascade, k = 5, eps = 0.5): 2.45 ms with the lanes, 1.33 without; OPIM-C on
-// 200,003 vertices (calls of a few thousand sets): 10.3 and 6.9 ms.  Past
-// this the stage's few thousand resident waves become the limit, where the
-// lanes hold hundreds of thousands of samples (thresholds of 4,096 and 65,536
-// measured the same on these and on IMM and serving at 65K-262K vertices).
-constexpr uint64_t kWaveDirectMax = 16384;
+// Calls of at most this many samples skip the lanes: they fill the stage's
+// waves just so, and a kernel and a host synchronisation are saved.  IMM on
+// 1,000 vertices (weighted cascade, k = 5, eps = 0.5): 1.2 ms with the lanes,
+// 0.97 without; OPIM-C on 200,003 vertices (calls of a few thousand sets): 5.6
+// and 5.2 ms.  Past it the lanes, which hold hundreds of thousands of samples,
+// are the better place for the short ones: twelve served queries took 29.5,
+// 29.4, 30.8 and 31.1 ms with lines of 1,024, 4,096, 16,384 and 65,536, the
+// rest measured the same with all four.
+constexpr uint64_t kWaveDirectMax = 4096;
 
 uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &cfg,
                    const rip_tune *tune) {

@@ -18,6 +18,9 @@
 // Finished sets of up to 16 vertices are sorted by the lane in registers
 // and written through the wave's output chunk; longer ones are written
 // unsorted, listed, and sorted by ic_lane_sort_kernel afterwards.
+//
+// With the wave stage behind the lanes another kernel takes their place
+// (ic_short_kernel, below).
 #include <algorithm>
 
 #include "device_util.h"
@@ -75,12 +78,9 @@ __device__ inline void cswap(uint32_t &a, uint32_t &b) {
   b = hi;
 }
 
-// Sorts list[0, len) for len <= 16 in registers (bitonic network over 16
-// slots padded with kEmptyVertex; every index is a compile-time constant).
-__device__ inline void sort16(uint32_t *list, uint32_t len) {
-  uint32_t r[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) r[i] = i < static_cast<int>(len) ? list[i] : kEmptyVertex;
+// Sorts 16 values in registers (bitonic network; every index is a
+// compile-time constant).
+__device__ inline void sort_regs(uint32_t (&r)[16]) {
 #pragma unroll
   for (int k = 2; k <= 16; k <<= 1) {
 #pragma unroll
@@ -97,6 +97,14 @@ __device__ inline void sort16(uint32_t *list, uint32_t len) {
       }
     }
   }
+}
+
+// Sorts list[0, len) for len <= 16 in registers, padded with kEmptyVertex.
+__device__ inline void sort16(uint32_t *list, uint32_t len) {
+  uint32_t r[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r[i] = i < static_cast<int>(len) ? list[i] : kEmptyVertex;
+  sort_regs(r);
 #pragma unroll
   for (int i = 0; i < 16; ++i)
     if (i < static_cast<int>(len)) list[i] = r[i];
@@ -295,6 +303,228 @@ __global__ void __launch_bounds__(BT) ic_lane_kernel(LaneParams P) {
   report_stats(P.ctl, st_bytes, st_cand, st_draws, st_exp, st_live);
 }
 
+// The lanes in front of the wave stage: a sample per lane as above, up to
+// kShort vertices, in rounds.  A round takes every lane through a vertex: the
+// next of its list (LDS, which is also the visited set: a scan of at most
+// kShort entries), its record, up to kShortDraws candidates of the current gap
+// block, their edges read together.  So a round waits for two trips to memory
+// where the kernel above, whose steps meet lanes in every state, waits for
+// half a dozen to do a third as much.  Finished lanes wait until kShortDone of
+// them can be written (and replaced) together (8, 16 and 32 measured alike).
+// A million samples of R-MAT scale 22 under weighted cascade: 1.94 ms with the
+// kernel above and 64 vertices, 1.48 with it and 16, 0.98 with this one.
+constexpr uint32_t kShort = 16;
+constexpr uint32_t kShortDraws = 3;
+constexpr int kShortDone = 16;
+
+template <int BT>
+__global__ void __launch_bounds__(BT, 4) ic_short_kernel(LaneParams P) {
+  __shared__ Affine s_p2[64];
+  __shared__ IcGapTab s_tab;
+  __shared__ uint32_t s_list[BT / 64][kShort][64];
+  if (threadIdx.x == 0) fill_step_powers(P.step, s_p2);
+  ic_load_tables(&s_tab);
+  __syncthreads();
+  const uint32_t lane = lane_id();
+  uint32_t(*list)[64] = s_list[threadIdx.x >> 6];
+  const Affine Pst = uniform_affine(s_p2[0]), P2 = uniform_affine(s_p2[1]);
+  // wave-uniform: the claimed range of sample indices and the output chunk
+  uint64_t next = 0, hi = 0;
+  bool left = true;
+  unsigned long long out_cur = 0, out_end = 0;
+  // lane state: a sample (held) with its list, a row of it (in_row)
+  bool held = false, in_row = false;
+  uint32_t idx = 0, head = 0, tail = 0;
+  uint64_t z = 0;
+  uint32_t begin = 0, deg = 0, T = 0, beta = 0, nblk = 0, k = 0, pos = 0, len = 0;
+  uint32_t ufull = 0, ulast = 0;
+  uint64_t q = 0, xb = 0, x = 0;
+  double inv = 0.0;
+  bool uniform = true;
+  unsigned long long st_cand = 0, st_draws = 0, st_exp = 0, st_bytes = 0, st_live = 0;
+
+  // block k of the row, whose first element is xb
+  auto open_block = [&]() {
+    x = xb;
+    pos = 0;
+    len = min(deg - (k << beta), 1u << beta);
+    ++st_draws;
+    // a block without candidates costs one compare
+    if ((xb >> 32) + 1 <= (len == (1u << beta) ? ufull : ulast)) pos = len;
+  };
+  for (;;) {
+    const bool done = held && !in_row && head == tail;
+    const uint64_t dm = __ballot(done), am = __ballot(held && !done);
+    if (__popcll(dm) + (left ? 64 - __popcll(__ballot(held)) : 0) >= kShortDone || am == 0) {
+      // ---- finished sets, in vertex order, through the wave's output chunk
+      if (dm) {
+        uint32_t r[kShort];
+#pragma unroll
+        for (uint32_t i = 0; i < kShort; ++i) r[i] = done && i < tail ? list[i][lane] : kEmptyVertex;
+        sort_regs(r);
+        const uint32_t flen = done ? tail : 0u;
+        const uint32_t incl = wave_inclusive_scan(flen);
+        const uint32_t total = uniform_u32(__shfl(incl, 63, 64));
+        if (out_end - out_cur < total) {
+          const unsigned long long want = total > P.chunk ? total : P.chunk;
+          unsigned long long nb = 0;
+          if (lane == 0) nb = atomicAdd(&P.ctl[kCtlDataBump], want);
+          nb = uniform_u64(nb);
+          out_cur = nb;
+          out_end = nb + want;
+        }
+        const unsigned long long base = out_cur + incl - flen;
+        out_cur += total;
+        if (done) {
+          const uint64_t s = P.first + idx;
+          if (base + flen > P.cap_data) {
+            atomicOr(&P.ctl[kCtlOverflow], 1ull);
+            P.set_len[s] = kLenFail;
+          } else {
+#pragma unroll
+            for (uint32_t i = 0; i < kShort; ++i)
+              if (i < flen) P.data[base + i] = r[i];
+            P.set_off[s] = base;
+            P.set_len[s] = flen;
+            st_bytes += 4ull * flen;
+          }
+          held = false;
+        }
+      }
+      // ---- idle lanes take the next ids of the wave's claimed range
+      uint64_t im = __ballot(!held);
+      while (left && im) {
+        if (next >= hi) {
+          unsigned long long c = 0;
+          if (lane == 0)
+            c = atomicAdd(&P.ctl[kCtlGroupCounter], static_cast<unsigned long long>(kLaneClaim));
+          c = uniform_u64(c);
+          next = std::min<uint64_t>(c, P.count);
+          hi = std::min<uint64_t>(c + kLaneClaim, P.count);
+          if (next >= hi) {
+            left = false;
+            break;
+          }
+        }
+        const uint64_t my = next + __popcll(im & lanes_below());
+        next = std::min<uint64_t>(next + __popcll(im), hi);
+        if (!held && my < hi) {
+          idx = static_cast<uint32_t>(my);
+          z = sample_z(P.seed, P.first + idx);
+          list[0][lane] = uniform_index(z, P.n);
+          head = 0;
+          tail = 1;
+          held = true;
+          in_row = false;
+        }
+        im = __ballot(!held);
+      }
+      if (__ballot(held) == 0) break;
+    }
+    // ---- the next vertex of lanes between rows
+    if (held && !in_row && head < tail) {
+      const VertexRec rv = P.vrec[list[head++][lane]];
+      ++st_exp;
+      T = rv.thr;
+      if (T != 0) {
+        in_row = true;
+        begin = rv.begin;
+        deg = rv.end - rv.begin;
+        uniform = (rv.flags & kRowUniform) != 0;
+        beta = (rv.flags >> kBetaShift) & 31u;
+        q = rv.q;
+        inv = rv.inv;
+        ufull = rv.ufull;
+        ulast = rv.ulast;
+        nblk = ((deg - 1) >> beta) + 1;
+        k = 0;
+        xb = rv.ja * z + rv.jb;                    // the row's first element
+        open_block();
+      }
+    }
+    // ---- up to kShortDraws draws of the row
+    uint32_t e[kShortDraws], th[kShortDraws], t[kShortDraws], u[kShortDraws];
+    bool cand[kShortDraws];
+#pragma unroll
+    for (uint32_t i = 0; i < kShortDraws; ++i) {
+      cand[i] = false;
+      e[i] = 0;
+      th[i] = 0;
+      if (in_row) {
+        if (pos < len) {
+          const uint32_t gap = ic_gap_draw(x, q, inv, &s_tab);
+          if (gap >= len - pos) {
+            pos = len;
+          } else {
+            pos += gap;
+            e[i] = begin + (k << beta) + pos;
+            cand[i] = true;
+            // kept iff the edge's threshold passes this (ic_accept)
+            if (!uniform) th[i] = static_cast<uint32_t>(((aff_apply(Pst, x) >> 32) * T) >> 32);
+            x = aff_apply(P2, x);                  // next gap element
+            if (++pos < len) ++st_draws;
+          }
+        }
+        if (pos >= len) {
+          if (++k < nblk) {
+            xb = aff_apply(s_p2[beta + 1], xb);    // 2 B elements: the next block
+            open_block();
+          } else {
+            in_row = false;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kShortDraws; ++i) {
+      t[i] = 0xFFFFFFFFu;
+      u[i] = 0;
+      if (cand[i]) {
+        u[i] = P.ids[e[i]];
+        ++st_cand;
+        if (!uniform) {
+          t[i] = P.val[e[i]];
+          ++st_draws;
+          st_bytes += 4;
+        }
+      }
+    }
+    bool over = false;
+#pragma unroll
+    for (uint32_t i = 0; i < kShortDraws; ++i) {
+      if (cand[i] && t[i] > th[i] && !over) {
+        ++st_live;
+        st_bytes += 4;
+        bool fresh = true;
+        for (uint32_t j = 0; j < tail; ++j)
+          if (list[j][lane] == u[i]) {
+            fresh = false;
+            break;
+          }
+        if (fresh) {
+          if (tail == kShort)
+            over = true;
+          else
+            list[tail++][lane] = u[i];
+        }
+      }
+    }
+    // ---- too large for a lane: the wave stage redoes them
+    const uint64_t om = __ballot(over);
+    if (om) {
+      unsigned long long b = 0;
+      if (lane == 0)
+        b = atomicAdd(&P.ctl[kCtlLongCount], static_cast<unsigned long long>(__popcll(om)));
+      b = uniform_u64(b);
+      if (over) {
+        P.over_ids[b + __popcll(om & lanes_below())] = idx;
+        held = in_row = false;
+      }
+    }
+  }
+  report_stats(P.ctl, st_bytes + kIcRecBytes * st_exp, st_cand, st_draws, st_exp, st_live);
+}
+
 // Sorts the sets the lane kernel wrote unsorted (17 .. cap vertices), one
 // wave per set, bitonic in LDS.
 template <int BT, int CAP>
@@ -392,9 +622,15 @@ uint64_t ic_lane_launch(rip_pool *p, uint64_t first, uint64_t count, const rip_t
   rip_graph *g = p->g;
   WaveScratch &w = g->wave;
   const uint32_t cap = ic_lane_cap(tune);
-  const uint32_t bt = ic_lane_block(tune);
-  const uint64_t lanes = lane_lanes(count, cap, bt);
-  if (w.lane_lanes < lanes || w.lane_cap != cap) {
+  const bool staged = ic_wave_stage(tune);
+  uint32_t bt = ic_lane_block(tune);
+  uint64_t lanes = lane_lanes(count, cap, bt);
+  if (staged) {
+    // within the lanes that the output slack is sized for
+    bt = kLaneBT;
+    const int per_cu = blocks_per_cu(reinterpret_cast<const void *>(&ic_short_kernel<kLaneBT>), kLaneBT);
+    lanes = std::min<uint64_t>(lanes, static_cast<uint64_t>(per_cu) * cu_count() * kLaneBT);
+  } else if (w.lane_lanes < lanes || w.lane_cap != cap) {
     dev_free(w.d_ltable);
     dev_free(w.d_llist);
     dev_free(w.d_lepoch);
@@ -445,6 +681,13 @@ uint64_t ic_lane_launch(rip_pool *p, uint64_t first, uint64_t count, const rip_t
   hipLaunchKernelGGL(reset_lane_kernel, dim3(1), dim3(1), 0, p->stream, p->d_ctl);
   RIP_HIP(hipEventRecord(p->ev0, p->stream));
   const dim3 grid(static_cast<uint32_t>(lanes / bt));
+  if (staged) {
+    hipLaunchKernelGGL((ic_short_kernel<kLaneBT>), grid, dim3(kLaneBT), 0, p->stream, P);
+    RIP_HIP(hipGetLastError());
+    RIP_HIP(hipEventRecord(p->ev1, p->stream));
+    pool_read_ctl(p, true);
+    return p->h_ctl[kCtlLongCount];
+  }
   switch (bt) {
     case 512: hipLaunchKernelGGL((ic_lane_kernel<512>), grid, dim3(512), 0, p->stream, P); break;
     case 1024: hipLaunchKernelGGL((ic_lane_kernel<1024>), grid, dim3(1024), 0, p->stream, P); break;

@@ -137,8 +137,9 @@ WIDE = LONG + [1535, 1536, 2047, 2048, 2049, 4095, 4096, 4097]
 
 @pytest.mark.parametrize("lengths,reps,isolated,count", [
     (LONG, 3, 100, 1),
-    (LONG, 3, 100, 4000),              # a sample per wave
-    (LONG, 3, 100, 16384),             # two
+    (LONG, 3, 100, 4096),              # a sample per wave
+    (LONG, 3, 100, 4097),              # lanes first from here on
+    (LONG, 3, 100, 19000),             # two per wave
     (SHORT, 40, 100, 45000),           # lanes first, four per wave behind them
     (WIDE, 6, 1 << 20, 1500),          # past 2^20 vertices: sets of up to 4096
     (WIDE, 6, 1 << 20, 17000),
