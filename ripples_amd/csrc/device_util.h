@@ -33,6 +33,19 @@ __device__ inline uint32_t wave_inclusive_scan(uint32_t x) {
   return x;
 }
 
+// The largest x of the wave, in every lane: rows of 16 by DPP shifts, then the
+// rows' last lanes broadcast onward to lane 63.
+__device__ inline uint32_t wave_max_u32(uint32_t x) {
+  auto step = [&](uint32_t y) { x = max(x, y); };
+  step(__builtin_amdgcn_update_dpp(0u, x, 0x111, 0xF, 0xF, false));   // row_shr 1
+  step(__builtin_amdgcn_update_dpp(0u, x, 0x112, 0xF, 0xF, false));   // row_shr 2
+  step(__builtin_amdgcn_update_dpp(0u, x, 0x114, 0xF, 0xF, false));   // row_shr 4
+  step(__builtin_amdgcn_update_dpp(0u, x, 0x118, 0xF, 0xF, false));   // row_shr 8
+  step(__builtin_amdgcn_update_dpp(0u, x, 0x142, 0xA, 0xF, false));   // row_bcast 15
+  step(__builtin_amdgcn_update_dpp(0u, x, 0x143, 0xC, 0xF, false));   // row_bcast 31
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
 __device__ inline uint32_t wave_sum(uint32_t x) {
   return __shfl(wave_inclusive_scan(x), 63, 64);
 }
