@@ -236,8 +236,14 @@ def measure(name, seed, steps, warmup, batch, tune, host, cpu_s, with_cpu_imm, f
             "call_ms": call_ms}
     if wl["model"] == R.IC:
         per_launch = ks["algo_bytes"]
-        roof["kernel"] = "ic_lane_kernel" if (tune or {}).get("sampler", 0) in (0, 3) \
-            else "ic_wave_kernel"
+        tn = tune or {}
+        staged = tn.get("sampler", 0) == 0 and (not tn.get("queue_cap") or tn.get("wave_stage"))
+        roof["kernel"] = "ic_short_kernel" if staged else \
+            "ic_lane_kernel" if tn.get("sampler", 0) in (0, 3) else "ic_wave_kernel"
+        # up to 2^20 vertices the large sets get a workgroup each
+        team = wl["scale"] <= 20 and not tn.get("colors") and not tn.get("frontier_cap")
+        large = "ic_team_kernel (one sample per workgroup)" if team \
+            else "grid_level_kernel (all BFS levels of the call)"
         grid_ms = float(np.mean([gr[0] for gr in grids]))
         grid_levels = float(np.mean([gr[1] for gr in grids]))
         grid_bytes = float(np.mean([gr[2]["algo_bytes"] for gr in grids]))
@@ -248,12 +254,12 @@ def measure(name, seed, steps, warmup, batch, tune, host, cpu_s, with_cpu_imm, f
         roof["grid_levels_ms"] = grid_ms
         roof["grid_levels"] = grid_levels
         # the dominant kernel of the call: the lane kernel, the wave stage's
-        # kernel (samples past the lane capacity) or the grid sampler's level
-        # kernels (timed over all levels)
+        # kernel (samples past the lane capacity), or the team kernel or the grid
+        # sampler's level kernels (timed over all levels) for the large sets
         stage_ms, stage_kernel, stage_bytes = max(
             (kernel_ms, roof["kernel"], per_launch),
-            (wave_ms, "ic_wave_kernel (vertex-parallel wave stage)", wave_bytes),
-            (grid_ms, "grid_level_kernel (all BFS levels of the call)", grid_bytes))
+            (wave_ms, "ic_stage_kernel (wave stage)", wave_bytes),
+            (grid_ms, large, grid_bytes))
         roof["kernel"] = stage_kernel
         per_launch = stage_bytes
         kernel_ms = stage_ms
