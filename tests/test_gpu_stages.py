@@ -24,7 +24,7 @@ GRAPHS = {
 
 
 @pytest.mark.parametrize("name", sorted(GRAPHS))
-@pytest.mark.parametrize("count", [1, 63, 64, 65, 16384, 16385])
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 4096, 4097, 16385])
 def test_automatic_setting_matches_oracle(name, count, orc):
     index, edges, w = GRAPHS[name]()
     g = R.Graph(index, edges, w, model=R.IC)
