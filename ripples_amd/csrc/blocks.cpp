@@ -35,9 +35,7 @@ Registry &registry() {
 }  // namespace
 
 BlockCache::BlockCache(int device) : device_(device) {
-  size_t free_b = 0, total_b = 0;
-  RIP_HIP(hipMemGetInfo(&free_b, &total_b));
-  limit_ = total_b / kIdleShare;
+  limit_ = device_total_bytes(device) / kIdleShare;
   std::lock_guard<std::mutex> hold(registry().mu);
   registry().all.insert(this);
 }
@@ -160,6 +158,12 @@ void *device_malloc(size_t bytes) {
     throw Error(-2, std::string("hipMalloc of ") + std::to_string(bytes) +
                         " bytes failed: " + hipGetErrorString(e));
   return p;
+}
+
+uint64_t device_total_bytes(int device) {
+  size_t total_b = 0;
+  RIP_HIP(hipDeviceTotalMem(&total_b, device));
+  return total_b;
 }
 
 uint64_t device_free_bytes() {

@@ -542,7 +542,9 @@ IcLaunch ic_tune(const rip_pool *p, const rip_tune *tune) {
   (void)ic_lane_cap(tune);  // validates queue_cap
   RIP_REQUIRE(c.block == 256 || c.block == 512 || c.block == 1024, -1,
               "tune: block must be 256, 512 or 1024");
-  if (c.slots == 0) {
+  // (only the colour sampler's kernel has slots; asking for the free memory takes
+  // the driver tens of microseconds)
+  if (c.slots == 0 && c.sampler == RIP_SAMPLER_COLOUR) {
     const size_t free_b = device_free_bytes();
     const size_t per = slot_bytes_for(p->g, c.heavy_degree);
     // keep the sampler scratch within an eighth of the memory it may use

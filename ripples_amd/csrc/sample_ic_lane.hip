@@ -599,10 +599,9 @@ static const void *lane_kernel_ptr(uint32_t bt) {
 // Lanes of a lane-sampler launch of `count` samples: every resident lane,
 // at most one per sample, within 1/16 of the device memory; a multiple of
 // the block size bt.
-static uint64_t lane_lanes(uint64_t count, uint32_t cap, uint32_t bt) {
+static uint64_t lane_lanes(int device, uint64_t count, uint32_t cap, uint32_t bt) {
   const int per_cu = blocks_per_cu(lane_kernel_ptr(bt), static_cast<int>(bt));
-  size_t free_b = 0, total_b = 0;
-  RIP_HIP(hipMemGetInfo(&free_b, &total_b));
+  const uint64_t total_b = device_total_bytes(device);
   const uint64_t per_lane = 20ull * cap + 4;       // table 16 cap + list 4 cap + epoch
   uint64_t lanes = static_cast<uint64_t>(per_cu) * cu_count() * bt;
   lanes = std::min<uint64_t>(lanes, std::max<uint64_t>(bt, (total_b / 16) / per_lane));
@@ -611,7 +610,7 @@ static uint64_t lane_lanes(uint64_t count, uint32_t cap, uint32_t bt) {
 }
 
 uint64_t ic_lane_slack(const rip_pool *p, uint64_t count, const rip_tune *tune) {
-  const uint64_t waves = lane_lanes(count, ic_lane_cap(tune), ic_lane_block(tune)) / 64;
+  const uint64_t waves = lane_lanes(p->g->device, count, ic_lane_cap(tune), ic_lane_block(tune)) / 64;
   const uint32_t chunk = tune && tune->out_chunk ? tune->out_chunk : 0;
   return waves * (chunk ? chunk : 4096u);
 }
@@ -624,7 +623,7 @@ uint64_t ic_lane_launch(rip_pool *p, uint64_t first, uint64_t count, const rip_t
   const uint32_t cap = ic_lane_cap(tune);
   const bool staged = ic_wave_stage(tune);
   uint32_t bt = ic_lane_block(tune);
-  uint64_t lanes = lane_lanes(count, cap, bt);
+  uint64_t lanes = lane_lanes(g->device, count, cap, bt);
   if (staged) {
     // within the lanes that the output slack is sized for
     bt = kLaneBT;

@@ -515,8 +515,7 @@ void ic_big_launch(rip_pool *p, uint64_t first, uint64_t count) {
   WaveScratch &w = g->wave;
   const uint32_t words = (g->n + 31) / 32, swords = (words + 31) / 32;
   const uint64_t per_wave = 4ull * (static_cast<uint64_t>(g->n) + words + swords);
-  size_t free_b = 0, total_b = 0;
-  RIP_HIP(hipMemGetInfo(&free_b, &total_b));
+  const uint64_t total_b = device_total_bytes(g->device);
   const int per_cu = blocks_per_cu(reinterpret_cast<const void *>(&ic_big_kernel<BT>), BT);
   const int cus = cu_count();
   uint64_t waves = std::min<uint64_t>(static_cast<uint64_t>(per_cu) * cus * (BT / 64),
