@@ -467,6 +467,7 @@ uint64_t ic_wave_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
   }
   if (w.cap_big < count) {
     dev_free(w.d_big);
+    w.cap_big = 0;
     w.d_big = dev_alloc<uint32_t>(count);
     w.cap_big = count;
   }

@@ -734,6 +734,7 @@ uint32_t lt_launch(rip_pool *p, uint64_t first, uint64_t count,
   // long-walk ids: at most `count`
   if (p->g->lt.cap_ids < count) {
     dev_free(p->g->lt.d_long_ids);
+    p->g->lt.cap_ids = 0;
     p->g->lt.d_long_ids = dev_alloc<uint32_t>(count);
     p->g->lt.cap_ids = count;
   }
@@ -742,6 +743,7 @@ uint32_t lt_launch(rip_pool *p, uint64_t first, uint64_t count,
   const uint64_t spill_words = static_cast<uint64_t>(blocks) * BT * SPILL;
   if (p->g->lt.cap_spill < spill_words) {
     dev_free(p->g->lt.d_spill);
+    p->g->lt.cap_spill = 0;
     p->g->lt.d_spill = dev_alloc<uint32_t>(spill_words);
     p->g->lt.cap_spill = spill_words;
   }

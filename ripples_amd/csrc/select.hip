@@ -671,27 +671,36 @@ void ensure_select_scratch(rip_pool *p, uint64_t num_sets, uint64_t inv_elems,
     s.d_cursor = pool_alloc<unsigned long long>(p, n);
     s.n = n;
   }
+  // (a capacity is zero while its buffers are being replaced: an allocation
+  // may fail, and the next call must not take them for there)
   if (s.cap_sets < num_sets) {
+    const uint64_t cap = std::max<uint64_t>(num_sets, s.cap_sets + s.cap_sets / 2);
     pool_free(p, s.d_covered);
     pool_free(p, s.d_soff);
-    s.cap_sets = std::max<uint64_t>(num_sets, s.cap_sets + s.cap_sets / 2);
-    s.d_covered = pool_alloc<uint8_t>(p, s.cap_sets);
-    s.d_soff = pool_alloc<unsigned long long>(p, s.cap_sets + 1);
+    s.cap_sets = 0;
+    s.d_covered = pool_alloc<uint8_t>(p, cap);
+    s.d_soff = pool_alloc<unsigned long long>(p, cap + 1);
+    s.cap_sets = cap;
   }
   if (s.cap_elems < inv_elems) {
+    const uint64_t cap = std::max<uint64_t>(inv_elems, s.cap_elems + s.cap_elems / 2);
     pool_free(p, s.d_inv);
-    s.cap_elems = std::max<uint64_t>(inv_elems, s.cap_elems + s.cap_elems / 2);
-    s.d_inv = pool_alloc<uint32_t>(p, s.cap_elems);
+    s.cap_elems = 0;
+    s.d_inv = pool_alloc<uint32_t>(p, cap);
+    s.cap_elems = cap;
   }
   if (s.cap_kill < kill_sets) {
+    const uint64_t cap = std::max<uint64_t>(kill_sets, s.cap_kill + s.cap_kill / 2);
     pool_free(p, s.d_kill);
-    s.cap_kill = std::max<uint64_t>(kill_sets, s.cap_kill + s.cap_kill / 2);
-    s.d_kill = pool_alloc<uint32_t>(p, s.cap_kill);
+    s.cap_kill = 0;
+    s.d_kill = pool_alloc<uint32_t>(p, cap);
+    s.cap_kill = cap;
   }
   if (s.cap_k < k) {
     pool_free(p, s.d_keys);
-    s.cap_k = k;
+    s.cap_k = 0;
     s.d_keys = pool_alloc<unsigned long long>(p, k);
+    s.cap_k = k;
   }
   if (s.cap_groups < p->groups) {
     pool_free(p, s.d_gactive);

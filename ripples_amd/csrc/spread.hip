@@ -436,6 +436,7 @@ void spread_run(rip_graph *g, const uint32_t *seeds, uint32_t nseeds, uint64_t s
   uint64_t wgs = std::max<uint64_t>(1, std::min<uint64_t>({count, 1024, budget / (per_wg * 4)}));
   if (g->fwd.per_wg != per_wg || g->fwd.wgs < wgs) {
     dev_free(g->fwd.d_scratch);
+    g->fwd.wgs = 0;   // until the new scratch is there
     g->fwd.d_scratch = dev_alloc<uint32_t>(wgs * per_wg);
     RIP_HIP(hipMemset(g->fwd.d_scratch, 0, sizeof(uint32_t) * wgs * per_wg));
     g->fwd.wgs = wgs;
