@@ -1030,15 +1030,15 @@ static void grid_ensure(rip_graph *g, uint32_t groups, uint64_t fcap, hipStream_
     s.d_fb = dev_alloc<unsigned long long>(fcap);
     s.fcap = fcap;
   }
-  if (!s.d_gctl) {
-    s.d_ring = dev_alloc<unsigned long long>(kRWords * kRing);
-    s.d_heavy = dev_alloc<unsigned long long>(2ull * kHeavyCap);
-    s.d_segs = dev_alloc<unsigned long long>(kSegCap);
-    s.d_gctl = dev_alloc<unsigned long long>(kGWords);
-    s.d_union = dev_alloc<unsigned long long>(256);
+  // (each by itself: an allocation that fails leaves the rest for the next call)
+  if (!s.d_ring) s.d_ring = dev_alloc<unsigned long long>(kRWords * kRing);
+  if (!s.d_heavy) s.d_heavy = dev_alloc<unsigned long long>(2ull * kHeavyCap);
+  if (!s.d_segs) s.d_segs = dev_alloc<unsigned long long>(kSegCap);
+  if (!s.d_gctl) s.d_gctl = dev_alloc<unsigned long long>(kGWords);
+  if (!s.d_union) s.d_union = dev_alloc<unsigned long long>(256);
+  if (!s.h_ctl)
     RIP_HIP(hipHostMalloc(reinterpret_cast<void **>(&s.h_ctl), sizeof(unsigned long long) * 256,
                           hipHostMallocDefault));
-  }
 }
 
 // Room for `words` 64-bit words of output tables.

@@ -1,164 +1,16 @@
 // Host check of what a failed device allocation leaves behind: the library on
-// a HIP runtime made here, whose device memory is host memory, whose kernels do
-// nothing, and whose allocations fail from the n-th of a call on.
+// a HIP runtime (fake_hip.h) whose allocations fail from the n-th of a call on.
 //
-// For every n: a small call, a larger one that fails, the small one again.  A
-// buffer whose capacity still claims room after the failure would not be
-// allocated by the last call, so there must be as many allocations alive as
-// after the small calls alone (idle blocks aside, which a failure frees).
-#include <cstdint>
-#include <cstdio>
-#include <cstdlib>
-#include <cstring>
+// For every n: a small call, a larger one that fails, the small one again; and
+// a small one that fails, then again.  A buffer whose capacity still claims
+// room after the failure would not be allocated by the last call, so there must
+// be as many allocations alive as after the small calls alone (idle blocks
+// aside, which a failure frees).
 #include <functional>
-#include <map>
-#include <set>
-#include <string>
 #include <vector>
 
+#include "fake_hip.h"
 #include "ripples_amd.h"
-
-namespace {
-
-struct Dim3 {
-  uint32_t x, y, z;
-};
-
-std::set<void *> &live() {
-  static std::set<void *> s;
-  return s;
-}
-
-std::map<const void *, std::string> &kernels() {   // host function -> kernel name
-  static std::map<const void *, std::string> m;
-  return m;
-}
-
-long g_fail_at = -1;   // allocations left before they fail; < 0: never
-bool g_failed = false;
-int g_null = 0;        // copies and fills of a null buffer
-
-struct {
-  Dim3 grid, block;
-  size_t lds;
-  void *stream;
-} g_call;
-
-}  // namespace
-
-extern "C" {
-void **__hipRegisterFatBinary(const void *) {
-  static void *module;
-  return &module;
-}
-void __hipUnregisterFatBinary(void **) {}
-void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
-void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *,
-                           void *, void *, void *, int *) {
-  kernels()[host] = name;
-}
-int __hipPushCallConfiguration(Dim3 grid, Dim3 block, size_t lds, void *stream) {
-  g_call = {grid, block, lds, stream};
-  return 0;
-}
-int __hipPopCallConfiguration(Dim3 *grid, Dim3 *block, size_t *lds, void **stream) {
-  *grid = g_call.grid;
-  *block = g_call.block;
-  *lds = g_call.lds;
-  *stream = g_call.stream;
-  return 0;
-}
-int hipLaunchKernel(const void *f, Dim3, Dim3, void **args, size_t, void *) {
-  // the selection's rounds: its state (the first pointer) says that every set
-  // is covered (word 10)
-  if (kernels()[f].find("top_rounds_kernel") != std::string::npos)
-    (**static_cast<uint32_t ***>(static_cast<void *>(args)))[10] = 1;
-  return 0;
-}
-int hipMalloc(void **p, size_t bytes) {
-  if (g_fail_at == 0) {
-    g_failed = true;
-    *p = nullptr;
-    return 2;
-  }
-  if (g_fail_at > 0) --g_fail_at;
-  *p = calloc(bytes, 1);
-  live().insert(*p);
-  return 0;
-}
-int hipFree(void *p) {
-  live().erase(p);
-  free(p);
-  return 0;
-}
-int hipHostMalloc(void **p, size_t bytes, unsigned) { return (*p = calloc(bytes, 1)) ? 0 : 2; }
-int hipHostFree(void *p) {
-  free(p);
-  return 0;
-}
-int hipMemcpy(void *d, const void *s, size_t n, int) {
-  if (d && s)
-    memcpy(d, s, n);
-  else if (n)
-    ++g_null;
-  return 0;
-}
-int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *) { return hipMemcpy(d, s, n, kind); }
-int hipMemset(void *p, int v, size_t n) {
-  if (p)
-    memset(p, v, n);
-  else if (n)
-    ++g_null;
-  return 0;
-}
-int hipMemsetAsync(void *p, int v, size_t n, void *) { return hipMemset(p, v, n); }
-int hipMemGetInfo(size_t *f, size_t *t) {
-  *f = *t = 64ull << 30;
-  return 0;
-}
-int hipDeviceTotalMem(size_t *t, int) {
-  *t = 64ull << 30;
-  return 0;
-}
-int hipDeviceGetAttribute(int *v, int, int) {
-  *v = 4;
-  return 0;
-}
-int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *v, const void *, int, size_t) {
-  *v = 2;
-  return 0;
-}
-int hipEventElapsedTime(float *ms, void *, void *) {
-  *ms = 0;
-  return 0;
-}
-static int handle(void **h) {
-  *h = malloc(1);
-  return 0;
-}
-int hipEventCreate(void **e) { return handle(e); }
-int hipStreamCreateWithFlags(void **s, unsigned) { return handle(s); }
-int hipStreamEndCapture(void *, void **g) { return handle(g); }
-int hipGraphInstantiate(void **x, void *, void *, char *, size_t) { return handle(x); }
-int hipEventDestroy(void *) { return 0; }
-int hipEventRecord(void *, void *) { return 0; }
-int hipStreamBeginCapture(void *, int) { return 0; }
-int hipStreamDestroy(void *) { return 0; }
-int hipStreamSynchronize(void *) { return 0; }
-int hipGraphDestroy(void *) { return 0; }
-int hipGraphExecDestroy(void *) { return 0; }
-int hipGraphLaunch(void *, void *) { return 0; }
-int hipFuncSetAttribute(const void *, int, int) { return 0; }
-int hipDeviceSynchronize() { return 0; }
-int hipSetDevice(int) { return 0; }
-int hipGetDevice(int *d) { return *d = 0; }
-int hipGetDeviceCount(int *n) {
-  *n = 1;
-  return 0;
-}
-int hipGetLastError() { return 0; }
-const char *hipGetErrorString(int) { return "out of memory"; }
-}
 
 namespace {
 
@@ -178,8 +30,9 @@ struct Case {
 };
 
 // Allocations alive after small, [large, failing from its n-th allocation on,]
-// small; n < 0: without the large call.
-size_t alive(const Case &c, long n, bool *failed) {
+// small; n < 0: without the large call; fresh: a small call in the place of
+// the first two.
+size_t alive(const Case &c, long n, bool fresh, bool *failed) {
   // in-neighbours v + 1 .. v + 4 of every v
   std::vector<uint64_t> index(c.n + 1);
   std::vector<uint32_t> edges;
@@ -196,11 +49,11 @@ size_t alive(const Case &c, long n, bool *failed) {
   require(rip_graph_create(0, c.model, c.n, edges.size(), index.data(), edges.data(), w.data(), &g) == 0, c.name);
   require(rip_pool_create(g, 1, &p) == 0, c.name);
   if (c.fill) c.fill(p);
-  require(c.call(g, p, false) == 0, c.name);
+  if (!fresh) require(c.call(g, p, false) == 0, c.name);
   if (n >= 0) {
     g_fail_at = n;
     g_failed = false;
-    const int rc = c.call(g, p, true);
+    const int rc = c.call(g, p, !fresh);
     g_fail_at = -1;
     require(rc == (g_failed ? RIP_ENOMEM : 0), c.name);
     *failed = g_failed;
@@ -240,10 +93,24 @@ int select(rip_pool *p, uint64_t sets, uint32_t k) {
   return rip_pool_select(p, sets, k, seeds.data(), &got, &covered);
 }
 
-int sample(rip_pool *p, bool large, uint32_t sampler) {
+int sample(rip_pool *p, bool large, uint32_t sampler, uint32_t colors = 0) {
   rip_tune t{};
   t.sampler = sampler;
+  t.colors = colors;
   return rip_pool_sample(p, large ? 60000 : 100, &t);
+}
+
+// The same when samples outgrow what the first kernels hold: the kernels that
+// clear the count of them (word 3 of the control words) leave that many.
+int sample_long(rip_pool *p, bool large, uint32_t sampler, uint32_t colors = 0) {
+  g_on_launch = [large](const std::string &kernel, Dim3, Dim3, size_t, void **args) {
+    for (const char *k : {"reset_lane_kernel", "reset_stage_kernel", "reset_wave_kernel", "reset_long_kernel"})
+      if (kernel.find(k) != std::string::npos)
+        (**static_cast<uint64_t ***>(static_cast<void *>(args)))[3] = large ? 40000 : 64;
+  };
+  const int rc = sample(p, large, sampler, colors);
+  g_on_launch = end_rounds;
+  return rc;
 }
 
 int spread(rip_graph *g, bool large) {
@@ -275,21 +142,27 @@ int main() {
       {"IC, waves", RIP_IC, 2000, nullptr, [](rip_graph *, rip_pool *p, bool l) { return sample(p, l, RIP_SAMPLER_WAVE); }},
       {"IC, lanes", RIP_IC, 2000, nullptr, [](rip_graph *, rip_pool *p, bool l) { return sample(p, l, RIP_SAMPLER_LANE); }},
       {"IC, colours", RIP_IC, 2000, nullptr, [](rip_graph *, rip_pool *p, bool l) { return sample(p, l, RIP_SAMPLER_COLOUR); }},
+      {"IC, grid", RIP_IC, 2000, nullptr, [](rip_graph *, rip_pool *p, bool l) { return sample_long(p, l, RIP_SAMPLER_AUTO, 64); }},
+      {"IC, teams", RIP_IC, 2000, nullptr, [](rip_graph *, rip_pool *p, bool l) { return sample_long(p, l, RIP_SAMPLER_AUTO); }},
+      {"IC, large by waves", RIP_IC, 2000, nullptr, [](rip_graph *, rip_pool *p, bool l) { return sample_long(p, l, RIP_SAMPLER_WAVE); }},
   };
   int bad = 0;   // calls left without a buffer
   for (const Case &c : cases) {
     bool failed = false;
-    const size_t want = alive(c, -1, &failed);
-    long n = 0;
-    for (failed = true; failed; ++n) {
-      const size_t got = alive(c, n, &failed);
-      if (failed && got < want) {
-        printf("%s: %zu allocations after a failure of number %ld, %zu without\n", c.name, got, n, want);
-        ++bad;
+    const size_t want = alive(c, -1, false, &failed);
+    for (const bool fresh : {false, true}) {
+      long n = 0;
+      for (failed = true; failed; ++n) {
+        const size_t got = alive(c, n, fresh, &failed);
+        if (failed && got < want) {
+          printf("%s: %zu allocations after a failure of number %ld%s, %zu without\n", c.name, got, n,
+                 fresh ? " of the first call" : "", want);
+          ++bad;
+        }
       }
+      printf("%s: %ld failures\n", c.name, n - 1);
+      if (n < 2) ++bad;   // the call must allocate
     }
-    printf("%s: %ld failures\n", c.name, n - 1);
-    if (n < 2) ++bad;   // the large call must allocate
   }
   if (g_null) printf("%d copies or fills of a null buffer\n", g_null);
   return bad != 0 || g_null != 0;
