@@ -770,19 +770,25 @@ uint32_t lt_finish_long(rip_pool *p, uint64_t first, uint64_t count, uint64_t nl
   const uint64_t per_lane = 4ull * g->n + 4ull * ((g->n + 31) / 32);
   const uint64_t lanes = std::max<uint64_t>(
       1, std::min<uint64_t>({nlong, 256, (static_cast<uint64_t>(1) << 29) / per_lane}));
-  uint32_t *lists = dev_alloc<uint32_t>(lanes * g->n);
-  uint32_t *bms = dev_alloc<uint32_t>(lanes * ((g->n + 31) / 32));
-  RIP_HIP(hipMemsetAsync(bms, 0, sizeof(uint32_t) * lanes * ((g->n + 31) / 32), p->stream));
+  uint32_t *lists = dev_alloc<uint32_t>(lanes * g->n), *bms = nullptr;
   uint32_t launches = 0;
-  for (uint64_t lo = 0; lo < nlong; lo += lanes) {
-    const uint32_t blocks_l = static_cast<uint32_t>((lanes + 63) / 64);
-    hipLaunchKernelGGL(lt_long_kernel, dim3(blocks_l), dim3(64), 0, p->stream, P,
-                       static_cast<uint32_t>(nlong), static_cast<uint32_t>(lo),
-                       static_cast<uint32_t>(lanes), lists, bms);
-    RIP_HIP(hipGetLastError());
-    ++launches;
+  try {
+    bms = dev_alloc<uint32_t>(lanes * ((g->n + 31) / 32));
+    RIP_HIP(hipMemsetAsync(bms, 0, sizeof(uint32_t) * lanes * ((g->n + 31) / 32), p->stream));
+    for (uint64_t lo = 0; lo < nlong; lo += lanes) {
+      const uint32_t blocks_l = static_cast<uint32_t>((lanes + 63) / 64);
+      hipLaunchKernelGGL(lt_long_kernel, dim3(blocks_l), dim3(64), 0, p->stream, P,
+                         static_cast<uint32_t>(nlong), static_cast<uint32_t>(lo),
+                         static_cast<uint32_t>(lanes), lists, bms);
+      RIP_HIP(hipGetLastError());
+      ++launches;
+    }
+    RIP_HIP(hipStreamSynchronize(p->stream));
+  } catch (...) {
+    dev_free(lists);
+    dev_free(bms);
+    throw;
   }
-  RIP_HIP(hipStreamSynchronize(p->stream));
   dev_free(lists);
   dev_free(bms);
   return launches;

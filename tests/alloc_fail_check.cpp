@@ -145,6 +145,7 @@ int main() {
       {"IC, grid", RIP_IC, 2000, nullptr, [](rip_graph *, rip_pool *p, bool l) { return sample_long(p, l, RIP_SAMPLER_AUTO, 64); }},
       {"IC, teams", RIP_IC, 2000, nullptr, [](rip_graph *, rip_pool *p, bool l) { return sample_long(p, l, RIP_SAMPLER_AUTO); }},
       {"IC, large by waves", RIP_IC, 2000, nullptr, [](rip_graph *, rip_pool *p, bool l) { return sample_long(p, l, RIP_SAMPLER_WAVE); }},
+      {"LT, long walks", RIP_LT, 2000, nullptr, [](rip_graph *, rip_pool *p, bool l) { return sample_long(p, l, 0); }},
   };
   int bad = 0;   // calls left without a buffer
   for (const Case &c : cases) {
