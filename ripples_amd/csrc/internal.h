@@ -132,6 +132,7 @@ struct WaveScratch {
 struct GridScratch {
   uint32_t groups = 0, n = 0;
   uint64_t fcap = 0;
+  bool searching = false;   // masks and bitmaps may be set (they are zero between calls)
   unsigned long long *d_vis = nullptr;  // groups x n pairs (visited, pending colours)
   uint32_t *d_bm0 = nullptr, *d_bm1 = nullptr;
   unsigned long long *d_z = nullptr;   // groups x 64

@@ -1000,7 +1000,7 @@ static void grid_plan(const rip_graph *g, uint64_t count, uint32_t colors, uint3
 static void grid_ensure(rip_graph *g, uint32_t groups, uint64_t fcap, hipStream_t st) {
   GridScratch &s = g->grid;
   const uint32_t n = g->n;
-  if (s.n != n || s.groups < groups) {
+  if (s.searching || s.n != n || s.groups < groups) {
     dev_free(s.d_vis);
     dev_free(s.d_bm0);
     dev_free(s.d_bm1);
@@ -1021,6 +1021,7 @@ static void grid_ensure(rip_graph *g, uint32_t groups, uint64_t fcap, hipStream_
     RIP_HIP(hipMemsetAsync(s.d_bm1, 0, 4ull * groups * nw1, st));
     s.groups = groups;
     s.n = n;
+    s.searching = false;
   }
   if (s.fcap < fcap) {
     dev_free(s.d_fa);
@@ -1080,6 +1081,7 @@ void grid_scratch_free(GridScratch &s) {
   s.groups = 0;
   s.fcap = 0;
   s.n = 0;
+  s.searching = false;
 }
 
 // Samples first + ids[i] (first + i without ids), i in [0, count), with the
@@ -1130,6 +1132,7 @@ uint32_t ic_grid_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
                                    kExpBT);
   const uint32_t exp_grid = static_cast<uint32_t>(per_cu * cu_count());
   uint32_t launches = 0;
+  s.searching = true;   // an error from here on leaves masks and bitmaps set
   for (uint64_t b0 = 0; b0 < count; b0 += static_cast<uint64_t>(C) * G) {
     const uint32_t Gb = static_cast<uint32_t>(std::min<uint64_t>(G, (count - b0 + C - 1) / C));
     hipLaunchKernelGGL(grid_samples_kernel, dim3((64 * Gb + 255) / 256), dim3(256), 0, st,
@@ -1287,6 +1290,7 @@ uint32_t ic_grid_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
     }
     launches += 1;
   }
+  s.searching = false;
   return launches;
 }
 

@@ -45,6 +45,7 @@ void end_rounds(const std::string &kernel, Dim3, Dim3, size_t, void **args) {
     (**static_cast<uint32_t ***>(static_cast<void *>(args)))[10] = 1;
 }
 std::function<void(const std::string &, Dim3, Dim3, size_t, void **)> g_on_launch = end_rounds;
+std::function<void(size_t)> g_on_fill = [](size_t) {};   // bytes of a fill of device memory
 
 }  // namespace
 
@@ -104,6 +105,7 @@ int hipMemcpy(void *d, const void *s, size_t n, int) {
 }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *) { return hipMemcpy(d, s, n, kind); }
 int hipMemset(void *p, int v, size_t n) {
+  g_on_fill(n);
   if (p)
     memset(p, v, n);
   else if (n)

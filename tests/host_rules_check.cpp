@@ -1,0 +1,90 @@
+// Host checks of what the library does around its kernels, on the HIP runtime
+// of fake_hip.h.  Each check has a name, given as the argument.
+#include <vector>
+
+#include "fake_hip.h"
+#include "ripples_amd.h"
+
+namespace {
+
+void require(bool ok, const char *what) {
+  if (ok) return;
+  printf("%s: %s\n", what, rip_last_error());
+  exit(1);
+}
+
+bool is(const std::string &kernel, const char *name) { return kernel.find(name) != std::string::npos; }
+
+// In-neighbours v + 1 .. v + 4 of every v.
+rip_graph *ring(int model, uint32_t n) {
+  std::vector<uint64_t> index(n + 1);
+  std::vector<uint32_t> edges;
+  for (uint32_t v = 0; v < n; ++v) {
+    for (uint32_t d = 1; d <= 4; ++d) edges.push_back((v + d) % n);
+    index[v + 1] = edges.size();
+  }
+  const std::vector<float> w(edges.size(), 0.2f);
+  rip_graph *g;
+  require(rip_graph_create(0, model, n, edges.size(), index.data(), edges.data(), w.data(), &g) == 0,
+          "graph");
+  return g;
+}
+
+// The count of samples that outgrew the lanes or waves (word 3 of the control
+// words), set where the kernels clear it.
+void set_long(const std::string &kernel, void **args, uint64_t count) {
+  for (const char *k : {"reset_lane_kernel", "reset_stage_kernel", "reset_wave_kernel"})
+    if (is(kernel, k)) (**static_cast<uint64_t ***>(static_cast<void *>(args)))[3] = count;
+}
+
+// A grid call that fails after its search began leaves colour masks and bitmaps
+// behind: the next call must clear them before its own search.
+void grid_scratch_after_failure() {
+  const uint32_t n = 4000;
+  rip_tune t{};
+  t.colors = 64;
+  bool cut = false;   // some call failed in that state
+  for (long at = 0;; ++at) {
+    rip_graph *g = ring(RIP_IC, n);
+    rip_pool *p;
+    require(rip_pool_create(g, 1, &p) == 0, "pool");
+    bool searched = false, cleared = true;
+    g_on_launch = [&](const std::string &kernel, Dim3, Dim3, size_t, void **args) {
+      set_long(kernel, args, 64);
+      if (!is(kernel, "grid_seed_kernel")) return;
+      searched = true;
+      if (!cleared) {
+        printf("failure %ld: the next call searched in what was left\n", at);
+        exit(1);
+      }
+    };
+    g_fail_at = at;
+    g_failed = false;
+    require(rip_pool_sample(p, 100, &t) == (g_failed ? RIP_ENOMEM : 0), "first call");
+    g_fail_at = -1;
+    if (g_failed && searched) {
+      cut = true;
+      cleared = false;
+      g_on_fill = [&](size_t bytes) { cleared = cleared || bytes >= 16ull * n; };
+      require(rip_pool_sample(p, 100, &t) == 0, "second call");
+      g_on_fill = [](size_t) {};
+    }
+    g_on_launch = end_rounds;
+    rip_pool_destroy(p);
+    rip_graph_destroy(g);
+    if (!g_failed) break;
+  }
+  require(cut, "no call failed after its search began");
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+  const std::map<std::string, void (*)()> checks = {
+      {"grid_scratch_after_failure", grid_scratch_after_failure},
+  };
+  const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
+  if (it == checks.end()) return 2;
+  it->second();
+  return 0;
+}
