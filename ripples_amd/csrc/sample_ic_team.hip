@@ -317,8 +317,10 @@ uint32_t ic_team_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
   uint32_t bt = lds <= (32u << 10) ? 256u : lds <= (64u << 10) ? 512u : 1024u;
   while (bt < 1024 && count * bt < static_cast<uint64_t>(cus) * 1024) bt *= 2;
   const void *kernel = team_kernel_ptr(bt);
+  // the limit belongs to the process: one value for every graph, as calls on
+  // others may be about to launch
   RIP_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(lds)));
+                              static_cast<int>(kTeamMaxNodes / 8)));
   const uint64_t resident = static_cast<uint64_t>(cus) *
                             team_blocks_per_cu(kernel, static_cast<int>(bt), lds);
   // a batch's rows take at most 1 GiB, and at least a group of samples

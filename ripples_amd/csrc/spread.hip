@@ -482,9 +482,11 @@ void spread_run(rip_graph *g, const uint32_t *seeds, uint32_t nseeds, uint64_t s
     const SpreadKernel kernel = bt == 1024   ? spread_kernel_of<1024>(g->model, lds)
                                 : bt == 512 ? spread_kernel_of<512>(g->model, lds)
                                             : spread_kernel_of<256>(g->model, lds);
+    // the limit belongs to the process: one value for every graph, as calls on
+    // others may be about to launch
     RIP_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(lds_bytes)));
+                                static_cast<int>(kSpreadLds)));
     hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(wgs)), dim3(bt), lds_bytes, 0, P);
     RIP_HIP(hipGetLastError());
     RIP_HIP(hipDeviceSynchronize());

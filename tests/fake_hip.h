@@ -45,6 +45,7 @@ void end_rounds(const std::string &kernel, Dim3, Dim3, size_t, void **args) {
     (**static_cast<uint32_t ***>(static_cast<void *>(args)))[10] = 1;
 }
 std::function<void(const std::string &, Dim3, Dim3, size_t, void **)> g_on_launch = end_rounds;
+std::function<void(const std::string &, int, int)> g_on_attribute = [](const std::string &, int, int) {};
 std::function<void(size_t)> g_on_fill = [](size_t) {};   // bytes of a fill of device memory
 
 }  // namespace
@@ -149,7 +150,10 @@ int hipStreamSynchronize(void *) { return 0; }
 int hipGraphDestroy(void *) { return 0; }
 int hipGraphExecDestroy(void *) { return 0; }
 int hipGraphLaunch(void *, void *) { return 0; }
-int hipFuncSetAttribute(const void *, int, int) { return 0; }
+int hipFuncSetAttribute(const void *f, int attribute, int value) {
+  g_on_attribute(kernels()[f], attribute, value);
+  return 0;
+}
 int hipDeviceSynchronize() { return 0; }
 int hipSetDevice(int) { return 0; }
 int hipGetDevice(int *d) { return *d = 0; }

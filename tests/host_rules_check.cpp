@@ -77,11 +77,52 @@ void grid_scratch_after_failure() {
   require(cut, "no call failed after its search began");
 }
 
+// A kernel's limit of dynamic LDS belongs to the process: a call on a small
+// graph must not lower what a call on a large one, in another thread, is about
+// to launch with.
+void lds_limit_is_kept() {
+  std::map<std::string, int> limit;
+  std::map<std::string, int> launched;
+  bool lowered = false;
+  g_on_attribute = [&](const std::string &kernel, int attribute, int value) {
+    if (attribute != 8) return;   // hipFuncAttributeMaxDynamicSharedMemorySize
+    lowered = lowered || value < limit[kernel];
+    limit[kernel] = value;
+  };
+  g_on_launch = [&](const std::string &kernel, Dim3, Dim3, size_t lds, void **args) {
+    set_long(kernel, args, 1);
+    if (lds == 0) return;
+    ++launched[kernel];
+    if (lds > static_cast<size_t>(limit[kernel])) require(false, kernel.c_str());
+  };
+  for (const uint32_t n : {400000u, 2000u}) {
+    for (const int model : {RIP_IC, RIP_LT}) {
+      rip_graph *g = ring(model, n);
+      const uint32_t seed = 3;
+      uint64_t act;
+      uint32_t lev;
+      require(rip_spread(g, &seed, 1, 1, 0, 1, &act, &lev) == 0, "spread");
+      if (model == RIP_IC) {
+        rip_pool *p;
+        require(rip_pool_create(g, 1, &p) == 0, "pool");
+        require(rip_pool_sample(p, 100, nullptr) == 0, "sample");
+        rip_pool_destroy(p);
+      }
+      rip_graph_destroy(g);
+    }
+  }
+  size_t both = 0;
+  for (const auto &k : launched) both += k.second == 2 ? 1 : 0;
+  require(both == 3, "the team and both spread kernels did not run on both graphs");
+  require(!lowered, "a limit was lowered");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> checks = {
       {"grid_scratch_after_failure", grid_scratch_after_failure},
+      {"lds_limit_is_kept", lds_limit_is_kept},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
