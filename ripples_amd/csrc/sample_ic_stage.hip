@@ -487,9 +487,18 @@ uint64_t ic_stage_launch(rip_pool *p, uint64_t first, uint64_t count, const uint
   const void *kernel = cap == kStageCap
                            ? reinterpret_cast<const void *>(&ic_stage_kernel<BT, kTab>)
                            : reinterpret_cast<const void *>(&ic_stage_kernel<BT, kTabTeam>);
-  const uint32_t blocks =
+  const uint32_t resident =
       std::min<uint32_t>(plain, static_cast<uint32_t>(blocks_per_cu(kernel, BT) * cu_count()));
-  const uint64_t waves = static_cast<uint64_t>(blocks) * (BT / 64);
+  uint64_t waves = static_cast<uint64_t>(resident) * (BT / 64);
+  const uint64_t wave_bytes = 12ull * kPack * cap;   // tables 8 cap, lists 4 cap a slot
+  if (w.stage_waves < waves) {
+    // fewer waves where the scratch would pass an eighth of the memory it may
+    // use (free plus what it already holds)
+    const uint64_t budget = (device_free_bytes() + w.stage_waves * wave_bytes) / 8;
+    const uint64_t fit = std::max<uint64_t>(1, budget / (wave_bytes * (BT / 64))) * (BT / 64);
+    waves = std::min(waves, std::max(fit, w.stage_waves));
+  }
+  const uint32_t blocks = static_cast<uint32_t>(waves / (BT / 64));
   if (w.stage_waves < waves) {
     dev_free(w.d_shtab);
     dev_free(w.d_slist);

@@ -323,11 +323,19 @@ uint32_t ic_team_launch(rip_pool *p, uint64_t first, uint64_t count, const uint3
                               static_cast<int>(kTeamMaxNodes / 8)));
   const uint64_t resident = static_cast<uint64_t>(cus) *
                             team_blocks_per_cu(kernel, static_cast<int>(bt), lds);
-  // a batch's rows take at most 1 GiB, and at least a group of samples
+  // a batch's rows take at most 1 GiB, and at least a group of samples; rows
+  // and queues stay within an eighth of the memory they may use (free plus what
+  // they already hold) when that is less
   const uint64_t row_bytes = 4ull * nw;
-  const uint64_t batch = std::min<uint64_t>(
+  uint64_t batch = std::min<uint64_t>(
       (count + 63) / 64 * 64, std::max<uint64_t>(64, (1ull << 30) / row_bytes / 64 * 64));
-  const uint64_t wgs = std::min<uint64_t>(resident, batch);
+  uint64_t wgs = std::min<uint64_t>(resident, batch);
+  if (s.queue_words < wgs * n || s.row_words < batch * nw) {
+    const uint64_t budget = (device_free_bytes() + 4 * (s.queue_words + s.row_words)) / 8;
+    batch = std::min(batch, std::max<uint64_t>({64, s.row_words / nw / 64 * 64,
+                                                budget / 2 / row_bytes / 64 * 64}));
+    wgs = std::min({wgs, batch, std::max<uint64_t>({1, s.queue_words / n, budget / 2 / (4ull * n)})});
+  }
   if (s.queue_words < wgs * n) {
     dev_free(s.d_queue);
     s.queue_words = 0;

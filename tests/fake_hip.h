@@ -31,6 +31,14 @@ std::map<const void *, std::string> &kernels() {   // host function -> kernel na
 long g_fail_at = -1;   // allocations left before they fail; < 0: never
 bool g_failed = false;
 int g_null = 0;        // copies and fills of a null buffer
+size_t g_memory = 64ull << 30;   // device memory there is
+int g_cus = 4;                   // compute units
+
+size_t used() {
+  size_t bytes = 0;
+  for (const auto &b : live()) bytes += b.second;
+  return bytes;
+}
 
 struct {
   Dim3 grid, block;
@@ -77,7 +85,7 @@ int hipLaunchKernel(const void *f, Dim3 grid, Dim3 block, void **args, size_t ld
   return 0;
 }
 int hipMalloc(void **p, size_t bytes) {
-  if (g_fail_at == 0) {
+  if (g_fail_at == 0 || used() + bytes > g_memory) {
     g_failed = true;
     *p = nullptr;
     return 2;
@@ -115,7 +123,8 @@ int hipMemset(void *p, int v, size_t n) {
 }
 int hipMemsetAsync(void *p, int v, size_t n, void *) { return hipMemset(p, v, n); }
 int hipMemGetInfo(size_t *f, size_t *t) {
-  *f = *t = 64ull << 30;
+  *f = g_memory - used();
+  *t = 64ull << 30;
   return 0;
 }
 int hipDeviceTotalMem(size_t *t, int) {
@@ -123,7 +132,7 @@ int hipDeviceTotalMem(size_t *t, int) {
   return 0;
 }
 int hipDeviceGetAttribute(int *v, int, int) {
-  *v = 4;
+  *v = g_cus;
   return 0;
 }
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *v, const void *, int, size_t) {

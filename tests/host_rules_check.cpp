@@ -117,12 +117,43 @@ void lds_limit_is_kept() {
   require(!lowered, "a limit was lowered");
 }
 
+// With little device memory left, samplers take less scratch, not an error.
+void scratch_fits_little_memory() {
+  g_cus = 256;
+  g_on_launch = [](const std::string &kernel, Dim3, Dim3, size_t, void **args) {
+    set_long(kernel, args, 300);
+  };
+  const struct {
+    const char *what;
+    uint32_t n;
+    uint64_t sets;
+    size_t left;   // bytes
+  } cases[] = {
+      {"wave stage and grid", (1u << 20) + 1, 1000, 160u << 20},
+      {"wave stage and teams", 1u << 20, 1000, 130u << 20},
+      {"lanes, wave stage and teams", 1u << 20, 5000, 260u << 20},
+  };
+  for (const auto &c : cases) {
+    rip_graph *g = ring(RIP_IC, c.n);
+    rip_pool *p;
+    require(rip_pool_create(g, 1, &p) == 0, "pool");
+    g_memory = used() + c.left;
+    require(rip_pool_sample(p, c.sets, nullptr) == 0, c.what);
+    require(rip_pool_sample(p, c.sets, nullptr) == 0, c.what);
+    g_memory = 64ull << 30;
+    require(rip_pool_sample(p, c.sets, nullptr) == 0, c.what);
+    rip_pool_destroy(p);
+    rip_graph_destroy(g);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> checks = {
       {"grid_scratch_after_failure", grid_scratch_after_failure},
       {"lds_limit_is_kept", lds_limit_is_kept},
+      {"scratch_fits_little_memory", scratch_fits_little_memory},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
