@@ -154,9 +154,11 @@ void *device_malloc(size_t bytes) {
     each_cache(dev, [](BlockCache *c) { c->release(); });
     e = hipMalloc(&p, bytes);
   }
-  if (e != hipSuccess)
+  if (e != hipSuccess) {
+    (void)hipGetLastError();   // or the next call's launch check finds it
     throw Error(-2, std::string("hipMalloc of ") + std::to_string(bytes) +
                         " bytes failed: " + hipGetErrorString(e));
+  }
   return p;
 }
 

@@ -132,11 +132,15 @@ struct Error : std::runtime_error {
 
 void set_last_error(const std::string &msg);
 
+// (The runtime keeps an error until it is asked for: one that is thrown must not
+// be found again by the launch check of a later call.)
 #define RIP_HIP(expr)                                                        \
   do {                                                                       \
     hipError_t _e = (expr);                                                  \
-    if (_e != hipSuccess)                                                    \
+    if (_e != hipSuccess) {                                                  \
+      (void)hipGetLastError();                                               \
       throw ::rip::Error(-3, std::string(#expr) + ": " + hipGetErrorString(_e)); \
+    }                                                                        \
   } while (0)
 
 #define RIP_REQUIRE(cond, code, msg)                                         \

@@ -33,6 +33,7 @@ bool g_failed = false;
 int g_null = 0;        // copies and fills of a null buffer
 size_t g_memory = 64ull << 30;   // device memory there is
 int g_cus = 4;                   // compute units
+int g_last = 0;                  // the error that hipGetLastError returns next
 
 size_t used() {
   size_t bytes = 0;
@@ -88,7 +89,7 @@ int hipMalloc(void **p, size_t bytes) {
   if (g_fail_at == 0 || used() + bytes > g_memory) {
     g_failed = true;
     *p = nullptr;
-    return 2;
+    return g_last = 2;
   }
   if (g_fail_at > 0) --g_fail_at;
   *p = calloc(bytes, 1);
@@ -170,6 +171,10 @@ int hipGetDeviceCount(int *n) {
   *n = 1;
   return 0;
 }
-int hipGetLastError() { return 0; }
+int hipGetLastError() {   // an error stays until it is asked for
+  const int e = g_last;
+  g_last = 0;
+  return e;
+}
 const char *hipGetErrorString(int) { return "out of memory"; }
 }
