@@ -680,21 +680,29 @@ void count_plain(rip_pool *p, uint64_t num_sets, uint64_t total, const uint8_t *
                      s.d_counts, static_cast<uint64_t>(n));
   if (num_sets == 0 || total == 0) return;
   const uint32_t buckets = (n + kBucketWidth - 1) >> kBucketBits;
-  if (total < kBucketMin || total >= (1ull << 32) - kSlice || buckets > kMaxBuckets) {
+  const uint32_t blocks = grid_for(num_sets, kCountBT, 1024);
+  bool deal = total >= kBucketMin && total < (1ull << 32) - kSlice && buckets <= kMaxBuckets;
+  if (deal) {
+    const uint64_t words = 3ull * (buckets + 1) + static_cast<uint64_t>(blocks) * buckets +
+                           (total + 1) / 2;
+    if (s.cap_part < words) {
+      pool_free(p, s.d_part);
+      s.cap_part = 0;
+      try {
+        s.d_part = pool_alloc<uint32_t>(p, words);
+        s.cap_part = words;
+      } catch (const Error &e) {
+        if (e.code != RIP_ENOMEM) throw;
+        deal = false;   // no room for the buckets: an atomic per member needs none
+      }
+    }
+  }
+  if (!deal) {
     hipLaunchKernelGGL(member_count_kernel, dim3(grid_for(num_sets, kCountBT, 4096)),
                        dim3(kCountBT), 0, st, p->d_off, p->d_len, p->d_data, num_sets, covered,
                        s.d_counts);
     RIP_HIP(hipGetLastError());
     return;
-  }
-  const uint32_t blocks = grid_for(num_sets, kCountBT, 1024);
-  const uint64_t words = 3ull * (buckets + 1) + static_cast<uint64_t>(blocks) * buckets +
-                         (total + 1) / 2;
-  if (s.cap_part < words) {
-    pool_free(p, s.d_part);
-    s.cap_part = 0;
-    s.d_part = pool_alloc<uint32_t>(p, words);
-    s.cap_part = words;
   }
   uint32_t *bcnt = s.d_part, *bstart = bcnt + buckets + 1, *sstart = bstart + buckets + 1;
   uint32_t *where = sstart + buckets + 1;

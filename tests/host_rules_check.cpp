@@ -147,6 +147,36 @@ void scratch_fits_little_memory() {
   }
 }
 
+// Counts need no scratch beside the counts themselves: they do not fail where
+// there is no room for the buckets.
+void counts_fit_little_memory() {
+  const uint32_t n = 1000, size = 10;
+  const uint64_t sets = 60000;
+  rip_graph *g = ring(RIP_IC, n);
+  rip_pool *p;
+  require(rip_pool_create(g, 1, &p) == 0, "pool");
+  std::vector<uint64_t> off(1, 0);
+  std::vector<uint32_t> ver, counts(n);
+  for (uint64_t s = 0; s < sets; ++s) {
+    for (uint32_t i = 0; i < size; ++i) ver.push_back(s % (n - size) + i);
+    off.push_back(ver.size());
+  }
+  require(rip_pool_append_host(p, sets, off.data(), ver.data()) == 0, "append");
+  bool buckets = false, members = false;
+  g_on_launch = [&](const std::string &kernel, Dim3, Dim3, size_t, void **) {
+    buckets = buckets || is(kernel, "bucket_count_kernel");
+    members = members || is(kernel, "member_count_kernel");
+  };
+  g_memory = used() + (1u << 20);
+  require(rip_pool_count(p, sets, counts.data()) == 0, "counts");
+  require(members && !buckets, "not counted member by member");
+  g_memory = 64ull << 30;
+  require(rip_pool_count(p, sets, counts.data()) == 0, "counts");
+  require(buckets, "not counted by bucket");
+  rip_pool_destroy(p);
+  rip_graph_destroy(g);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -154,6 +184,7 @@ int main(int argc, char **argv) {
       {"grid_scratch_after_failure", grid_scratch_after_failure},
       {"lds_limit_is_kept", lds_limit_is_kept},
       {"scratch_fits_little_memory", scratch_fits_little_memory},
+      {"counts_fit_little_memory", counts_fit_little_memory},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;

@@ -25,6 +25,7 @@ def exe(tmp_path_factory):
     "grid_scratch_after_failure",
     "lds_limit_is_kept",
     "scratch_fits_little_memory",
+    "counts_fit_little_memory",
 ])
 def test_host_rules(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=300)
