@@ -177,6 +177,59 @@ void counts_fit_little_memory() {
   rip_graph_destroy(g);
 }
 
+// A pool of `sets` sets of `size` vertices each, from a moving start.
+rip_pool *runs(rip_graph *g, uint32_t n, uint64_t sets, uint32_t size) {
+  rip_pool *p;
+  require(rip_pool_create(g, 1, &p) == 0, "pool");
+  std::vector<uint64_t> off(1, 0);
+  std::vector<uint32_t> ver;
+  for (uint64_t s = 0; s < sets; ++s) {
+    for (uint32_t i = 0; i < size; ++i) ver.push_back(s * 7 % (n - size) + i);
+    off.push_back(ver.size());
+  }
+  require(rip_pool_append_host(p, sets, off.data(), ver.data()) == 0, "append");
+  return p;
+}
+
+int select(rip_pool *p, uint64_t sets, uint32_t k) {
+  std::vector<uint32_t> seeds(k);
+  uint32_t got;
+  uint64_t covered;
+  return rip_pool_select(p, sets, k, seeds.data(), &got, &covered);
+}
+
+// A few long sets are walked by as many workgroups as their members fill, as
+// many short ones are.
+void long_sets_fill_the_chip() {
+  rip_graph *g = ring(RIP_IC, 100000);
+  const struct {
+    uint64_t sets;
+    uint32_t size;
+    uint32_t least, most;   // workgroups
+  } cases[] = {{800, 1000, 100, 1024}, {100, 5000, 13, 1024}, {20, 10, 1, 3}, {60000, 10, 100, 1024}};
+  for (const auto &c : cases) {
+    rip_pool *p = runs(g, 100000, c.sets, c.size);
+    int walks = 0;
+    g_on_launch = [&](const std::string &kernel, Dim3 grid, Dim3 block, size_t lds, void **args) {
+      end_rounds(kernel, grid, block, lds, args);
+      for (const char *k : {"bucket_size", "bucket_deal", "member_count", "top_index"})
+        if (is(kernel, k)) {
+          ++walks;
+          if (grid.x < c.least || grid.x > c.most) {
+            printf("%s: %u workgroups for %llu sets of %u\n", kernel.c_str(), grid.x,
+                   static_cast<unsigned long long>(c.sets), c.size);
+            exit(1);
+          }
+        }
+    };
+    require(select(p, c.sets, 3) == 0, "select");
+    require(walks >= 2, "no counts or index");
+    g_on_launch = end_rounds;
+    rip_pool_destroy(p);
+  }
+  rip_graph_destroy(g);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -185,6 +238,7 @@ int main(int argc, char **argv) {
       {"lds_limit_is_kept", lds_limit_is_kept},
       {"scratch_fits_little_memory", scratch_fits_little_memory},
       {"counts_fit_little_memory", counts_fit_little_memory},
+      {"long_sets_fill_the_chip", long_sets_fill_the_chip},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
