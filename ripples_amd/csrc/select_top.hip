@@ -58,7 +58,8 @@ constexpr uint32_t kCountBT = 512;
 constexpr uint64_t kFullBlocks = 512;
 inline uint32_t wave_sets(uint64_t num_sets, uint64_t total) {
   uint32_t step = 64;
-  while (step > 1 && num_sets < kFullBlocks * (kCountBT / 64) * step && total * step > 512 * num_sets)
+  while (step > 1 && num_sets < kFullBlocks * (kCountBT / 64) * step &&
+         total * step > 512 * num_sets)
     step /= 2;
   return step;
 }
@@ -74,8 +75,8 @@ template <int BT, typename F>
 __device__ inline void for_block_members(const unsigned long long *set_off,
                                          const uint32_t *set_len, const uint32_t *data,
                                          uint64_t num_sets, uint32_t step,
-                                         const uint8_t *covered, uint32_t (*s_pre)[65], unsigned long long (*s_off)[64],
-                                         F &&f) {
+                                         const uint8_t *covered, uint32_t (*s_pre)[65],
+                                         unsigned long long (*s_off)[64], F &&f) {
   const uint32_t lane = lane_id(), wid = threadIdx.x >> 6;
   const uint64_t per = share_of(num_sets, gridDim.x, step);
   const uint64_t sb = blockIdx.x * per;
@@ -535,6 +536,7 @@ struct TopRounds {
   SetRec *rec;
   const uint16_t *members;
   uint8_t *covered;
+  uint64_t num_sets;
   uint32_t *picked;           // per round its candidate: the rank, once its launch ends the vertex
 };
 
@@ -595,6 +597,12 @@ __device__ inline void kill_sets(const TopRounds &R, uint32_t p, uint32_t stride
 // costs about as much as one such turn (lines of 2,048 and 4,096 measured
 // alike, 8,192 and 16,384 slower: 12 served queries 66, 66, 78 and 83 ms).
 constexpr uint32_t kWideList = 4096;
+// That line is for sets of a few candidates each (two on R-MAT scale 22 under
+// weighted cascade).  Where they hold more it lies at this many together: one
+// workgroup takes some 120 us for 4,095 sets of 150 candidates, whose LDS
+// decrements meet on a few counters (10,000 sets of 205 under U[0,0.1] on 4096
+// vertices, k = 10: 1.82 ms by sets alone, 0.91 with this line).
+constexpr uint32_t kWideMembers = 8 * kWideList;
 constexpr uint32_t kWideBlocks = 64;
 constexpr uint32_t kRoundLaunches = 16;
 constexpr uint32_t kRoundBT = 1024;
@@ -637,7 +645,12 @@ __global__ void __launch_bounds__(kRoundBT) top_rounds_kernel(TopRounds R, uint3
     cnt[c] = load_u32(&R.cnt[c]);
     start[c] = R.cstart[c];
   }
-  if (tid == 0) start[nc] = R.cstart[nc];
+  const uint32_t held = R.cstart[nc];     // the sets' candidates together
+  if (tid == 0) start[nc] = held;
+  const uint64_t each = held / R.num_sets;
+  const uint32_t wide = each <= kWideMembers / kWideList
+                            ? kWideList
+                            : max(64u, static_cast<uint32_t>(kWideMembers / each));
   uint32_t stop = kStopNone, rank = 0, gain = 0;
   for (;;) {
     __syncthreads();
@@ -663,7 +676,7 @@ __global__ void __launch_bounds__(kRoundBT) top_rounds_kernel(TopRounds R, uint3
       break;
     }
     const uint32_t b = start[rank], e = start[rank + 1];
-    if (e - b >= kWideList && !all) break;             // for the next launch
+    if (e - b >= wide && !all) break;             // for the next launch
     for (uint32_t p = b + tid; p < e; p += 4 * kRoundBT)
       kill_sets<4>(R, p, kRoundBT, e, [&](uint32_t m) { atomicSub(&cnt[m], 1u); });
     if (tid == 0) R.picked[i] = rank;
@@ -777,7 +790,8 @@ uint32_t select_top(rip_pool *p, uint64_t num_sets, uint64_t total, uint32_t k, 
   uint32_t *ccur = cstart + kTopMax + 1, *tiles = ccur + kTopMax + 1;
   unsigned long long *is_cand = reinterpret_cast<unsigned long long *>(s.d_rank + 4 * ((n + 3ull) / 4));
   const TopRounds R{ts, cand, cnt, cstart, s.d_inv, reinterpret_cast<SetRec *>(s.d_rec),
-                    s.d_members, s.d_covered, reinterpret_cast<uint32_t *>(s.d_keys)};
+                    s.d_members, s.d_covered, std::max<uint64_t>(num_sets, 1),
+                    reinterpret_cast<uint32_t *>(s.d_keys)};
   const uint32_t step = wave_sets(num_sets, total);
   uint32_t got = 0, restarts = 0;
   uint64_t cov = 0;
@@ -796,13 +810,13 @@ uint32_t select_top(rip_pool *p, uint64_t num_sets, uint64_t total, uint32_t k, 
     hipLaunchKernelGGL(top_pick_kernel, dim3(vgrid), dim3(kPickBT), 0, st, s.d_counts, n, ts, tiles,
                        ntiles, cand, cnt, s.d_rank, is_cand, cstart, ccur);
     hipLaunchKernelGGL(top_index_kernel, dim3(grid_for(num_sets, step * (kCountBT / 64), 1024)),
-                       dim3(kCountBT), 0, st, p->d_off, p->d_len, p->d_data, num_sets, step, cflags, s.d_rank, is_cand,
-                       ts, ccur, s.d_inv, R.rec, s.d_members);
+                       dim3(kCountBT), 0, st, p->d_off, p->d_len, p->d_data, num_sets, step, cflags,
+                       s.d_rank, is_cand, ts, ccur, s.d_inv, R.rec, s.d_members);
     // launches until the rounds are done: one when no list can be long, else
     // a few between looks at the state (one with no long round pending ends
     // the selection or costs its launch only)
     uint32_t w[kTopWords];
-    const bool all = num_sets < kWideList;
+    const bool all = num_sets < kWideList && total < 4 * kWideMembers;
     hipLaunchKernelGGL(top_rounds_kernel, dim3(1), dim3(kRoundBT), 0, st, R, left, all ? 1u : 0u);
     do {
       for (uint32_t i = 0; i < (all ? 0u : kRoundLaunches); ++i)

@@ -47,11 +47,19 @@ struct {
   void *stream;
 } g_call;
 
-// A kernel launch and its arguments; the default ends the selection's rounds:
-// their state (the first pointer) says that every set is covered (word 10).
+// Ends a pass of the selection's rounds: their state (the first pointer of
+// top_rounds_kernel) gets the rounds done (word 8), the sets they cover (9) and
+// why they ended (10; 1: every set is covered, 2: the candidates ran out).
+void set_rounds(void **args, uint32_t rounds, uint32_t covered, uint32_t why) {
+  uint32_t *state = **static_cast<uint32_t ***>(static_cast<void *>(args));
+  state[8] = rounds;
+  state[9] = covered;
+  state[10] = why;
+}
+
+// A kernel launch and its arguments; the default covers every set at once.
 void end_rounds(const std::string &kernel, Dim3, Dim3, size_t, void **args) {
-  if (kernel.find("top_rounds_kernel") != std::string::npos)
-    (**static_cast<uint32_t ***>(static_cast<void *>(args)))[10] = 1;
+  if (kernel.find("top_rounds_kernel") != std::string::npos) set_rounds(args, 0, 0, 1);
 }
 std::function<void(const std::string &, Dim3, Dim3, size_t, void **)> g_on_launch = end_rounds;
 std::function<void(const std::string &, int, int)> g_on_attribute = [](const std::string &, int, int) {};

@@ -230,6 +230,30 @@ void long_sets_fill_the_chip() {
   rip_graph_destroy(g);
 }
 
+// Rounds whose list holds many members together run on the whole chip, also
+// where the pool has few sets; pools of short sets stay with one workgroup.
+void long_lists_go_wide() {
+  rip_graph *g = ring(RIP_IC, 100000);
+  const struct {
+    uint64_t sets;
+    uint32_t size;
+    bool wide;
+  } cases[] = {{1000, 300, true}, {1000, 20, false}, {4000, 20, false}, {5000, 20, true}};
+  for (const auto &c : cases) {
+    rip_pool *p = runs(g, 100000, c.sets, c.size);
+    int wide = 0;
+    g_on_launch = [&](const std::string &kernel, Dim3 grid, Dim3 block, size_t lds, void **args) {
+      end_rounds(kernel, grid, block, lds, args);
+      if (is(kernel, "top_rounds") && grid.x > 1) ++wide;
+    };
+    require(select(p, c.sets, 3) == 0, "select");
+    require((wide != 0) == c.wide, c.wide ? "one workgroup for long lists" : "wide rounds for short lists");
+    g_on_launch = end_rounds;
+    rip_pool_destroy(p);
+  }
+  rip_graph_destroy(g);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -239,6 +263,7 @@ int main(int argc, char **argv) {
       {"scratch_fits_little_memory", scratch_fits_little_memory},
       {"counts_fit_little_memory", counts_fit_little_memory},
       {"long_sets_fill_the_chip", long_sets_fill_the_chip},
+      {"long_lists_go_wide", long_lists_go_wide},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;

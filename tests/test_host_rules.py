@@ -27,6 +27,7 @@ def exe(tmp_path_factory):
     "scratch_fits_little_memory",
     "counts_fit_little_memory",
     "long_sets_fill_the_chip",
+    "long_lists_go_wide",
 ])
 def test_host_rules(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=300)
