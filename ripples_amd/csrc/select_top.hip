@@ -696,6 +696,17 @@ __global__ void __launch_bounds__(kRoundBT) top_rounds_kernel(TopRounds R, uint3
 
 }  // namespace
 
+// When the candidates run out (the best falls below the bound) another pass over
+// the pool finds new ones; after this many passes in a row of fewer rounds than
+// this the full index takes over.  A pass costs 0.1 to 1 ms, a round of the full
+// index some 8 us more than one among candidates.  R-MAT pools of 0.6 to 19M
+// members under cascade and LT yield 17 to 200 rounds in the first pass and 140
+// to 1000 in each later one, two or three passes for k = 1000 and up to eleven
+// for k = 5000; one of large sets (U[0,0.1], 10,000 sets of 205 on 4096 vertices)
+// 1 in the first and 900 in the next.  Forty cliques of 1100 vertices, each
+// vertex of a clique in all its sets (0.9M members, k = 10), yield one a pass.
+constexpr uint32_t kPoorRounds = 16, kPoorPasses = 2;
+
 // counts[v] (cleared first) = sets of [0, num_sets) holding v, covered ones
 // (covered != nullptr) left out; total: at least the members there are.
 void count_plain(rip_pool *p, uint64_t num_sets, uint64_t total, const uint8_t *covered) {
@@ -793,7 +804,7 @@ uint32_t select_top(rip_pool *p, uint64_t num_sets, uint64_t total, uint32_t k, 
                     s.d_members, s.d_covered, std::max<uint64_t>(num_sets, 1),
                     reinterpret_cast<uint32_t *>(s.d_keys)};
   const uint32_t step = wave_sets(num_sets, total);
-  uint32_t got = 0, restarts = 0;
+  uint32_t got = 0, restarts = 0, poor = 0;
   uint64_t cov = 0;
   std::vector<uint32_t> picked(k);
   *finished = false;
@@ -834,10 +845,11 @@ uint32_t select_top(rip_pool *p, uint64_t num_sets, uint64_t total, uint32_t k, 
       *finished = true;
       break;
     }
-    // a pass over the pool per restart: a few are normal (they also drop the
-    // covered sets from the lists), many mean that the candidates share their
-    // sets, and the full index is the better form
-    if (++restarts > 8 + k / 256 || w[kTopRound] == 0) break;
+    // passes over the pool that yield few rounds and leave most sets there: the
+    // candidates share their sets, and the full index is the better form
+    const uint64_t before = num_sets - (cov - w[kTopCovered]);
+    poor = w[kTopRound] < kPoorRounds && 2ull * w[kTopCovered] < before ? poor + 1 : 0;
+    if (poor == kPoorPasses || ++restarts > 8 + k / 256 || w[kTopRound] == 0) break;
   }
   *covered = cov;
   return got;

@@ -254,6 +254,35 @@ void long_lists_go_wide() {
   rip_graph_destroy(g);
 }
 
+// A selection whose passes yield a round or two and leave most sets there turns
+// to the full index after two of them; one whose passes yield more goes on.
+void poor_passes_end() {
+  const uint32_t n = 100000;
+  rip_graph *g = ring(RIP_IC, n);
+  const struct {
+    uint32_t rounds, covered;
+    int least, most;   // passes
+  } cases[] = {{1, 5, 2, 2}, {15, 150, 2, 2}, {20, 100, 8, 12}, {1, 600, 3, 12}};
+  for (const auto &c : cases) {
+    rip_pool *p = runs(g, n, 1000, 20);
+    int passes = 0;
+    bool full = false;
+    g_on_launch = [&](const std::string &kernel, Dim3, Dim3, size_t, void **args) {
+      if (is(kernel, "top_rounds")) set_rounds(args, c.rounds, c.covered, 2);
+      if (is(kernel, "top_index")) ++passes;
+      full = full || is(kernel, "fill_inverted");
+    };
+    require(select(p, 1000, 500) == 0, "select");
+    if (passes < c.least || passes > c.most || !full) {
+      printf("%d passes of %u rounds, full index: %d\n", passes, c.rounds, full);
+      exit(1);
+    }
+    g_on_launch = end_rounds;
+    rip_pool_destroy(p);
+  }
+  rip_graph_destroy(g);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -264,6 +293,7 @@ int main(int argc, char **argv) {
       {"counts_fit_little_memory", counts_fit_little_memory},
       {"long_sets_fill_the_chip", long_sets_fill_the_chip},
       {"long_lists_go_wide", long_lists_go_wide},
+      {"poor_passes_end", poor_passes_end},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;

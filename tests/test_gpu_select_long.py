@@ -15,6 +15,11 @@ def drawn(n, count, low, high, power, seed):
                for _ in range(count)]
 
 
+def cliques(n, count, size, copies):
+    """Vertices that share all their sets: a pass over the pool yields one round."""
+    return n, [np.arange(c * size, (c + 1) * size) for c in range(count) for _ in range(copies - c)]
+
+
 # below and above 4 x 32,768 members and 4,096 sets; lists either side of the
 # line, which lies at 32,768 members
 POOLS = {
@@ -23,6 +28,7 @@ POOLS = {
     "even": lambda: drawn(3000, 3000, 200, 400, 1, 3),
     "many": lambda: drawn(1500, 6000, 100, 300, 2, 4),
     "most": lambda: drawn(400, 5000, 300, 900, 1, 5),
+    "cliques": lambda: cliques(60000, 20, 1100, 60),
     "one": lambda: (70000, [np.arange(0, 70000, 2)]),
 }
 

@@ -28,6 +28,7 @@ def exe(tmp_path_factory):
     "counts_fit_little_memory",
     "long_sets_fill_the_chip",
     "long_lists_go_wide",
+    "poor_passes_end",
 ])
 def test_host_rules(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=300)
