@@ -1,5 +1,8 @@
-"""Selection of plain pools of long sets, whose rounds turn to the whole GPU by
-the members of a list and not by its sets, against the oracle."""
+"""Selection of plain pools of long sets against the oracle: rounds that turn to
+the whole GPU by the members of a list and not by its sets, and pools of more than
+2^23 members that end in the full index sorted by vertex."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -33,19 +36,50 @@ POOLS = {
 }
 
 
-@pytest.mark.parametrize("name", sorted(POOLS))
-def test_long_sets_match_oracle(name, orc):
-    n, sets = POOLS[name]()
+def filled(n, sets):
     off = np.zeros(len(sets) + 1, np.uint64)
     off[1:] = np.cumsum([len(s) for s in sets])
     ver = np.concatenate(sets).astype(np.uint32)
     g = R.Graph(np.zeros(n + 1, np.uint64), np.zeros(0, np.uint32), np.zeros(0, np.float32))
     p = g.pool(0)
     p.append(off, ver)
+    return off, ver, g, p
+
+
+def device_free():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL("libamdhip64.so").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("name", sorted(POOLS))
+def test_long_sets_match_oracle(name, orc):
+    n, sets = POOLS[name]()
+    off, ver, g, p = filled(n, sets)
     assert np.array_equal(p.count_occurrences(), orc.count(n, off, ver))
     for k in (1, 12, 150):
         seeds, cov = p.find_most_influential_set(k)
         es, ec = orc.select(n, off, ver, k)
         assert seeds.tolist() == es.tolist() and cov == ec
+    p.close()
+    g.close()
+
+
+# the search among candidates gives up after two seeds, and before the first
+# (more vertices of the largest count than it takes, that count past 127)
+@pytest.mark.parametrize("pool", [(1100000, 20, 4000, 120), (400000, 14, 1100, 560)])
+def test_sorted_index_matches_oracle(pool, orc):
+    n, sets = cliques(*pool)
+    off, ver, g, p = filled(n, sets)
+    total = int(off[-1])
+    assert total >= 1 << 23
+    before = device_free()
+    for k in (1, 2, 3, 40):
+        seeds, cov = p.find_most_influential_set(k)
+        es, ec = orc.select(n, off, ver, k)
+        assert seeds.tolist() == es.tolist() and cov == ec
+    # lists (4 bytes a member), buckets and candidates (2 each), and the pairs
+    # of the sort: 12 more
+    assert before - device_free() > 16 * total
     p.close()
     g.close()
