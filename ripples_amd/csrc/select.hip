@@ -817,24 +817,14 @@ bool build_counts(rip_pool *p, uint64_t num_sets, uint32_t k, Need need, uint64_
   return true;
 }
 
-// Captures clear + k seed rounds on the pool's stream as an executable graph:
-// (argmax, kill) per round, or for dense pools (argmax, scan, two decrement
-// kernels of which one does the work).  Only kernels are recorded (no memset
-// nodes); the capture mode is thread-local so other host threads' streams
-// are unaffected.
-void capture_rounds(rip_pool *p, uint32_t k, bool dense, bool cols) {
+// Clear + k seed rounds on the pool's stream.
+void launch_rounds(rip_pool *p, uint32_t k, bool dense, bool cols) {
   SelectScratch &s = p->sel;
-  if (s.graph) {
-    (void)hipGraphExecDestroy(s.graph);
-    s.graph = nullptr;
-    s.graph_k = 0;
-  }
   hipStream_t st = p->stream;
   const uint32_t n = p->g->n;
   const uint32_t argmax_grid = grid_for(n, kBT * 8, kArgmaxBlocks);
   const uint32_t ranges = ranges_of(n);
   const uint32_t dec_grid = ranges * dense_chunks(ranges, ~0ull);
-  RIP_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
   hipLaunchKernelGGL(clear_keys_kernel, dim3(1), dim3(256), 0, st, s.d_args, k);
   for (uint32_t i = 0; i < k; ++i) {
     hipLaunchKernelGGL(argmax_kernel, dim3(argmax_grid), dim3(kBT), 0, st, s.d_args);
@@ -853,6 +843,28 @@ void capture_rounds(rip_pool *p, uint32_t k, bool dense, bool cols) {
       hipLaunchKernelGGL(kill_kernel, dim3(256), dim3(kBT), 0, st, s.d_args, i, argmax_grid);
     }
   }
+}
+
+// Rounds of one graph at most.  Capturing or launching 100,000 rounds (200,000
+// nodes in a chain) ended the process inside the runtime, 20,000 did not; more
+// rounds than this (up to 24,577 nodes) are launched one by one.
+constexpr uint32_t kGraphRounds = 4096;
+
+// Captures clear + k seed rounds on the pool's stream as an executable graph:
+// (argmax, kill) per round, or for dense pools (argmax, scan, two decrement
+// kernels of which one does the work).  Only kernels are recorded (no memset
+// nodes); the capture mode is thread-local so other host threads' streams
+// are unaffected.
+void capture_rounds(rip_pool *p, uint32_t k, bool dense, bool cols) {
+  SelectScratch &s = p->sel;
+  if (s.graph) {
+    (void)hipGraphExecDestroy(s.graph);
+    s.graph = nullptr;
+    s.graph_k = 0;
+  }
+  hipStream_t st = p->stream;
+  RIP_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+  launch_rounds(p, k, dense, cols);
   const hipError_t launch = hipGetLastError();
   hipGraph_t graph = nullptr;
   const hipError_t end = hipStreamEndCapture(st, &graph);
@@ -915,8 +927,9 @@ uint32_t select_run(rip_pool *p, uint64_t num_sets, uint32_t k_total, uint32_t *
     count_plain(p, num_sets, total, done ? s.d_covered : nullptr);
   }
   const uint32_t k = k_total - done;
-  // the seed rounds run as one graph; this call's buffers travel in d_args
-  // (`args` stays alive until the stream is synchronised below)
+  // the seed rounds run as one graph where they are not too many; this call's
+  // buffers travel in d_args (`args` stays alive until the stream is
+  // synchronised below)
   const bool cols = p->groups > 0;
   const Args args{s.d_counts, s.d_inv_start, inv, p->d_off,
                   p->d_len, p->d_data,
@@ -924,12 +937,12 @@ uint32_t select_run(rip_pool *p, uint64_t num_sets, uint32_t k_total, uint32_t *
                   p->d_gref, p->d_colptr, p->g->d_hot_index, p->g->d_hot_vertex, s.d_gkill,
                   s.d_kgroups, cols ? p->groups : 0u, p->g->hot_n};
   RIP_HIP(hipMemcpyAsync(s.d_args, &args, sizeof(Args), hipMemcpyHostToDevice, st));
-  if (k) {
+  if (k && k <= kGraphRounds) {
     if (!s.graph || s.graph_k != k || s.graph_dense != dense || s.graph_cols != cols)
       capture_rounds(p, k, dense, cols);
     RIP_HIP(hipGraphLaunch(s.graph, st));
   } else {
-    hipLaunchKernelGGL(clear_keys_kernel, dim3(1), dim3(256), 0, st, s.d_args, 0u);
+    launch_rounds(p, k, dense, cols);
   }
   RIP_HIP(hipGetLastError());
   std::vector<unsigned long long> keys(std::max<uint32_t>(k, 1));

@@ -62,6 +62,8 @@ void end_rounds(const std::string &kernel, Dim3, Dim3, size_t, void **args) {
   if (kernel.find("top_rounds_kernel") != std::string::npos) set_rounds(args, 0, 0, 1);
 }
 std::function<void(const std::string &, Dim3, Dim3, size_t, void **)> g_on_launch = end_rounds;
+int g_captured = -1;             // launches of the capture under way; < 0: none
+int g_largest_graph = 0;         // launches of the largest capture
 std::function<void(const std::string &, int, int)> g_on_attribute = [](const std::string &, int, int) {};
 std::function<void(size_t)> g_on_fill = [](size_t) {};   // bytes of a fill of device memory
 
@@ -90,6 +92,7 @@ int __hipPopCallConfiguration(Dim3 *grid, Dim3 *block, size_t *lds, void **strea
   return 0;
 }
 int hipLaunchKernel(const void *f, Dim3 grid, Dim3 block, void **args, size_t lds, void *) {
+  if (g_captured >= 0) ++g_captured;
   g_on_launch(kernels()[f], grid, block, lds, args);
   return 0;
 }
@@ -158,11 +161,15 @@ static int handle(void **h) {
 }
 int hipEventCreate(void **e) { return handle(e); }
 int hipStreamCreateWithFlags(void **s, unsigned) { return handle(s); }
-int hipStreamEndCapture(void *, void **g) { return handle(g); }
+int hipStreamEndCapture(void *, void **g) {
+  if (g_captured > g_largest_graph) g_largest_graph = g_captured;
+  g_captured = -1;
+  return handle(g);
+}
 int hipGraphInstantiate(void **x, void *, void *, char *, size_t) { return handle(x); }
 int hipEventDestroy(void *) { return 0; }
 int hipEventRecord(void *, void *) { return 0; }
-int hipStreamBeginCapture(void *, int) { return 0; }
+int hipStreamBeginCapture(void *, int) { return g_captured = 0; }
 int hipStreamDestroy(void *) { return 0; }
 int hipStreamSynchronize(void *) { return 0; }
 int hipGraphDestroy(void *) { return 0; }

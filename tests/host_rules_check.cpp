@@ -283,6 +283,31 @@ void poor_passes_end() {
   rip_graph_destroy(g);
 }
 
+// However many seeds are asked for, no graph holds more than some 25,000 nodes.
+void graphs_stay_bounded() {
+  rip_graph *g = ring(RIP_IC, 20000);
+  rip_pool *plain = runs(g, 20000, 1000, 20), *dense = runs(g, 20000, 500, 10000);
+  int argmax = 0;
+  g_on_launch = [&](const std::string &kernel, Dim3, Dim3, size_t, void **args) {
+    if (is(kernel, "top_rounds")) set_rounds(args, 0, 0, 2);   // no round among candidates
+    if (is(kernel, "argmax_kernel")) ++argmax;
+  };
+  for (const auto &c : {std::make_pair(plain, 1000), std::make_pair(dense, 500)})
+    for (const uint32_t k : {10u, 4096u, 60000u}) {
+      argmax = 0;
+      require(select(c.first, c.second, k) == 0, "select");
+      require(argmax == static_cast<int>(k), "not a round per seed");
+    }
+  if (g_largest_graph < 4096 || g_largest_graph > 25000) {
+    printf("%d launches in a graph\n", g_largest_graph);
+    exit(1);
+  }
+  g_on_launch = end_rounds;
+  rip_pool_destroy(plain);
+  rip_pool_destroy(dense);
+  rip_graph_destroy(g);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -294,6 +319,7 @@ int main(int argc, char **argv) {
       {"long_sets_fill_the_chip", long_sets_fill_the_chip},
       {"long_lists_go_wide", long_lists_go_wide},
       {"poor_passes_end", poor_passes_end},
+      {"graphs_stay_bounded", graphs_stay_bounded},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;

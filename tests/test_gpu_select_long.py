@@ -83,3 +83,20 @@ def test_sorted_index_matches_oracle(pool, orc):
     assert before - device_free() > 16 * total
     p.close()
     g.close()
+
+
+def test_more_seeds_than_a_graph_holds(orc):
+    """A pool with column sets, whose rounds run over all vertices."""
+    src, dst = R.rmat_edges(14, seed=9)
+    index, edges, w = R.csr_from_edges(1 << 14, src, dst, R.W_UNIFORM, 0.1, 9)
+    g = R.Graph(index, edges, w)
+    p = g.pool(5)
+    p.generate_rrr_sets(20000)
+    assert p.columns()[0] > 0
+    off, ver = p.export()
+    for k in (4096, 4097, 6000):
+        seeds, cov = p.find_most_influential_set(k)
+        es, ec = orc.select(1 << 14, off, ver, k)
+        assert seeds.tolist() == es.tolist() and cov == ec
+    p.close()
+    g.close()

@@ -29,6 +29,7 @@ def exe(tmp_path_factory):
     "long_sets_fill_the_chip",
     "long_lists_go_wide",
     "poor_passes_end",
+    "graphs_stay_bounded",
 ])
 def test_host_rules(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=300)
