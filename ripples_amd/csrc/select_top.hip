@@ -244,10 +244,12 @@ struct TopState {
 };
 
 // Whether this is the last block of the launch to get here (every thread
-// gets the answer).  What the other blocks wrote with atomics before is then
-// there for atomic loads: every wave waits for its own before the block
-// counts itself done.  One fence per block, not per wave: an agent-scope
-// release writes back the XCD's L2, and 8,000 of them took 0.13 ms.
+// gets the answer).  What the other blocks wrote before is then there: each
+// waits for its waves' accesses and writes back its XCD's L2 before it counts
+// itself done, and the last one drops what its own L1 and L2 hold after the
+// count, so that plain loads (the rounds' records) find it as atomic ones do.
+// One fence per block, not per wave: an agent-scope release writes back the
+// XCD's L2, and 8,000 of them took 0.13 ms.
 __device__ inline bool last_block(uint32_t *done, uint32_t *s_flag) {
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
@@ -255,7 +257,10 @@ __device__ inline bool last_block(uint32_t *done, uint32_t *s_flag) {
     __threadfence();
     const uint32_t d = atomicAdd(done, 1u);
     *s_flag = d + 1 == gridDim.x;
-    if (*s_flag) atomicExch(done, 0u);
+    if (*s_flag) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      atomicExch(done, 0u);
+    }
   }
   __syncthreads();
   return *s_flag != 0;
