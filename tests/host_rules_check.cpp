@@ -308,6 +308,38 @@ void graphs_stay_bounded() {
   rip_graph_destroy(g);
 }
 
+// Spread workgroups have as many threads as leave 16 waves to a CU, by how many
+// of them it holds: one each where two bitmaps do not fit its 160 KiB of LDS.
+void spread_fills_its_cus() {
+  const struct {
+    int model;
+    uint32_t n;
+    uint64_t replicas;
+    uint32_t threads;
+  } cases[] = {
+      {RIP_IC, 700001, 8, 1024}, {RIP_IC, 700001, 4, 1024}, {RIP_IC, 1000003, 64, 1024},
+      {RIP_IC, 600000, 8, 512},  {RIP_IC, 300000, 64, 256}, {RIP_IC, 2000, 8, 512},
+      {RIP_LT, 400000, 8, 1024}, {RIP_LT, 280000, 8, 512},
+  };
+  for (const auto &c : cases) {
+    rip_graph *g = ring(c.model, c.n);
+    const uint32_t seed = 3;
+    std::vector<uint64_t> act(c.replicas);
+    std::vector<uint32_t> lev(c.replicas);
+    uint32_t threads = 0;
+    g_on_launch = [&](const std::string &kernel, Dim3, Dim3 block, size_t, void **) {
+      if (is(kernel, "spread_")) threads = block.x;
+    };
+    require(rip_spread(g, &seed, 1, 1, 0, c.replicas, act.data(), lev.data()) == 0, "spread");
+    if (threads != c.threads) {
+      printf("%u threads for %llu replicas on %u vertices, not %u\n", threads,
+             static_cast<unsigned long long>(c.replicas), c.n, c.threads);
+      exit(1);
+    }
+    rip_graph_destroy(g);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -320,6 +352,7 @@ int main(int argc, char **argv) {
       {"long_lists_go_wide", long_lists_go_wide},
       {"poor_passes_end", poor_passes_end},
       {"graphs_stay_bounded", graphs_stay_bounded},
+      {"spread_fills_its_cus", spread_fills_its_cus},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;

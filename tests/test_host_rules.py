@@ -30,6 +30,7 @@ def exe(tmp_path_factory):
     "long_lists_go_wide",
     "poor_passes_end",
     "graphs_stay_bounded",
+    "spread_fills_its_cus",
 ])
 def test_host_rules(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=300)
