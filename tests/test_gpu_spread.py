@@ -54,3 +54,12 @@ def test_lt_sums_at_the_threshold(orc):
     hit = rng.random(len(odd)) < 0.02
     odd[hit] = rng.choice(np.array([-0.5, np.inf, np.nan, -np.inf], np.float32), hit.sum())
     check(R.LT, (index, edges, odd), np.arange(9, dtype=np.uint32), 200, orc)
+
+
+@pytest.mark.parametrize("wscale", [0.2, 0.5, 0.8])
+def test_lt_replicas_one_after_the_other(wscale, orc):
+    """Several replicas to a workgroup, whose sums start at zero whether the one
+    before met few edges or many."""
+    seeds = np.arange(0, 40, 2, dtype=np.uint32)
+    check(R.LT, rmat(3001, 12, 6, R.W_LT_NORM, wscale, 5), seeds, 4000, orc)
+    check(R.LT, rmat(40009, 16, 8, R.W_LT_NORM, wscale, 6), seeds[:4], 2500, orc)
