@@ -20,15 +20,17 @@ constexpr uint64_t kProbeBase = 16384;   // sets of the first probe (probe_sets 
 constexpr double kProbeTargetMs = 20.0;    // time per candidate the probe is scaled to
 
 std::mutex g_tune_mu;
-std::map<std::tuple<int, int, int>, rip_tune> g_tune_cache;
+using Key = std::tuple<int, int, int, bool>;
+std::map<Key, rip_tune> g_tune_cache;
 
-// (model, log2 of the largest in-degree over the mean, log2 n): graphs alike
-// in these share their settings.
-std::tuple<int, int, int> skew_key(const rip_graph *g) {
+// (model, log2 of the largest in-degree over the mean, log2 n, which sampler
+// takes the large sets): graphs alike in these share their settings.
+Key skew_key(const rip_graph *g) {
   const double mean = g->n ? static_cast<double>(g->m) / g->n : 0.0;
   const double skew = mean > 0 ? g->max_degree / mean : 1.0;
   return std::make_tuple(g->model, static_cast<int>(std::lround(std::log2(std::max(1.0, skew)))),
-                         static_cast<int>(std::lround(std::log2(std::max(1.0, double(g->n))))));
+                         static_cast<int>(std::lround(std::log2(std::max(1.0, double(g->n))))),
+                         g->n <= kTeamMaxNodes);
 }
 
 // IC: the lane list capacity 64..4096 (how large a sample grows before the grid

@@ -340,6 +340,23 @@ void spread_fills_its_cus() {
   }
 }
 
+// A graph whose large sets the team sampler takes and one where the grid does
+// share no autotuned setting, alike as they are.
+void tuned_settings_part_at_the_team_line() {
+  rip_tune t{};
+  double ms;
+  uint32_t tried = 0;
+  rip_graph *above = ring(RIP_IC, (1u << 20) + 5), *alike = ring(RIP_IC, (1u << 20) + 9);
+  rip_graph *below = ring(RIP_IC, (1u << 20) - 5);
+  require(rip_autotune(above, 2000, 1, &t, &ms, &tried) == 0 && tried > 0, "tune");
+  require(rip_autotune(alike, 2000, 0, &t, &ms, &tried) == 0 && tried == 0, "a graph alike was timed again");
+  require(rip_autotune(below, 2000, 0, &t, &ms, &tried) == 0 && tried > 0,
+          "a setting timed with the grid was taken over");
+  rip_graph_destroy(above);
+  rip_graph_destroy(alike);
+  rip_graph_destroy(below);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -353,6 +370,7 @@ int main(int argc, char **argv) {
       {"poor_passes_end", poor_passes_end},
       {"graphs_stay_bounded", graphs_stay_bounded},
       {"spread_fills_its_cus", spread_fills_its_cus},
+      {"tuned_settings_part_at_the_team_line", tuned_settings_part_at_the_team_line},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
