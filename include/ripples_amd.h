@@ -178,15 +178,15 @@ int rip_pool_append_host(rip_pool *p, uint64_t count, const uint64_t *offsets,
                          const uint32_t *vertices);
 /* Autotuner: draws probe_sets samples (0: 16384 times the factor, 1 to 16,
  * that brings one candidate's draw to about 20 ms) with each candidate setting (IC: the
- * lane list capacity 64/256/1024/2048/4096 x the lane kernel's workgroup size,
- * capacities 64/256/1024 with the wave stage, then 32 against 64 samples per
- * colour group of the grid sampler
- * 256/512/1024; LT: the walk's output chunk) and keeps the fastest, which
- * the graph then uses for every sampling call given no tune (rip_pool_sample,
- * rip_imm, the server).  The choice is remembered per (model, degree skew =
- * round(log2(max in-degree / mean)), round(log2 n)); a later call on a graph
- * of the same key takes it without probing unless force is set.  *best_ms:
- * the winner's time per probe batch (0 when taken from the cache); *tried:
+ * lane list capacity 64/256/1024/2048/4096 x the lane kernel's workgroup size
+ * 256/512/1024, the wave stage with the output chunk 0/256/1024, then 32
+ * samples per colour group of the grid sampler; LT: the walk's output chunk)
+ * and keeps the fastest, which the graph then uses for every sampling call
+ * given no tune (rip_pool_sample, rip_imm, the server).  The choice is
+ * remembered per (model, degree skew = round(log2(max in-degree / mean)),
+ * round(log2 n), whether n <= 2^20); a later call on a graph of the same key
+ * takes it without probing unless force is set.  *best_ms: the winner's time
+ * per probe batch (0 when taken from the cache); *tried:
  * settings timed.  No counterpart call in the reference, whose GPU batch
  * size comes from a similar probe (streaming_rrr_generator.h:1150-1241). */
 int rip_autotune(rip_graph *g, uint64_t probe_sets, int force, rip_tune *best,

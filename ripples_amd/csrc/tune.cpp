@@ -33,10 +33,11 @@ Key skew_key(const rip_graph *g) {
                          g->n <= kTeamMaxNodes);
 }
 
-// IC: the lane list capacity 64..4096 (how large a sample grows before the grid
-// sampler takes it) and the lane kernel's workgroup size, and three settings
-// with the wave stage between the lanes and the grid; LT: the output chunk of
-// the walk kernel's waves.
+// IC: the lane list capacity 64..4096 (how large a sample grows before the
+// large-set samplers take it) and the lane kernel's workgroup size, and the wave
+// stage behind short lanes, which is the automatic setting, with three output
+// chunks of its waves (its lanes are the same whatever the capacity and the
+// workgroup size); LT: the output chunk of the walk kernel's waves.
 std::vector<rip_tune> candidates(int model) {
   std::vector<rip_tune> c;
   if (model == RIP_IC) {
@@ -47,12 +48,12 @@ std::vector<rip_tune> candidates(int model) {
         t.block = block;
         c.push_back(t);
       }
-    // the wave stage between the lanes and the grid sampler
-    for (uint32_t cap : {64u, 256u, 1024u}) {
+    for (uint32_t chunk : {0u, 256u, 1024u}) {
       rip_tune t{};
-      t.queue_cap = cap;
+      t.queue_cap = kLaneCapStaged;
       t.block = 256;
       t.wave_stage = 1;
+      t.out_chunk = chunk;
       c.push_back(t);
     }
   } else {
@@ -132,8 +133,9 @@ void autotune(rip_graph *g, uint64_t probe, bool force, rip_tune *best, double *
       }
     }
     if (g->model == RIP_IC) {
-      // then the samples per colour group of the grid sampler, with the
-      // lane setting chosen
+      // then the samples per colour group of the grid sampler, with the lane
+      // setting chosen (and the grid in place of the team sampler on small
+      // graphs)
       for (uint32_t colors : {32u}) {
         rip_tune c = pick;
         c.colors = colors;

@@ -1,5 +1,6 @@
 // Host checks of what the library does around its kernels, on the HIP runtime
 // of fake_hip.h.  Each check has a name, given as the argument.
+#include <chrono>
 #include <vector>
 
 #include "fake_hip.h"
@@ -357,6 +358,31 @@ void tuned_settings_part_at_the_team_line() {
   rip_graph_destroy(below);
 }
 
+// The autotuner's settings with the wave stage differ in what they run: each in
+// turn made the fastest, the last has another output chunk, not another lane
+// capacity, which those lanes do not heed.
+void staged_settings_differ() {
+  rip_graph *g = ring(RIP_IC, 5000);
+  rip_tune t{};
+  double ms;
+  uint32_t tried = 0;
+  int staged = 0;
+  g_on_launch = [&](const std::string &kernel, Dim3, Dim3, size_t, void **) {
+    int wait = is(kernel, "ic_lane_kernel") ? 40 : 0;
+    if (is(kernel, "ic_short_kernel")) wait = 30 - 5 * ++staged;   // two a setting
+    for (const auto end = std::chrono::steady_clock::now() + std::chrono::milliseconds(wait);
+         std::chrono::steady_clock::now() < end;) {}
+  };
+  require(rip_autotune(g, 20000, 1, &t, &ms, &tried) == 0, "tune");
+  g_on_launch = end_rounds;
+  if (staged < 6 || !t.wave_stage || t.queue_cap != 64 || t.out_chunk != 1024) {
+    printf("after %d calls: queue_cap %u, wave_stage %u, out_chunk %u\n", staged, t.queue_cap, t.wave_stage,
+           t.out_chunk);
+    exit(1);
+  }
+  rip_graph_destroy(g);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -371,6 +397,7 @@ int main(int argc, char **argv) {
       {"graphs_stay_bounded", graphs_stay_bounded},
       {"spread_fills_its_cus", spread_fills_its_cus},
       {"tuned_settings_part_at_the_team_line", tuned_settings_part_at_the_team_line},
+      {"staged_settings_differ", staged_settings_differ},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;

@@ -32,6 +32,7 @@ def exe(tmp_path_factory):
     "graphs_stay_bounded",
     "spread_fills_its_cus",
     "tuned_settings_part_at_the_team_line",
+    "staged_settings_differ",
 ])
 def test_host_rules(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=300)
