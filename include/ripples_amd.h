@@ -158,6 +158,9 @@ int rip_graph_create(int device, int model, uint32_t num_nodes,
 int rip_graph_destroy(rip_graph *g);
 int rip_graph_info(const rip_graph *g, uint32_t *num_nodes,
                    uint64_t *num_edges, int *model);
+/* Gives the device memory back that destroyed pools of the graph left for its
+ * next ones (at most a 64th of the device's); live pools keep theirs. */
+int rip_graph_trim(rip_graph *g);
 
 /* ---------------------------------------------------------------- pool */
 /* Empty RRR pool bound to graph g and the sampling stream of `seed`

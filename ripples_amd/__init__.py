@@ -124,6 +124,7 @@ def lib():
     L.rip_graph_create.argtypes = [C.c_int, C.c_int, C.c_uint32, C.c_uint64, _u64p,
                                    _u32p, _f32p, C.POINTER(vp)]
     L.rip_graph_destroy.argtypes = [vp]
+    L.rip_graph_trim.argtypes = [vp]
     L.rip_graph_info.argtypes = [vp, C.POINTER(C.c_uint32), C.POINTER(C.c_uint64),
                                  C.POINTER(C.c_int)]
     L.rip_pool_create.argtypes = [vp, C.c_uint64, C.POINTER(vp)]
@@ -324,6 +325,10 @@ class Graph:
             self.close()
         except Exception:
             pass
+
+    def trim(self):
+        """Give back the device memory closed pools left for the next ones."""
+        _check(lib().rip_graph_trim(self._h))
 
     def spread(self, seeds, replicas, seed=0, first=0):
         """Monte Carlo spread of `seeds` (diffusion_simulation.h:73-178):

@@ -84,6 +84,14 @@ int rip_graph_destroy(rip_graph *g) {
   });
 }
 
+int rip_graph_trim(rip_graph *g) {
+  return guarded([&] {
+    RIP_REQUIRE(g, RIP_EINVAL, "graph is NULL");
+    RIP_HIP(hipSetDevice(g->device));
+    g->blocks->release();
+  });
+}
+
 int rip_graph_info(const rip_graph *g, uint32_t *num_nodes, uint64_t *num_edges,
                    int *model) {
   return guarded([&] {

@@ -383,6 +383,30 @@ void staged_settings_differ() {
   rip_graph_destroy(g);
 }
 
+// What destroyed pools left to their graph goes back to the device when asked
+// for; live pools keep theirs.
+void idle_memory_is_given_back() {
+  rip_graph *g = ring(RIP_IC, 5000);
+  const size_t graph = used();
+  rip_pool *live_pool = runs(g, 5000, 1000, 10);
+  const size_t with_live = used();
+  rip_pool *p = runs(g, 5000, 60000, 10);
+  require(select(p, 60000, 5) == 0, "select");
+  rip_pool_destroy(p);
+  require(used() > with_live, "nothing was kept");
+  require(rip_graph_trim(g) == 0, "trim");
+  if (used() > with_live + 4096) {   // a stream kit's control words
+    printf("%zu bytes after, %zu before\n", used(), with_live);
+    exit(1);
+  }
+  require(select(live_pool, 1000, 5) == 0, "select");
+  rip_pool_destroy(live_pool);
+  require(rip_graph_trim(g) == 0, "trim");
+  require(used() <= graph + 4096, "idle blocks are left");
+  rip_graph_destroy(g);
+  require(rip_graph_trim(nullptr) == RIP_EINVAL, "no graph");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -398,6 +422,7 @@ int main(int argc, char **argv) {
       {"spread_fills_its_cus", spread_fills_its_cus},
       {"tuned_settings_part_at_the_team_line", tuned_settings_part_at_the_team_line},
       {"staged_settings_differ", staged_settings_differ},
+      {"idle_memory_is_given_back", idle_memory_is_given_back},
   };
   const auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;

@@ -33,6 +33,7 @@ def exe(tmp_path_factory):
     "spread_fills_its_cus",
     "tuned_settings_part_at_the_team_line",
     "staged_settings_differ",
+    "idle_memory_is_given_back",
 ])
 def test_host_rules(exe, name):
     r = subprocess.run([exe, name], capture_output=True, text=True, timeout=300)
