@@ -773,12 +773,11 @@ __device__ inline unsigned long long transpose64(unsigned long long x) {
   return x;
 }
 
-// Step 2: per chunk (one wave), members of each colour, all and hot.  Where 64
-// members hold many colours the masks are transposed, so that a lane counts its
-// colour at once: about 100 instructions, against 8 a colour (20,000 sets on an
-// R-MAT graph of 2^24 vertices and a selection: 108.0 -> 107.0 ms).
-constexpr int kManyColours = 12;
-
+// Step 2: per chunk (one wave), members of each colour, all and hot: 64 members'
+// masks are transposed, so that a lane counts its colour at once.  That is about
+// 100 instructions, against 8 for each colour they hold by ballots (20,000 sets
+// on an R-MAT graph of 2^24 vertices and a selection: 105.4 ms by ballots, 104.2
+// so; twenty sets on one of 2^21 2.20 either way).
 __global__ void __launch_bounds__(64) out_chunk_count_kernel(OutParams P) {
   const uint64_t c = blockIdx.x;
   const uint32_t i = group_of_chunk(P.cbase, P.groups, c);
@@ -790,24 +789,10 @@ __global__ void __launch_bounds__(64) out_chunk_count_kernel(OutParams P) {
   uint32_t all = 0, hot = 0;   // lane j: colour j's counts
   for (uint64_t t = e0; t < e1; t += 64) {
     const uint64_t e = t + lane;
-    const unsigned long long m = e < e1 ? masks[e] : 0ull;
     const bool h = P.colptr && e < e1 && P.hot_index[list[e]] != kNotHot;
-    unsigned long long u = uniform_u64(wave_or_u64(m));
-    if (__popcll(u) >= kManyColours) {
-      const unsigned long long col = transpose64(m);
-      all += static_cast<uint32_t>(__popcll(col));
-      hot += static_cast<uint32_t>(__popcll(col & __ballot(h)));
-      continue;
-    }
-    for (; u; u &= u - 1) {
-      const uint32_t col = static_cast<uint32_t>(__ffsll(u) - 1);
-      const uint64_t b = __ballot((m >> col) & 1ull);
-      const uint64_t bh = __ballot(h && ((m >> col) & 1ull));
-      if (lane == col) {
-        all += static_cast<uint32_t>(__popcll(b));
-        hot += static_cast<uint32_t>(__popcll(bh));
-      }
-    }
+    const unsigned long long col = transpose64(e < e1 ? masks[e] : 0ull);
+    all += static_cast<uint32_t>(__popcll(col));
+    hot += static_cast<uint32_t>(__popcll(col & __ballot(h)));
   }
   P.cc[c * 64 + lane] = all;
   P.cch[c * 64 + lane] = hot;
