@@ -91,7 +91,7 @@ struct IcSlots {
 };
 
 // Scratch of the wave IC sampler: per resident wave a visited table and a
-// BFS list; samples too large for them are handed to the colour sampler.
+// BFS list; samples too large for them are listed for the large-set kernels.
 struct WaveScratch {
   uint64_t waves = 0;
   unsigned long long *d_table = nullptr;  // waves x table capacity
@@ -106,8 +106,6 @@ struct WaveScratch {
   uint32_t *d_bbits = nullptr;
   uint32_t *d_bsum = nullptr;
   uint32_t *d_blist = nullptr;
-  // lane kernel: per lane a visited table of 2 cap entries, a list of cap
-  // vertices and an epoch; samples that outgrew a lane, sets to sort
   // wave stage: per wave and slot a visited table of 2 cap entries and a list
   // of cap vertices; sets to sort
   uint64_t stage_waves = 0;
@@ -115,6 +113,8 @@ struct WaveScratch {
   uint32_t *d_slist = nullptr;
   uint64_t cap_ssort = 0;
   uint32_t *d_ssort = nullptr;
+  // lane kernel: per lane a visited table of 2 cap entries, a list of cap
+  // vertices and an epoch; samples that outgrew a lane, sets to sort
   uint64_t lane_lanes = 0;
   uint32_t lane_cap = 0;
   unsigned long long *d_ltable = nullptr;
@@ -407,11 +407,8 @@ void pool_export(rip_pool *p, uint64_t first, uint64_t count,
 
 // sample_ic.hip
 struct IcLaunch {
-  uint32_t colors, block, slots, queue_cap, heavy_degree, sampler;
-  bool colors_auto;    // colours not set by the caller
+  uint32_t colors, block, slots, heavy_degree, sampler;
   uint32_t out_chunk;  // wave sampler's output chunk, 0 = automatic
-  bool block_auto;     // block size not set by the caller
-  bool slots_auto;     // slots not set by the caller
 };
 
 // Pool elements a sampler wave reserves at a time: a power of two in
@@ -426,12 +423,8 @@ inline uint32_t out_chunk_rule(double elems_per_wave, uint32_t max_chunk) {
 }
 IcLaunch ic_tune(const rip_pool *p, const rip_tune *tune);
 void ic_ensure_slots(rip_pool *p, uint32_t slots, uint32_t heavy_deg);
-// Colour sampler over samples first + i, i in [0, count), or first + ids[i].
-// With columns, groups whose sets hold many hot members store them in the
-// pool's column store (pool.hip).
-uint32_t ic_launch(rip_pool *p, uint64_t first, uint64_t count,
-                   const IcLaunch &cfg, const uint32_t *ids = nullptr,
-                   bool record_events = true, bool columns = false);
+// Colour sampler over samples [first, first + count).
+uint32_t ic_launch(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &cfg);
 
 // IC sampling of samples [first, first+count) with the configured sampler
 uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &cfg,

@@ -65,39 +65,13 @@ struct IcParams {
   uint32_t heavy_deg;   // rows at least this long wait for the hub phase
   uint32_t *hub;        // slots x 2 x hub_cap deferred-hub lists
   uint64_t hub_cap;
-  const uint32_t *sample_ids;  // optional: local index -> sample index (minus first)
-  uint32_t precheck;    // read visited masks before their atomics (giant components)
-  // column store (nullptr: every set a list): a group whose sets hold more
-  // than 2 hot_n hot members in all takes the next column (columns
-  // group_base, group_base + 1, ... as counted in ctl[kCtlGroupCounter2])
-  unsigned long long *const *colptr;
-  uint32_t *gsample;
-  uint32_t *gref;
-  const uint32_t *hot_index;
-  uint32_t hot_n;
-  uint32_t group_base;
 };
 
-__device__ inline uint64_t sample_id(const IcParams &P, uint64_t local) {
-  return P.first + (P.sample_ids ? P.sample_ids[local] : local);
-}
-
-// Mark (u, bits) discovered.  Every lane of the wave must call it.  With
-// precheck the visited mask is read first and the atomic skipped when no
-// colour is new: within a group masks only gain bits, so a read that lags
-// can only cost an extra atomic.  In a giant component most edges reach
-// vertices every colour has visited, and their atomics, many on the same hub
-// words, were most of the expansion time; elsewhere the read is one more
-// round trip.  The read is a device-scope atomic load, served by L2 like the
-// atomics: a plain load could meet a vector-L1 line from an earlier group,
-// whose masks have since been cleared.
-template <bool kPrecheck>
+// Mark (u, bits) discovered.  Every lane of the wave must call it.
 __device__ inline void discover(unsigned long long *vp, uint32_t *bm0, uint32_t *bm1, uint32_t u,
                                 unsigned long long bits, uint32_t *s_union, uint32_t *s_qn,
                                 uint32_t *qnext) {
   bool first = false, push = false;
-  if (kPrecheck && bits)
-    bits &= ~__hip_atomic_load(&vp[2ull * u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (bits) {
     unsigned long long old = atomicOr(&vp[2ull * u], bits);
     unsigned long long fresh = bits & ~old;
@@ -117,7 +91,7 @@ __device__ inline void discover(unsigned long long *vp, uint32_t *bm0, uint32_t 
   wave_append(push, u, s_qn, qnext);
 }
 
-template <int BT, bool kPrecheck>
+template <int BT>
 __global__ void __launch_bounds__(BT)
 ic_fused_kernel(IcParams P) {
   constexpr int NW = BT / 64;
@@ -145,8 +119,6 @@ ic_fused_kernel(IcParams P) {
   __shared__ unsigned long long s_ea[BT];
   __shared__ unsigned long long s_eb[BT];
   __shared__ unsigned long long s_em[BT];
-  __shared__ unsigned long long s_hot[BT / 64];
-  __shared__ uint32_t s_col;       // the group's column, or kNoGroup
 
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = lane_id();
@@ -192,14 +164,14 @@ ic_fused_kernel(IcParams P) {
     uint32_t root = 0;
     unsigned long long rbits = 0;
     if (tid < nb) {
-      unsigned long long z = sample_z(P.seed, sample_id(P, s0 + tid));
+      unsigned long long z = sample_z(P.seed, P.first + s0 + tid);
       s_z[tid] = z;
       root = uniform_index(z, P.n);
       rbits = 1ull << tid;
     }
     __syncthreads();
     if (tid < 64)
-      discover<kPrecheck>(vp, bm0, bm1, root, rbits, &s_union, &s_qn[0], q0);
+      discover(vp, bm0, bm1, root, rbits, &s_union, &s_qn[0], q0);
 
     // ---------------------------------------------------------- BFS levels
     // Light levels expand the frontier queue; rows of at least heavy_deg
@@ -343,7 +315,7 @@ ic_fused_kernel(IcParams P) {
               }
             }
             if (__ballot(bits != 0) == 0) break;
-            discover<kPrecheck>(vp, bm0, bm1, src, bits, &s_union, &s_qn[lnext], qnext);
+            discover(vp, bm0, bm1, src, bits, &s_union, &s_qn[lnext], qnext);
           }
         }
         __syncthreads();
@@ -384,48 +356,6 @@ ic_fused_kernel(IcParams P) {
       running += tot;
     }
     __syncthreads();
-    if (P.colptr) {
-      // per-group choice of representation: a column costs 8 bytes per hot
-      // vertex, lists 4 per member; the group's hot members decide
-      unsigned long long hot = 0;
-      for (uint32_t i = tid; i < U; i += BT)
-        if (P.hot_index[list[i]] != kNotHot) hot += __popcll(masks[i]);
-      unsigned long long tot_hot;
-      (void)block_exclusive_scan_u64<BT>(hot, s_hot, &tot_hot);
-      if (tid == 0) {
-        s_col = kNoGroup;
-        if (tot_hot > 2ull * P.hot_n)
-          s_col = P.group_base +
-                  static_cast<uint32_t>(atomicAdd(&P.ctl[kCtlGroupCounter2], 1ull));
-      }
-      __syncthreads();
-      const uint32_t colg = s_col;
-      if (colg != kNoGroup) {
-        unsigned long long *col = P.colptr[colg];
-        for (uint32_t h = tid; h < P.hot_n; h += BT) col[h] = 0ull;
-        __syncthreads();
-        // hot members go to the column, which the lists then leave out
-        for (uint32_t i = tid; i < U; i += BT) {
-          const uint32_t h = P.hot_index[list[i]];
-          if (h != kNotHot) {
-            col[h] = masks[i];
-            masks[i] = 0ull;
-          }
-        }
-        st_bytes += 8ull * ((P.hot_n + BT - 1 - tid) / BT);
-        // the pool's element count includes the members held in the column
-        if (tid == 0) atomicAdd(&P.ctl[kCtlElems], tot_hot);
-        if (tid < 64) {
-          uint32_t sid = kNoGroup;
-          if (tid < nb) {
-            sid = static_cast<uint32_t>(sample_id(P, s0 + tid));
-            P.gref[sid] = (colg << 6) | tid;
-          }
-          P.gsample[64ull * colg + tid] = sid;
-        }
-      }
-      __syncthreads();
-    }
     for (uint32_t i = tid; i < U; i += BT)
       for (unsigned long long mk = masks[i]; mk; mk &= mk - 1)
         atomicAdd(&s_cnt[__ffsll(mk) - 1], 1u);
@@ -458,13 +388,13 @@ ic_fused_kernel(IcParams P) {
         }
       }
       if (tid < nb) {
-        const uint64_t s = sample_id(P, s0 + tid);
+        const uint64_t s = P.first + s0 + tid;
         P.set_off[s] = base + s_cofs[tid];
         P.set_len[s] = s_cnt[tid];
         st_bytes += 4ull * s_cnt[tid];
       }
     } else if (tid < nb) {
-      P.set_len[sample_id(P, s0 + tid)] = 0xFFFFFFFFu;
+      P.set_len[P.first + s0 + tid] = 0xFFFFFFFFu;
     }
     __syncthreads();
   }
@@ -473,10 +403,7 @@ ic_fused_kernel(IcParams P) {
 
 template <int BT>
 void launch_one(const IcParams &P, uint32_t slots, hipStream_t stream) {
-  if (P.precheck)
-    hipLaunchKernelGGL((ic_fused_kernel<BT, true>), dim3(slots), dim3(BT), 0, stream, P);
-  else
-    hipLaunchKernelGGL((ic_fused_kernel<BT, false>), dim3(slots), dim3(BT), 0, stream, P);
+  hipLaunchKernelGGL((ic_fused_kernel<BT>), dim3(slots), dim3(BT), 0, stream, P);
 }
 
 __global__ void reset_counter_kernel(unsigned long long *ctl) {
@@ -486,7 +413,7 @@ __global__ void reset_counter_kernel(unsigned long long *ctl) {
 // Workgroups of the persistent kernel that fit on one CU at once.
 template <int BT>
 int occupancy_of() {
-  return blocks_per_cu(reinterpret_cast<const void *>(&ic_fused_kernel<BT, false>), BT);
+  return blocks_per_cu(reinterpret_cast<const void *>(&ic_fused_kernel<BT>), BT);
 }
 
 int resident_blocks(uint32_t block) {
@@ -518,21 +445,11 @@ IcLaunch ic_tune(const rip_pool *p, const rip_tune *tune) {
   // defaults from a sweep on R-MAT scale 22 weighted cascade: 8-edge runs and
   // 256-thread groups (more independent groups per CU); hub deferral off,
   // because colours of one group rarely meet at the same hub there
-  IcLaunch c{64, 256, 0, 0, 0xFFFFFFFFu, RIP_SAMPLER_AUTO, true, 0, true, true};
+  IcLaunch c{64, 256, 0, 0xFFFFFFFFu, RIP_SAMPLER_AUTO, 0};
   if (tune) {
-    if (tune->colors) {
-      c.colors = tune->colors;
-      c.colors_auto = false;
-    }
-    if (tune->block) {
-      c.block = tune->block;
-      c.block_auto = false;
-    }
-    if (tune->slots) {
-      c.slots = tune->slots;
-      c.slots_auto = false;
-    }
-    c.queue_cap = tune->queue_cap;
+    if (tune->colors) c.colors = tune->colors;
+    if (tune->block) c.block = tune->block;
+    if (tune->slots) c.slots = tune->slots;
     if (tune->heavy_degree) c.heavy_degree = tune->heavy_degree;
     c.sampler = tune->sampler;
     c.out_chunk = tune->out_chunk;
@@ -586,9 +503,7 @@ void ic_ensure_slots(rip_pool *p, uint32_t slots, uint32_t heavy_deg) {
   s.slot_bytes = slot_bytes_for(p->g, heavy_deg);
 }
 
-uint32_t ic_launch(rip_pool *p, uint64_t first, uint64_t count,
-                   const IcLaunch &cfg, const uint32_t *ids, bool record_events,
-                   bool columns) {
+uint32_t ic_launch(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &cfg) {
   // no more resident groups than there are groups; scratch only ever grows
   const uint64_t groups = (count + cfg.colors - 1) / cfg.colors;
   ic_ensure_slots(p, static_cast<uint32_t>(std::min<uint64_t>(cfg.slots, groups)),
@@ -620,39 +535,17 @@ uint32_t ic_launch(rip_pool *p, uint64_t first, uint64_t count,
   P.heavy_deg = cfg.heavy_degree;
   P.hub = p->g->ic.d_hub;
   P.hub_cap = p->g->ic.hub_cap;
-  P.sample_ids = ids;
-  P.colptr = nullptr;
-  P.gsample = nullptr;
-  P.gref = nullptr;
-  P.hot_index = nullptr;
-  P.hot_n = 0;
-  P.group_base = 0;
-  if (columns) {
-    // room for a column per group of the launch; groups whose sets are too
-    // small for one keep lists and leave theirs unused
-    pool_reserve_groups(p, p->groups + static_cast<uint32_t>(P.ngroups));
-    P.colptr = p->d_colptr;
-    P.gsample = p->d_gsample;
-    P.gref = p->d_gref;
-    P.hot_index = g->d_hot_index;
-    P.hot_n = g->hot_n;
-    P.group_base = p->groups;
-  }
-  // the large-set fallback walks giant components, where most edges reach
-  // vertices every colour has visited; a whole launch of mostly small sets
-  // (weighted cascade) gains nothing from the extra read
-  P.precheck = ids != nullptr;
   const uint32_t slots =
       static_cast<uint32_t>(std::min<uint64_t>(cfg.slots, P.ngroups));
   hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(1), 0, p->stream, p->d_ctl);
-  if (record_events) RIP_HIP(hipEventRecord(p->ev0, p->stream));
+  RIP_HIP(hipEventRecord(p->ev0, p->stream));
   switch (cfg.block) {
     case 256: launch_one<256>(P, slots, p->stream); break;
     case 1024: launch_one<1024>(P, slots, p->stream); break;
     default: launch_one<512>(P, slots, p->stream); break;
   }
   RIP_HIP(hipGetLastError());
-  if (record_events) RIP_HIP(hipEventRecord(p->ev1, p->stream));
+  RIP_HIP(hipEventRecord(p->ev1, p->stream));
   return 2;
 }
 
@@ -684,7 +577,7 @@ uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &
   if (cfg.sampler == RIP_SAMPLER_COLOUR) return ic_launch(p, first, count, cfg);
   uint32_t launches = 0;
   if (count <= kWaveDirectMax && ic_wave_stage(tune)) {
-    // few samples: one wave each from the start, with no lanes before
+    // few samples: the wave stage from the start, with no lanes before
     const uint64_t big = ic_stage_launch(p, first, count, nullptr, cfg.out_chunk, true);
     launches += 2;
     if (big == 0) return launches;
@@ -695,15 +588,16 @@ uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &
   const bool lanes = cfg.sampler == RIP_SAMPLER_AUTO || cfg.sampler == RIP_SAMPLER_LANE;
   if (lanes) {
     // one sample per lane first; the few that outgrow a lane's queue go to
-    // the grid sampler (AUTO) or to one BFS per wave (LANE)
+    // the wave stage and the large-set samplers (AUTO) or to one BFS per wave
+    // (LANE)
     wave_count = ic_lane_launch(p, first, count, tune);
     launches += 3;
     if (wave_count == 0) return launches;
     wave_ids = p->g->wave.d_over;
     if (cfg.sampler == RIP_SAMPLER_AUTO) {
       if (ic_wave_stage(tune)) {
-        // one BFS per wave, 64 frontier vertices at a time, for the samples
-        // up to the wave list; the grid sampler takes the larger ones
+        // several samples per wave, 64 frontier vertices at a time, up to the
+        // stage's lists; the large-set samplers take the rest
         const uint64_t big = ic_stage_launch(p, first, wave_count, wave_ids, cfg.out_chunk, false);
         launches += 2;
         if (big == 0) return launches;
@@ -715,35 +609,8 @@ uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &
   const uint64_t big = ic_wave_launch(p, first, wave_count, wave_ids, cfg.out_chunk, !lanes);
   launches += 2;
   if (big == 0) return launches;
-  // sets that outgrew a wave's list: by default colour groups over the listed
-  // sample indices (samples that reach a giant component share most of their
-  // rows, which the groups read once for 64 of them); WAVE and LANE finish
-  // them with the bitmap-visited BFS per wave instead
-  if (cfg.sampler == RIP_SAMPLER_WAVE || cfg.sampler == RIP_SAMPLER_LANE) {
-    ic_big_launch(p, first, big);
-  } else {
-    // the groups are latency-bound, one level at a time: 512-thread groups
-    // (on R-MAT scale 18 with U[0,0.1] weights, 100,000 samples: 0.119 s at
-    // 64 colours against 0.150 s with 256 threads and 0.123 s with 1024) and
-    // about one group per two resident slots, i.e. colours near 2 big / slots
-    // (rounded to a power of two), measured best on R-MAT scales 16 and 18
-    // with U[0,0.1] weights from 1,000 to 17,000 large samples
-    IcLaunch fb = cfg;
-    if (cfg.block_auto) {
-      fb.block = 512;
-      if (cfg.slots_auto) {
-        fb.slots = std::min<uint32_t>(
-            cfg.slots, static_cast<uint32_t>(cu_count()) * resident_blocks(fb.block));
-      }
-    }
-    if (cfg.colors_auto) {
-      const double want = 2.0 * static_cast<double>(big) / std::max<uint32_t>(fb.slots, 1);
-      uint32_t c = 1;
-      while (c < 64 && static_cast<double>(c) * 1.41421356 < want) c <<= 1;
-      fb.colors = c;
-    }
-    ic_launch(p, first, big, fb, p->g->wave.d_big, false, true);
-  }
+  // sets that outgrew a wave's list: the bitmap-visited BFS per wave
+  ic_big_launch(p, first, big);
   return launches + 2;
 }
 
