@@ -132,15 +132,18 @@ struct Error : std::runtime_error {
 
 void set_last_error(const std::string &msg);
 
-// (The runtime keeps an error until it is asked for: one that is thrown must not
-// be found again by the launch check of a later call.)
-#define RIP_HIP(expr)                                                        \
-  do {                                                                       \
-    hipError_t _e = (expr);                                                  \
-    if (_e != hipSuccess) {                                                  \
-      (void)hipGetLastError();                                               \
-      throw ::rip::Error(-3, std::string(#expr) + ": " + hipGetErrorString(_e)); \
-    }                                                                        \
+// The runtime keeps an error until it is asked for: one that is thrown must not
+// be found again by the launch check of a later call.  (Out of line: the code of
+// a throw beside every call slowed the host loops around them.)
+[[noreturn]] __attribute__((noinline, cold)) inline void throw_hip(const char *expr, hipError_t e) {
+  (void)hipGetLastError();
+  throw Error(-3, std::string(expr) + ": " + hipGetErrorString(e));
+}
+
+#define RIP_HIP(expr)                                       \
+  do {                                                      \
+    hipError_t _e = (expr);                                 \
+    if (_e != hipSuccess) ::rip::throw_hip(#expr, _e);      \
   } while (0)
 
 #define RIP_REQUIRE(cond, code, msg)                                         \
