@@ -71,11 +71,12 @@ __device__ inline void report_stats(unsigned long long *ctl, unsigned long long 
     live += __shfl_down(live, d, 64);
   }
   if (lane_id() == 0) {
-    if (bytes) atomicAdd(&ctl[kCtlStatBytes], bytes);
-    if (cand) atomicAdd(&ctl[kCtlStatEdges], cand);
-    if (draws) atomicAdd(&ctl[kCtlStatCoins], draws);
-    if (exp) atomicAdd(&ctl[kCtlStatExpansions], exp);
-    if (live) atomicAdd(&ctl[kCtlStatLevels], live);
+    unsigned long long *s = ctl + kCtlStripe0 + blockIdx.x % kCtlStripes * kCtlLine;
+    if (bytes) atomicAdd(&s[RIP_STAT_ALGO_BYTES], bytes);
+    if (cand) atomicAdd(&s[RIP_STAT_EDGES], cand);
+    if (draws) atomicAdd(&s[RIP_STAT_COINS], draws);
+    if (exp) atomicAdd(&s[RIP_STAT_EXPANSIONS], exp);
+    if (live) atomicAdd(&s[RIP_STAT_LEVELS], live);
   }
 }
 

@@ -346,14 +346,20 @@ struct rip_pool {
 
 namespace rip {
 
-// control word indices in rip_pool::d_ctl
+// Control word indices in rip_pool::d_ctl.  Atomics on one line take turns, 12 ns
+// each: 4,096 waves that end together and add their five work counters to one
+// line take 250 us.  So the words every wave adds to have lines of their own, and
+// the work counters are kept in stripes, one per workgroup modulo kCtlStripes,
+// which the host sums.  100 sets of 1.7M vertices on a lattice of 2.25M (1,774
+// narrow levels): 410 ms with one line, 262 so (246 before waves took the levels'
+// items by themselves, a report per workgroup); 2,000 sets of a vertex or two 0.19
+// and 0.13; IMM on R-MAT scale 22 under weighted cascade 26.5 and 24.3.
 enum : int {
-  kCtlGroupCounter = 0,  // work counter of the persistent samplers
-  kCtlDataBump = 1,      // used elements of d_data
   kCtlOverflow = 2,      // nonzero when d_data ran out
   kCtlLongCount = 3,     // LT: walks that outgrew the per-lane list
   kCtlCovered = 4,       // selector: sets covered so far
-  kCtlStatBytes = 5,     // stats of the last sampler launch (RIP_STAT_* order)
+  kCtlStatBytes = 5,     // stats of the last sampler launch (RIP_STAT_* order), on the
+                         // host only: the sums of the stripes
   kCtlStatEdges = 6,
   kCtlStatCoins = 7,
   kCtlStatExpansions = 8,
@@ -366,7 +372,13 @@ enum : int {
   kCtlKillGroups = 15,   // selector, column store: groups with sets killed this round
   kCtlGroupCounter2 = 16,  // IC colour groups: columns taken by the launch
   kCtlScratch2 = 17,     // a word kernels may count into and nobody reads
-  kCtlWords = 19,        // the last word is scratch too
+  kCtlScratch = 18,      // and one more
+  kCtlLine = 16,         // words of a 128-byte line
+  kCtlGroupCounter = 2 * kCtlLine,  // work counter of the persistent samplers
+  kCtlDataBump = 3 * kCtlLine,      // used elements of d_data
+  kCtlStripe0 = 4 * kCtlLine,       // first stripe of the work counters, a line each
+  kCtlStripes = 32,
+  kCtlWords = kCtlStripe0 + kCtlStripes * kCtlLine,
 };
 
 // graph.hip

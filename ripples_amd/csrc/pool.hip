@@ -90,13 +90,14 @@ __global__ void scan_apply(const uint32_t *in, uint64_t n,
 }
 
 __global__ void set_ctl_kernel(unsigned long long *ctl, unsigned long long bump) {
+  for (int i = kCtlStripe0 + static_cast<int>(threadIdx.x); i < kCtlWords; i += blockDim.x) ctl[i] = 0;
+  if (threadIdx.x != 0) return;
   ctl[kCtlDataBump] = bump;
   ctl[kCtlOverflow] = 0;
   ctl[kCtlGroupCounter] = 0;
   ctl[kCtlLongCount] = 0;
   ctl[kCtlElems] = 0;
   ctl[kCtlGroupCounter2] = 0;
-  for (int i = kCtlStatBytes; i <= kCtlStatLevels; ++i) ctl[i] = 0;
 }
 
 __global__ void zero_elems_kernel(unsigned long long *ctl) { ctl[kCtlElems] = 0; }
@@ -468,6 +469,11 @@ void pool_read_ctl(rip_pool *p, bool main) {
   RIP_HIP(hipMemcpyAsync(p->h_ctl, p->d_ctl, sizeof(unsigned long long) * kCtlWords,
                          hipMemcpyDeviceToHost, p->stream));
   RIP_HIP(hipStreamSynchronize(p->stream));
+  for (int i = 0; i < RIP_STAT_COUNT; ++i) {
+    unsigned long long sum = 0;
+    for (int s = 0; s < kCtlStripes; ++s) sum += p->h_ctl[kCtlStripe0 + s * kCtlLine + i];
+    p->h_ctl[kCtlStatBytes + i] = sum;
+  }
   if (main)
     for (int i = 0; i < RIP_STAT_COUNT; ++i) p->main_stats[i] = p->h_ctl[kCtlStatBytes + i];
 }
@@ -526,7 +532,7 @@ void pool_sample(rip_pool *p, uint64_t count, const rip_tune *tune) {
     p->wave_ms = 0.0;
     p->wave_ran = false;
     p->team_ran = false;
-    hipLaunchKernelGGL(set_ctl_kernel, dim3(1), dim3(1), 0, p->stream, p->d_ctl,
+    hipLaunchKernelGGL(set_ctl_kernel, dim3(1), dim3(256), 0, p->stream, p->d_ctl,
                        static_cast<unsigned long long>(p->used_data));
     pool_clear_gref(p, first, first + count);
     // the launchers bracket their main kernel with ev0 / ev1
@@ -537,22 +543,17 @@ void pool_sample(rip_pool *p, uint64_t count, const rip_tune *tune) {
       launches = lt_launch(p, first, count, tune);
     RIP_HIP(hipEventRecord(p->ev2, p->stream));
     launch_sum_u32(p->d_len + first, count, p->d_ctl + kCtlElems, p->stream);
-    unsigned long long *ctl = p->h_ctl;
-    const size_t ctl_bytes = sizeof(unsigned long long) * kCtlWords;
-    RIP_HIP(hipMemcpyAsync(ctl, p->d_ctl, ctl_bytes, hipMemcpyDeviceToHost, p->stream));
-    RIP_HIP(hipStreamSynchronize(p->stream));
+    const unsigned long long *ctl = p->h_ctl;
     // LT: the walk kernel is the main one and the stats so far are its own;
     // IC colour groups alone: one kernel
-    if (p->g->model == RIP_LT || ic.sampler == RIP_SAMPLER_COLOUR)
-      for (int i = 0; i < RIP_STAT_COUNT; ++i) p->main_stats[i] = ctl[kCtlStatBytes + i];
+    pool_read_ctl(p, p->g->model == RIP_LT || ic.sampler == RIP_SAMPLER_COLOUR);
     if (p->g->model == RIP_LT && ctl[kCtlOverflow] == 0 && ctl[kCtlLongCount] != 0) {
       // walks longer than the walk kernel's lists, then the sizes again
       launches += lt_finish_long(p, first, count, ctl[kCtlLongCount]);
       RIP_HIP(hipEventRecord(p->ev2, p->stream));
       hipLaunchKernelGGL(zero_elems_kernel, dim3(1), dim3(1), 0, p->stream, p->d_ctl);
       launch_sum_u32(p->d_len + first, count, p->d_ctl + kCtlElems, p->stream);
-      RIP_HIP(hipMemcpyAsync(ctl, p->d_ctl, ctl_bytes, hipMemcpyDeviceToHost, p->stream));
-      RIP_HIP(hipStreamSynchronize(p->stream));
+      pool_read_ctl(p, false);
     }
     if (ctl[kCtlOverflow] == 0) {
       float ms = 0.0f, call = 0.0f;

@@ -544,13 +544,14 @@ __global__ void __launch_bounds__(BT) lt_walk_kernel(LtParams P) {
     o64 += __shfl_down(o64, d, 64);
     s64 += __shfl_down(s64, d, 64);
   }
-  if (lane == 0 && s64) atomicAdd(&P.ctl[kCtlStatExpansions], s64);
-  if (lane == 0 && rounds) atomicAdd(&P.ctl[kCtlStatLevels], static_cast<unsigned long long>(rounds));
+  unsigned long long *stats = P.ctl + kCtlStripe0 + blockIdx.x % kCtlStripes * kCtlLine;
+  if (lane == 0 && s64) atomicAdd(&stats[RIP_STAT_EXPANSIONS], s64);
+  if (lane == 0 && rounds) atomicAdd(&stats[RIP_STAT_LEVELS], static_cast<unsigned long long>(rounds));
   // algorithmic bytes of the subtraction loop: 8 per visited vertex (its CSR
   // offsets), 8 per scanned in-edge (id + weight), 4 per output id
-  if (lane == 0 && (e64 || o64)) atomicAdd(&P.ctl[kCtlStatBytes], 12ull * o64 + 8ull * e64);
-  if (lane == 0 && e64) atomicAdd(&P.ctl[kCtlStatEdges], e64);
-  if (lane == 0 && p64) atomicAdd(&P.ctl[kCtlStatCoins], p64);
+  if (lane == 0 && (e64 || o64)) atomicAdd(&stats[RIP_STAT_ALGO_BYTES], 12ull * o64 + 8ull * e64);
+  if (lane == 0 && e64) atomicAdd(&stats[RIP_STAT_EDGES], e64);
+  if (lane == 0 && p64) atomicAdd(&stats[RIP_STAT_COINS], p64);
 }
 
 template <int BT, int CAP, int SPILL, int UNROLL>

@@ -784,9 +784,9 @@ bool build_counts(rip_pool *p, uint64_t num_sets, uint32_t k, Need need, uint64_
   // total element count: known for the whole of a pool without columns
   unsigned long long total = p->num_elements;
   if (cols || num_sets != p->num_sets) {
-    hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(1), 0, st, p->d_ctl + kCtlWords - 1);
-    launch_sum_u32(p->d_len, num_sets, p->d_ctl + kCtlWords - 1, st);
-    RIP_HIP(hipMemcpyAsync(&total, p->d_ctl + kCtlWords - 1, sizeof(total),
+    hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(1), 0, st, p->d_ctl + kCtlScratch);
+    launch_sum_u32(p->d_len, num_sets, p->d_ctl + kCtlScratch, st);
+    RIP_HIP(hipMemcpyAsync(&total, p->d_ctl + kCtlScratch, sizeof(total),
                            hipMemcpyDeviceToHost, st));
     RIP_HIP(hipStreamSynchronize(st));
   }
@@ -982,7 +982,7 @@ uint64_t coverage_run(rip_pool *p, uint64_t num_sets, const uint32_t *seeds,
   if (num_seeds)
     hipLaunchKernelGGL(flag_seeds_kernel, dim3(grid_for(num_seeds, kBT, 64)), dim3(kBT), 0, st,
                        reinterpret_cast<const uint32_t *>(s.d_keys), num_seeds, s.d_counts);
-  unsigned long long *out = p->d_ctl + kCtlWords - 1;
+  unsigned long long *out = p->d_ctl + kCtlScratch;
   hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(1), 0, st, out);
   if (num_sets && num_seeds && p->groups) {
     // column sets: hits through their lists or their hot members, counted

@@ -395,14 +395,14 @@ void idle_memory_is_given_back() {
   rip_pool_destroy(p);
   require(used() > with_live, "nothing was kept");
   require(rip_graph_trim(g) == 0, "trim");
-  if (used() > with_live + 4096) {   // a stream kit's control words
+  if (used() > with_live + 8192) {   // a stream kit's control words
     printf("%zu bytes after, %zu before\n", used(), with_live);
     exit(1);
   }
   require(select(live_pool, 1000, 5) == 0, "select");
   rip_pool_destroy(live_pool);
   require(rip_graph_trim(g) == 0, "trim");
-  require(used() <= graph + 4096, "idle blocks are left");
+  require(used() <= graph + 8192, "idle blocks are left");
   rip_graph_destroy(g);
   require(rip_graph_trim(nullptr) == RIP_EINVAL, "no graph");
 }
