@@ -402,7 +402,7 @@ void idle_memory_is_given_back() {
   require(select(live_pool, 1000, 5) == 0, "select");
   rip_pool_destroy(live_pool);
   require(rip_graph_trim(g) == 0, "trim");
-  require(used() <= graph + 8192, "idle blocks are left");
+  require(used() <= graph + 16384, "idle blocks are left");
   rip_graph_destroy(g);
   require(rip_graph_trim(nullptr) == RIP_EINVAL, "no graph");
 }
