@@ -466,7 +466,8 @@ __global__ void __launch_bounds__(BT, kGridWaves) grid_level_kernel(GridParams P
     P.gctl[kGLevels] += 1;
     if (raw > P.cap) P.gctl[kGOver] = 1;
   }
-  const uint64_t each = ncur / (static_cast<uint64_t>(gridDim.x) * NW);
+  const uint64_t waves = static_cast<uint64_t>(gridDim.x) * NW;
+  const uint64_t each = (ncur + waves - 1) / waves;
   const uint32_t take = each >= 64 ? 64u : max(kMinTake, static_cast<uint32_t>(each));
   if (static_cast<uint64_t>(blockIdx.x) * NW * take >= ncur) return;   // no items for it
   P.next = L & 1u ? P.buf[0] : P.buf[1];
@@ -474,13 +475,15 @@ __global__ void __launch_bounds__(BT, kGridWaves) grid_level_kernel(GridParams P
   const unsigned long long *cur = L & 1u ? P.buf[1] : P.buf[0];
   expand_tables<BT>(P, S);
   Expander<BT> E(P, S);
-  for (;;) {
-    unsigned long long i0 = 0;
-    if (E.lane == 0) i0 = atomicAdd(ring_word(P, kRTaken, L), static_cast<unsigned long long>(take));
-    i0 = uniform_u64(i0);
-    if (i0 >= ncur) break;
+  // a wave's first items are its own, later ones claimed past everyone's
+  const uint64_t own = waves * take;
+  for (uint64_t i0 = (static_cast<uint64_t>(blockIdx.x) * NW + E.wid) * take; i0 < ncur;) {
     const bool have = E.lane < take && i0 + E.lane < ncur;
     E.items(have, have ? cur[i0 + E.lane] : 0ull, L, false);
+    if (own >= ncur) break;
+    unsigned long long c = 0;
+    if (E.lane == 0) c = atomicAdd(ring_word(P, kRTaken, L), static_cast<unsigned long long>(take));
+    i0 = own + uniform_u64(c);
   }
   E.finish();
   E.report();

@@ -328,8 +328,13 @@ __global__ void __launch_bounds__(BT, 4) ic_short_kernel(LaneParams P) {
   const uint32_t lane = lane_id();
   uint32_t(*list)[64] = s_list[threadIdx.x >> 6];
   const Affine Pst = uniform_affine(s_p2[0]), P2 = uniform_affine(s_p2[1]);
-  // wave-uniform: the claimed range of sample indices and the output chunk
-  uint64_t next = 0, hi = 0;
+  // wave-uniform: the range of sample indices (the first is the wave's own, later
+  // ones are claimed past everyone's) and the output chunk
+  const uint64_t waves = static_cast<uint64_t>(gridDim.x) * (BT / 64);
+  uint64_t next = (static_cast<uint64_t>(blockIdx.x) * (BT / 64) + (threadIdx.x >> 6)) * kLaneClaim;
+  uint64_t hi = std::min<uint64_t>(next + kLaneClaim, P.count);
+  next = std::min<uint64_t>(next, P.count);
+  const uint64_t own = waves * kLaneClaim;
   bool left = true;
   unsigned long long out_cur = 0, out_end = 0;
   // lane state: a sample (held) with its list, a row of it (in_row)
@@ -395,10 +400,12 @@ __global__ void __launch_bounds__(BT, 4) ic_short_kernel(LaneParams P) {
       uint64_t im = __ballot(!held);
       while (left && im) {
         if (next >= hi) {
-          unsigned long long c = 0;
-          if (lane == 0)
-            c = atomicAdd(&P.ctl[kCtlGroupCounter], static_cast<unsigned long long>(kLaneClaim));
-          c = uniform_u64(c);
+          unsigned long long c = P.count;
+          if (own < P.count) {
+            if (lane == 0)
+              c = atomicAdd(&P.ctl[kCtlGroupCounter], static_cast<unsigned long long>(kLaneClaim));
+            c = own + uniform_u64(c);
+          }
           next = std::min<uint64_t>(c, P.count);
           hi = std::min<uint64_t>(c + kLaneClaim, P.count);
           if (next >= hi) {

@@ -156,6 +156,9 @@ __global__ void __launch_bounds__(BT, 4) ic_stage_kernel(StageParams P) {
   uint32_t head = 0;       // lane k: slot k's
   bool held = false;       // lane k: slot k has a sample
   bool left = true;        // samples may be left to claim (wave-uniform)
+  // the wave's first samples are its own, later ones claimed past everyone's
+  const uint64_t own = static_cast<uint64_t>(gridDim.x) * NW * P.slots;
+  bool first = true;
 
   uint32_t qn = 0;         // edges queued (wave-uniform)
 
@@ -304,12 +307,15 @@ __global__ void __launch_bounds__(BT, 4) ic_stage_kernel(StageParams P) {
       const bool idle = lane < P.slots && !held;
       const uint64_t m = __ballot(idle);
       if (m) {
-        unsigned long long i0 = 0;
-        if (lane == 0)
-          i0 = atomicAdd(&P.ctl[kCtlGroupCounter], static_cast<unsigned long long>(__popcll(m)));
-        i0 = uniform_u64(i0);
+        unsigned long long i0 = wave * P.slots;
+        if (!first) {
+          if (lane == 0)
+            i0 = atomicAdd(&P.ctl[kCtlGroupCounter], static_cast<unsigned long long>(__popcll(m)));
+          i0 = own + uniform_u64(i0);
+        }
         const unsigned long long i = i0 + __popcll(m & lanes_below());
-        left = i0 + __popcll(m) < P.count;
+        left = first ? own < P.count : i0 + __popcll(m) < P.count;
+        first = false;
         const bool got = idle && i < P.count;
         uint32_t root = 0;
         if (got) {
