@@ -322,7 +322,11 @@ __global__ void __launch_bounds__(BT, 4) ic_short_kernel(LaneParams P) {
   __shared__ Affine s_p2[64];
   __shared__ IcGapTab s_tab;
   __shared__ uint32_t s_list[BT / 64][kShort][64];
-  if (threadIdx.x == 0) fill_step_powers(P.step, s_p2);
+  __shared__ unsigned long long s_out;   // the workgroup's first output
+  if (threadIdx.x == 0) {
+    s_out = atomicAdd(&P.ctl[kCtlDataBump], static_cast<unsigned long long>(BT / 64) * P.chunk);
+    fill_step_powers(P.step, s_p2);
+  }
   ic_load_tables(&s_tab);
   __syncthreads();
   const uint32_t lane = lane_id();
@@ -336,7 +340,8 @@ __global__ void __launch_bounds__(BT, 4) ic_short_kernel(LaneParams P) {
   next = std::min<uint64_t>(next, P.count);
   const uint64_t own = waves * kLaneClaim;
   bool left = true;
-  unsigned long long out_cur = 0, out_end = 0;
+  unsigned long long out_cur = s_out + static_cast<unsigned long long>(threadIdx.x >> 6) * P.chunk;
+  unsigned long long out_end = out_cur + P.chunk;
   // lane state: a sample (held) with its list, a row of it (in_row)
   bool held = false, in_row = false;
   uint32_t idx = 0, head = 0, tail = 0;

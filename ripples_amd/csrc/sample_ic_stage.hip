@@ -136,10 +136,14 @@ __global__ void __launch_bounds__(BT, 4) ic_stage_kernel(StageParams P) {
   __shared__ uint64_t s_z[NW][kPack];
   __shared__ Affine s_p2[64];                 // P^(2^j): jumps between gap blocks
   __shared__ IcGapTab s_gap;
+  __shared__ unsigned long long s_out;        // the workgroup's first output
   const uint32_t lane = lane_id();
   const uint32_t wid = threadIdx.x >> 6;
   const uint64_t wave = static_cast<uint64_t>(blockIdx.x) * NW + wid;
-  if (threadIdx.x == 0) fill_step_powers(P.step, s_p2);
+  if (threadIdx.x == 0) {
+    s_out = atomicAdd(&P.ctl[kCtlDataBump], static_cast<unsigned long long>(NW) * P.chunk);
+    fill_step_powers(P.step, s_p2);
+  }
   ic_load_tables(&s_gap);
   if (lane < kPack) s_tail[wid][lane] = s_big[wid][lane] = 0;
   __syncthreads();
@@ -149,9 +153,11 @@ __global__ void __launch_bounds__(BT, 4) ic_stage_kernel(StageParams P) {
   uint32_t *tabs = s_tab[wid];
   uint32_t *htab = P.htab + wave * kPack * 2 * cap;
   uint32_t *list = P.list + wave * kPack * cap;
-  // the wave's reserved output [out_cur, out_end) (wave-uniform); the rest
-  // of a chunk that cannot take the next set stays a gap in the pool's data
-  unsigned long long out_cur = 0, out_end = 0;
+  // the wave's reserved output [out_cur, out_end) (wave-uniform), the first of
+  // it reserved for all waves together; the rest of a chunk that cannot take the
+  // next set stays a gap in the pool's data
+  unsigned long long out_cur = s_out + static_cast<unsigned long long>(wid) * P.chunk;
+  unsigned long long out_end = out_cur + P.chunk;
   unsigned long long st_cand = 0, st_draws = 0, st_exp = 0, st_bytes = 0, st_live = 0;
   uint32_t head = 0;       // lane k: slot k's
   bool held = false;       // lane k: slot k has a sample
