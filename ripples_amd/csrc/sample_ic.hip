@@ -564,12 +564,12 @@ static uint32_t large_sets(rip_pool *p, uint64_t first, uint64_t count, const ui
 
 // Calls of at most this many samples skip the lanes: they fill the stage's
 // waves just so, and a kernel and a host synchronisation are saved.  IMM on
-// 1,000 vertices (weighted cascade, k = 5, eps = 0.5): 1.2 ms with the lanes,
-// 0.97 without; OPIM-C on 200,003 vertices (calls of a few thousand sets): 5.6
-// and 5.2 ms.  Past it the lanes, which hold hundreds of thousands of samples,
-// are the better place for the short ones: twelve served queries took 29.5,
-// 29.4, 30.8 and 31.1 ms with lines of 1,024, 4,096, 16,384 and 65,536, the
-// rest measured the same with all four.
+// 1,000 vertices (weighted cascade, k = 5, eps = 0.5): 1.13 ms with the lanes,
+// 0.85 without; OPIM-C on 200,003 vertices (calls of a few thousand sets): 5.45
+// and 4.65 ms.  Past it the lanes, which hold hundreds of thousands of samples,
+// are the better place for the short ones: twelve served queries took 25.9,
+// 25.8, 26.2 and 26.7 ms with lines of 1,024, 4,096, 16,384 and 65,536, OPIM-C
+// 5.07, 4.65, 4.69 and 4.64, the rest within 3% with all four.
 constexpr uint64_t kWaveDirectMax = 4096;
 
 uint32_t ic_sample(rip_pool *p, uint64_t first, uint64_t count, const IcLaunch &cfg,
