@@ -74,10 +74,9 @@ __host__ __device__ inline float u01(uint64_t x) {
 
 // Integer threshold of an IC edge: live iff (x >> 40) < thr.
 inline uint32_t ic_threshold(float w) {
-  if (!(w > 0.0f)) return 0;  // also NaN
-  if (w >= 1.0f) return 1u << 24;
-  float scaled = w * 16777216.0f;  // exact: power-of-two scaling
-  return static_cast<uint32_t>(scaled);  // floor for positive values
+  const float c = w > 0.0f ? (w < 1.0f ? w : 1.0f) : 0.0f;  // NaN: 0
+  // exact (power-of-two scaling), then floor for what is not negative
+  return static_cast<uint32_t>(static_cast<int32_t>(c * 16777216.0f));
 }
 
 // Device vertex record, one aligned 64-byte line: the jump to the vertex's
