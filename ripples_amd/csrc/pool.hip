@@ -90,7 +90,8 @@ __global__ void scan_apply(const uint32_t *in, uint64_t n,
 }
 
 __global__ void set_ctl_kernel(unsigned long long *ctl, unsigned long long bump) {
-  for (int i = kCtlStripe0 + static_cast<int>(threadIdx.x); i < kCtlWords; i += blockDim.x) ctl[i] = 0;
+  for (int i = kCtlStripe0 + static_cast<int>(threadIdx.x); i < kCtlWords; i += blockDim.x)
+    ctl[i] = 0;
   if (threadIdx.x != 0) return;
   ctl[kCtlDataBump] = bump;
   ctl[kCtlOverflow] = 0;

@@ -30,7 +30,8 @@
 // through hundreds of rounds, about 1 ms however few samples there are.  IMM on
 // R-MAT scale 22 under weighted cascade, one sample per wave and visited checks
 // edge by edge: 33.0 ms; slots 32.0; marks together 29.6; the lanes in front
-// cut to 16 vertices 28.3; sets sorted in registers and list ends in LDS 27.6.
+// cut to 16 vertices 28.3; sets sorted in registers and list ends in LDS 27.6;
+// counters and claims of the waves off one line 24.3.
 #include <algorithm>
 
 #include "device_util.h"
@@ -373,7 +374,7 @@ __global__ void __launch_bounds__(BT, 4) ic_stage_kernel(StageParams P) {
       ++st_exp;
     }
     expand_rows_units<false>(P.ids, P.val, have, rec, z, slot, s_p2, &s_gap, st_cand, st_draws,
-                             st_bytes,                             st_live, take);
+                             st_bytes, st_live, take);
     while (qn) discover();
   }
   report_stats(P.ctl, st_bytes + kIcRecBytes * st_exp, st_cand, st_draws, st_exp, st_live);
