@@ -83,7 +83,7 @@ struct SpreadParams {
   unsigned long long *act_out;
   uint32_t *lev_out;
   unsigned long long *ctl;  // [0]: replica counter
-  uint32_t *scratch;        // per workgroup: LT sums, queue, LT candidates, bitmaps
+  uint32_t *scratch;        // per workgroup: LT sums, queue, LT candidates, bitmaps, 2 words
   uint64_t per_wg;          // its words
   uint64_t words;           // 32-bit words per bitmap
   Affine step;
@@ -260,11 +260,12 @@ __device__ inline bool lt_reaches(const SpreadParams &P, const uint32_t *act, ui
   return total >= th;
 }
 
-// A replica that met fewer than this share of n edges clears its sums edge by
-// edge.  1,024 replicas of 5 seeds that reach a handful of 2^22 vertices: 5.9 ms
-// when each cleared them all, 0.12 this way; 512 of 20 seeds on 2^18 vertices
-// with weights of 0.3 to 0.9 a row 0.37 to 2.07 and 0.17 to 1.68.  Lines of n and
-// n / 16 measured the same.
+// The sums are zero between replicas, or known not to be: one that met fewer than
+// this share of n edges clears those of its targets as it ends, after any other
+// all are cleared before the next.  1,024 replicas of 5 seeds that reach a
+// handful of 2^22 vertices: 5.9 ms when each cleared them all, 0.12 this way; 512
+// of 20 seeds on 2^18 vertices with weights of 0.3 to 0.9 a row 0.37 to 2.07 and
+// 0.17 to 1.68.  Lines of n and n / 16 measured the same.
 constexpr uint32_t kClearShare = 4;
 
 template <int BT, bool kLds>
@@ -273,6 +274,10 @@ __global__ void __launch_bounds__(BT) spread_lt_kernel(SpreadParams P) {
   __shared__ uint32_t s_len, s_next, s_nc, s_edges;
   __shared__ unsigned long long s_r;
   const uint32_t tid = threadIdx.x, lane = lane_id();
+  // whether sums are left from the workgroup's last replica, of an earlier launch
+  // perhaps
+  uint32_t *left = P.scratch + static_cast<uint64_t>(blockIdx.x + 1) * P.per_wg - 2;
+  bool dirty = *left != 0;
   double *sum = reinterpret_cast<double *>(P.scratch + static_cast<uint64_t>(blockIdx.x) * P.per_wg);
   uint32_t *queue = reinterpret_cast<uint32_t *>(sum + P.n);
   uint32_t *clist = queue + P.n;
@@ -284,13 +289,15 @@ __global__ void __launch_bounds__(BT) spread_lt_kernel(SpreadParams P) {
     const unsigned long long r = next_replica(P.ctl, &s_r);
     if (r >= P.count) break;
     if (tid == 0) s_len = s_next = s_nc = s_edges = 0;
+    if (dirty)
+      for (uint32_t v = tid; v < P.n; v += BT) sum[v] = 0.0;
     __syncthreads();
     const uint64_t z = sample_z(P.seed, P.first + r);
     for (uint32_t i = tid; i < P.nseeds; i += BT) {
       const uint32_t v = P.seeds[i];
       if (set_bit(act, v)) queue[atomicAdd(&s_len, 1u)] = v;
     }
-    __syncthreads();
+    barrier();   // the zeroes are in place before the atomics
     uint32_t lo = 0, hi = s_len, lev = 0, edges = 0;
     __syncthreads();
     do {
@@ -360,13 +367,12 @@ __global__ void __launch_bounds__(BT) spread_lt_kernel(SpreadParams P) {
       P.lev_out[r] = lev;
     }
     for (uint32_t i = tid; i < hi; i += BT) clear_bits<kLds>(act, queue[i]);
-    // the sums are zero between replicas: all of them again, or those of the
-    // activated vertices' targets where they are few (next_replica() waits for
-    // the stores before the next atomics)
+    // (next_replica() waits for these stores before the next atomics)
     edges = wave_sum(edges);
     if (lane == 0) atomicAdd(&s_edges, edges);
     __syncthreads();
-    if (s_edges < P.n / kClearShare) {
+    dirty = s_edges >= P.n / kClearShare;
+    if (!dirty) {
       for_level<BT / 64>(0, hi, &s_next, [&](bool have, uint32_t at) {
         uint32_t begin = 0, deg = 0;
         if (have) {
@@ -378,10 +384,9 @@ __global__ void __launch_bounds__(BT) spread_lt_kernel(SpreadParams P) {
           if (valid) sum[P.fdst[f]] = 0.0;
         });
       });
-    } else {
-      for (uint32_t v = tid; v < P.n; v += BT) sum[v] = 0.0;
     }
   }
+  if (tid == 0) *left = dirty ? 1u : 0u;
 }
 
 using SpreadKernel = void (*)(SpreadParams);
@@ -459,7 +464,8 @@ void spread_run(rip_graph *g, const uint32_t *seeds, uint32_t nseeds, uint64_t s
   const uint64_t bitmaps = 4 * words * (ic ? 1 : 2);   // bytes
   const bool lds = bitmaps <= kSpreadLds;
   // 32-bit words per workgroup: queue, bitmaps outside LDS; LT: sums, candidates
-  const uint64_t per_wg = ((ic ? n : 4 * n) + (lds ? 0 : bitmaps / 4) + 1) / 2 * 2;
+  // and, last, whether sums are left
+  const uint64_t per_wg = ((ic ? n : 4 * n) + (lds ? 0 : bitmaps / 4) + 1) / 2 * 2 + 2;
   const uint64_t free_b = device_free_bytes();
   const uint64_t held = g->fwd.wgs * g->fwd.per_wg * 4;
   const uint64_t budget = std::min<uint64_t>((free_b + held) / 8, 16ull << 30);

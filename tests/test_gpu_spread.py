@@ -63,3 +63,15 @@ def test_lt_replicas_one_after_the_other(wscale, orc):
     seeds = np.arange(0, 40, 2, dtype=np.uint32)
     check(R.LT, rmat(3001, 12, 6, R.W_LT_NORM, wscale, 5), seeds, 4000, orc)
     check(R.LT, rmat(40009, 16, 8, R.W_LT_NORM, wscale, 6), seeds[:4], 2500, orc)
+
+
+def test_lt_calls_one_after_the_other(orc):
+    """Calls on one graph that leave sums behind and calls that do not."""
+    index, edges, w = rmat(9001, 14, 8, R.W_LT_NORM, 0.9, 7)
+    g = R.Graph(index, edges, w, model=R.LT)
+    many, few = np.arange(400, dtype=np.uint32), np.array([8999], np.uint32)
+    for seeds, count in ((many, 40), (few, 60), (many, 3), (few, 2), (many, 1500), (few, 1500), (many, 30)):
+        act, lev = g.spread(seeds, count, seed=11)
+        ea, el = orc.spread(R.LT, index, edges, w, seeds, 11, 0, count)
+        assert np.array_equal(act, ea) and np.array_equal(lev, el)
+    g.close()
